@@ -35,11 +35,12 @@ enum {
     UQK_SHALLOW_WATER2D_BARRIER = 4    /* SW2D with a log barrier on h (no reference)    */
 };
 
-/* Arithmetic of the Hessian assembly. */
+/* Arithmetic of the Newton steps. */
 enum {
-    UQK_FP64 = 0,   /* everything in FP64 (the plain path)                        */
-    UQK_MIXED = 1   /* Hessian on MFMA in reduced precision, FP64 Cholesky,
-                       FP64 gradient/residual/accept test                         */
+    UQK_FP64 = 0,   /* everything in FP64, a factorisation per step (the plain path) */
+    UQK_MIXED = 1   /* steps on kept FP32 factorisations (uqk_set_factor_reuse), the
+                       workgroup kernel's Hessian on FP32 MFMA; factorisation,
+                       gradient, residual and accept test in FP64                  */
 };
 
 /* Per-cell closure status (replaces the reference's exit(EXIT_FAILURE)). */
@@ -249,10 +250,10 @@ double uqk_last_closure_ms(const uqk_ctx* ctx);
 int uqk_last_closure_stats(const uqk_ctx* ctx, int64_t* newton_steps, int64_t* gradient_evaluations);
 /* Reuse of the factorisation in the mixed closure (no counterpart in the
  * reference; on by default for UQK_MIXED contexts).  In the time loop, after
- * a cell's FP64 Cholesky of its (FP32-assembled) Hessian in one step, the
- * library keeps P = H^{-1} of the factored matrix: the wave kernel (uniform
- * orders, n < 64) as an explicit inverse computed after the launch (FP64,
- * kept in FP32), the workgroup kernel (n up to 128, per-cell orders too) as
+ * a cell's FP64 factorisation of its Hessian in one step, the library keeps
+ * P = H^{-1} of the factored matrix: the wave kernel (uniform orders,
+ * n < 64) as an explicit inverse (computed in FP64 with the step, kept in
+ * FP32), the workgroup kernel (n up to 128, per-cell orders too) as
  * the factor U rounded to FP32 and tagged with the cell's order, replaced
  * by U^{-1} (P = U^{-1} U^{-T}) the first time a later step uses it.  The
  * cell's Newton steps in later time steps take d = P g refined once with
@@ -261,14 +262,14 @@ int uqk_last_closure_stats(const uqk_ctx* ctx, int64_t* newton_steps, int64_t* g
  * a contraction clearly worse than a damped Newton step's (above
  * 1.2 (1 - alpha) + 1e-3; + 0.05 from n = 64 on, where a factorisation costs
  * over ten steps on the kept one), the cell's current Hessian is factored
- * and the reference Newton step runs.  Memory per cell: n (n + 1) floats and
- * n (n + 3) / 2 doubles (wave kernel), n (n + 1) / 2 floats (workgroup
+ * and the reference Newton step runs.  Memory per cell: n times n rounded up
+ * to a multiple of four floats (wave kernel), n (n + 1) / 2 floats (workgroup
  * kernel), n = S M.  In a single closure call (wave kernel, uniform
  * orders, damped Newton: alpha < 1, whose steps contract linearly anyway)
  * a cell's Newton steps after a factorisation
- * solve with that factor (d = (U^T U)^{-1} g) under the same accept and
+ * apply that step's FP64 inverse (d = H^{-1} g) under the same accept and
  * contraction tests, with no memory beyond the call.  Results match the
- * plain mixed closure to the Newton tolerance, not bit for bit.
+ * plain closure to the Newton tolerance, not bit for bit.
  * uqk_invalidate_factors forgets the kept factorisations (after replacing the
  * duals wholesale). */
 int uqk_set_factor_reuse(uqk_ctx* ctx, int32_t on);

@@ -36,13 +36,14 @@ HIP_FLAGS = [
 
 # extra flags per source file
 EXTRA_FLAGS = {
-    # the one-wavefront closure is a chain of dependent steps (pivot
-    # broadcasts, Newton steps); LLVM's iterative ILP scheduler orders it
-    # better than the default occupancy-driven one (about 3% more throughput
-    # for the mixed closure, the same for FP64); closure_wave_reuse.hip keeps
-    # the default one, which spills less there
-    "closure_wave.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-    "closure_wave_lag.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+    # the one-wavefront closure is one long loop per cell with many constants
+    # (the polynomials of exp and log) and lane addresses: hoisted out of the
+    # loop they take the registers that the loop's own values then spill from
+    # (the mixed time loop's kernel: 76 VGPRs spilled with the hoisting, 2
+    # without)
+    "closure_wave.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wave_lag.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wave_reuse.hip": ["-mllvm", "-disable-machine-licm"],
 }
 
 

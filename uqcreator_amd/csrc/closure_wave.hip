@@ -1,8 +1,7 @@
 // closure_wave.hip -- instantiations and dispatch of the one-wavefront
-// Newton closure (closure_wave_kernel.h): FP64 (PREC 0) and mixed (PREC 1);
-// the mixed closure with kept inverses (PREC 2) and the kernel that turns a
-// time step's new Cholesky factors into those inverses live in
-// closure_wave_reuse.hip, the mixed closure reusing factors within one call
+// Newton closure (closure_wave_kernel.h): FP64 and mixed without reuse (PREC 0);
+// the mixed closure with kept inverses (PREC 2) lives in
+// closure_wave_reuse.hip, the mixed closure reusing inverses within one call
 // (PREC 4) in closure_wave_lag.hip.
 #include "closure_wave_kernel.h"
 
@@ -19,28 +18,21 @@ template <int KIND, int M, int Q>
 static bool wave_try(int kind, int m, int q, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
                      hipError_t* err, const LaunchShape& shape) {
     if (!wave_fits<KIND, M, Q>(kind, m, q, max_lds)) return false;
-    if (a.prec == UQK_FP64) {
-        wave_go<KIND, M, Q, 0>(a, max_lds, num_cu, st, err, shape);
-        return true;
-    }
+    // (pinv_mode is 0 in FP64)
     // the time loop's mixed closure with kept inverses
     if (a.pinv_mode == 1 && newton_wave_reuse_launch(kind, m, q, a, max_lds, num_cu, st, err, shape)) return true;
     // one closure call's mixed closure reusing each cell's factor within the call
     if (a.pinv_mode == 2 && newton_wave_lag_launch(kind, m, q, a, max_lds, num_cu, st, err, shape)) return true;
-    wave_go<KIND, M, Q, 1>(a, max_lds, num_cu, st, err, shape);
+    wave_go<KIND, M, Q, 0>(a, max_lds, num_cu, st, err, shape);
     return true;
 }
 
 template <int KIND, int M, int Q>
 static bool wave_limits(int kind, int m, int q, int prec, int max_lds, int waves, int* max_waves, int* occupancy) {
     if (!wave_fits<KIND, M, Q>(kind, m, q, max_lds)) return false;
-    if (prec == UQK_FP64) {
-        *max_waves = wave_max_waves<KIND, M, Q, 0>(max_lds);
-        *occupancy = wave_occupancy<KIND, M, Q, 0>(waves < *max_waves ? waves : *max_waves);
-    } else {
-        *max_waves = wave_max_waves<KIND, M, Q, 1>(max_lds);
-        *occupancy = wave_occupancy<KIND, M, Q, 1>(waves < *max_waves ? waves : *max_waves);
-    }
+    (void)prec;
+    *max_waves = wave_max_waves<KIND, M, Q, 0>(max_lds);
+    *occupancy = wave_occupancy<KIND, M, Q, 0>(waves < *max_waves ? waves : *max_waves);
     return true;
 }
 

@@ -125,27 +125,17 @@ int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
 // capture only; a change of mode starts with no kept factor.
 int ensure_factor_buffers(uqk_ctx* ctx, long n_cells, int mode) {
     const long n = (long)ctx->S * ctx->M;
-    // mode 1: n x n FP32 inverse (row stride n + 1) and the FP64 factor
-    // (packed U, 1/U_rr); mode 2: the FP32 factor (packed U)
-    const long nn = mode == 1 ? n * (n + 1) : n * (n + 1) / 2;
-    const long nu = n * (n + 1) / 2 + n;
+    // mode 1: the FP32 inverse; mode 2: the FP32 factor (packed U)
+    const long nn = mode == 1 ? uqk::newton_wave_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
     if (ctx->pinv_cell_cap >= n_cells && ctx->factor_mode == mode) return 0;
     if (ctx->capturing) return fail(ctx, -1, "kept factors: buffers must exist before graph capture");
     hipFree(ctx->pinv_cell);
-    hipFree(ctx->ufac_cell);
     hipFree(ctx->pinv_ok);
-    hipFree(ctx->pinv_list);
     ctx->pinv_cell = nullptr;
-    ctx->ufac_cell = nullptr;
     ctx->pinv_ok = nullptr;
-    ctx->pinv_list = nullptr;
     ctx->pinv_cell_cap = 0;
     ctx->factor_mode = 0;
     UQK_HIP(ctx, hipMalloc(&ctx->pinv_cell, sizeof(float) * (size_t)nn * n_cells));
-    if (mode == 1) {
-        UQK_HIP(ctx, hipMalloc(&ctx->ufac_cell, sizeof(double) * (size_t)nu * n_cells));
-        UQK_HIP(ctx, hipMalloc(&ctx->pinv_list, sizeof(int) * (size_t)n_cells));
-    }
     UQK_HIP(ctx, hipMalloc(&ctx->pinv_ok, sizeof(int) * (size_t)n_cells));
     UQK_HIP(ctx, hipMemsetAsync(ctx->pinv_ok, 0, sizeof(int) * (size_t)n_cells, ctx->stream));
     ctx->pinv_cell_cap = n_cells;
@@ -238,18 +228,15 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
     a.took = counters + 4;
     a.nfactor = counters + 5;
     // mixed precision: kept factorisations (per cell in the time loop: the
-    // wave kernel's inverses, computed after the launch that factored, or the
-    // workgroup kernel's FP32 factors; per wave for a single closure call);
+    // wave kernel's inverses or the workgroup kernel's FP32 factors; in
+    // registers for a single closure call);
     // the buffers exist before a graph is captured
     const int fmode = factors_per_cell ? factor_mode(ctx, nt != nullptr) : 0;
     if (fmode) {
         if (int rc = ensure_factor_buffers(ctx, n, fmode)) return rc;
         a.pinv_mode = 1;
         a.pinv = ctx->pinv_cell;
-        a.ufac = ctx->ufac_cell;
         a.pinv_ok = ctx->pinv_ok;
-        a.plist = ctx->pinv_list;
-        a.plist_count = counters + 7;
         a.pinv_slots = ctx->pinv_cell_cap;
     } else if (ctx->precision == UQK_MIXED && ctx->factor_reuse && !nt && ctx->c.max_iter != 1 && !factors_per_cell &&
                ctx->c.alpha < 1.0) {
@@ -304,14 +291,6 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
         if (uqk::newton_wave_launch(ctx->kind, ctx->M, ctx->Q, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream, &e,
                                     ctx->shape)) {
             UQK_HIP(ctx, e);
-            if (a.pinv_mode == 1) {
-                // the inverses of this launch's new factors, for the next steps
-                if (!uqk::factor_inverse_launch(ctx->kind, ctx->M, ctx->Q, n, counters + 7, ctx->pinv_list,
-                                                ctx->pinv_ok, ctx->ufac_cell, ctx->pinv_cell, active, ctx->num_cu,
-                                                ctx->stream, &e))
-                    return fail(ctx, -3, "no factor inverse kernel for this shape");
-                UQK_HIP(ctx, e);
-            }
             if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev1, ctx->stream));
             // every cell's uQ, moments and ComputeDt are now those of its lambda
             ctx->step_recon = a.dt_cell != nullptr;
@@ -625,9 +604,7 @@ int uqk_destroy(uqk_ctx* ctx) {
     hipFree(ctx->d_partial);
     hipFree(ctx->d_scalars);
     hipFree(ctx->pinv_cell);
-    hipFree(ctx->ufac_cell);
     hipFree(ctx->pinv_ok);
-    hipFree(ctx->pinv_list);
     hipFree(ctx->check_list);
     hipFree(ctx->check_grad);
     hipFree(ctx->check_dt);

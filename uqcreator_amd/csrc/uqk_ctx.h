@@ -57,17 +57,14 @@ struct uqk_ctx {
     uqk_mlp* warm = nullptr;  // learned warm start run before each closure (not owned)
     uqk::RefineArgs refine{};  // adaptive levels: refine.nlev > 1 turns refinement on in the step
     unsigned char* scratch = nullptr;  // device address of the library's static staging array on `device`
-    // reuse of the factorisation in the mixed wave kernel across time
-    // steps: each cell's kept inverse Hessian (FP32, n x n, row stride n + 1),
-    // its last factor (FP64 packed U, 1/U_rr) and state (0 none, 1 inverse
-    // kept, 2 factor stored, inverse pending)
+    // reuse of the factorisation in the mixed closure across time steps: each
+    // cell's kept inverse Hessian or factor (FP32) and its state (wave
+    // kernel: 0 none, 1 inverse kept)
     bool factor_reuse = true;
     float* pinv_cell = nullptr;
-    double* ufac_cell = nullptr;
     int* pinv_ok = nullptr;
-    int* pinv_list = nullptr;  // cells with a new factor, per launch
-    // what the buffers hold: 1 the wave kernel's kept inverses (with ufac
-    // and pinv_list), 2 the workgroup kernel's kept FP32 factors; 0 none
+    // what the buffers hold: 1 the wave kernel's kept inverses, 2 the
+    // workgroup kernel's kept FP32 factors; 0 none
     int factor_mode = 0;
     // residual check before the wave kernel in the time loop (on by
     // default): the cells it leaves to the Newton kernel

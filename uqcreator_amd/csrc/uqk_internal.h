@@ -63,22 +63,17 @@ struct NewtonArgs {
     // its uQ, moments and ComputeDt
     double* dt_cell;
     const int* recon_ok;
-    // mixed precision, wave kernel: reuse of the factorisation.
+    // mixed precision: reuse of the factorisation.
     // pinv_mode 1 (time loop, across steps): a cell whose pinv_ok is 1 holds
-    // a kept inverse Hessian in pinv (FP32, n x n, row stride n + 1) and
-    // takes Newton steps d = P g refined once with the FP64 Hessian-vector
-    // product; a factored step stores its factor in ufac (packed upper U,
-    // then 1/U_rr, FP64), sets pinv_ok to 2 and appends the cell to
-    // plist[(*plist_count)++], and factor_inverse_kernel turns the listed
-    // factors into the next inverses.  pinv_mode 2 (one closure call): a
-    // cell's later Newton steps solve with the factor of its last Cholesky
-    // while they contract.  nfactor[0] += Cholesky factorisations,
-    // nfactor[1] += accepted steps on a kept factor or inverse.
+    // a kept inverse Hessian in pinv (wave kernel: FP32, row r's entries
+    // 4 t + q in runs over t, q = 0..3) and takes Newton steps d = P g refined
+    // once with the FP64 Hessian-vector product; a factored step stores its
+    // inverse and sets pinv_ok to 1.  pinv_mode 2 (one closure call): a
+    // cell's later Newton steps apply the inverse of its last Hessian while
+    // they contract.  nfactor[0] += factorisations, nfactor[1] += accepted
+    // steps on a kept factor or inverse.
     float* pinv;
-    double* ufac;
     int* pinv_ok;
-    int* plist;
-    unsigned long long* plist_count;
     int pinv_mode;
     long pinv_slots;
     unsigned long long* nfactor;
@@ -109,8 +104,8 @@ struct RunState {
 // Closure counters of a launch: [0] work-queue head, [1] failed cells, [2]
 // Newton steps, [3] gradient evaluations, [4] cells that started from the
 // learned warm start, [5] Cholesky factorisations, [6] steps on a kept
-// inverse, [7] cells listed for factor_inverse_kernel, [8] cells the
-// residual check left to the Newton kernel; all zero at launch.
+// inverse, [7] unused, [8] cells the residual check left to the Newton
+// kernel; all zero at launch.
 constexpr int kClosureCounters = 9;
 
 // Launch shape of the specialised closure kernel; 0 = automatic (as many
@@ -140,12 +135,8 @@ bool closure_check_wave_fits(int S, int M, int Q, int max_lds);
 hipError_t closure_check_wave_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st);
 // Whether (kind, M, Q) has the mixed wave kernel with kept inverses.
 bool newton_wave_reuse_fits(int kind, int M, int Q, int max_lds);
-// Inverses of the factors the last mixed wave launch stored and listed
-// (list[0 .. *count), flags 2 -> 1), up to ncell of them; false when there
-// is no such kernel for (kind, M, Q).
-bool factor_inverse_launch(int kind, int M, int Q, long ncell, const unsigned long long* count, const int* list,
-                           int* flags, const double* ufac, float* pinv, const int* active, int num_cu,
-                           hipStream_t st, hipError_t* err);
+// Floats of a cell's kept inverse (wave kernel).
+long newton_wave_kept_floats(int S, int M);
 // Largest waves per workgroup the LDS allows and the resident workgroups per
 // CU at `waves` for the specialised kernel of (kind, M, Q, prec); false when
 // there is none.
