@@ -13,16 +13,42 @@
 // wave kernel's order), U(Lambda_k) -> uQ (written for every cell; the
 // Newton kernel rewrites the cells it takes), ComputeDt there, and the
 // projection sum_k U(k) phiW(k, i) accumulated in k order.  The list grows
-// by one atomic per wave (ballot and prefix count); the gradients of the
-// listed cells are stored for the Newton kernel, which starts from them.
+// by one atomic per workgroup (ballots and prefix counts); the gradients of
+// the listed cells are stored for the Newton kernel, which starts from them.
 #include <hip/hip_runtime.h>
 
+#include "cell_queue.h"
 #include "uqk_device.h"
 #include "uqk_internal.h"
 
 namespace uqk {
 
 constexpr int kCheckThreads = 256;
+
+// Appends a workgroup's cells that are left to the Newton kernel to the list,
+// in order, with one atomic (12 ns each on the one address: one per wavefront
+// took 12 us of the check's 21 at 65,536 cells).
+__device__ __forceinline__ void append_left(const NewtonArgs& a, long cell, bool mine) {
+    constexpr int W = kCheckThreads / 64;
+    __shared__ int wave_n[W];
+    __shared__ unsigned long long base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long left = __ballot(mine);
+    if (lane == 0) wave_n[wave] = __popcll(left);
+    __syncthreads();
+    int at = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        at += w < wave ? wave_n[w] : 0;
+        all += wave_n[w];
+    }
+    if (threadIdx.x == 0 && all) base = atomicAdd(a.list_count, (unsigned long long)all);
+    __syncthreads();
+    if (mine) {
+        const unsigned long long below = lane ? (left & (~0ull >> (64 - lane))) : 0ull;
+        a.list_out[base + at + __popcll(below)] = (int)cell;
+    }
+}
 
 template <int KIND, int M, int Q>
 __global__ void __launch_bounds__(kCheckThreads) closure_check_kernel(NewtonArgs a) {
@@ -94,27 +120,13 @@ __global__ void __launch_bounds__(kCheckThreads) closure_check_kernel(NewtonArgs
 #pragma unroll
         for (int t = 0; t < N; ++t) gg[t] = acc[t] - ug[t];
     }
-    // the others to the list: one atomic per wave
-    const unsigned long long left = __ballot(valid && !conv);
-    const int lane = threadIdx.x & 63;
-    unsigned long long base = 0;
-    if (lane == 0 && left) base = atomicAdd(a.list_count, (unsigned long long)__popcll(left));
-    base = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(base >> 32)) << 32) |
-           (unsigned)__builtin_amdgcn_readfirstlane((unsigned)base);
-    if (valid && !conv) {
-        const unsigned long long below = lane ? (left & (~0ull >> (64 - lane))) : 0ull;
-        a.list_out[base + __popcll(below)] = (int)cell;
-    }
+    append_left(a, cell, valid && !conv);
     // counters: one gradient per cell (the listed cells' is their Newton
     // start); ComputeDt of finished cells
-    const unsigned long long evaluated = __ballot(valid);
-    double m = conv ? dtm : 1e10;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off, 64));
-    if (lane == 0) {
-        if (evaluated) atomicAdd(a.nfail + 2, (unsigned long long)__popcll(evaluated));
-        if (a.dt_min && m < 1e10) atomicMin(a.dt_min, (unsigned long long)__double_as_longlong(m));
-    }
+    unsigned long long n[7] = {};
+    n[3] = __popcll(__ballot(valid));
+    __shared__ double red[8 * (kCheckThreads / 64)];
+    add_counts(n, wave_min(conv ? dtm : 1e10), red, a.counter, a.dt_min);
 }
 
 // The residual check of a run's later steps: the last step's closure left,
@@ -152,21 +164,11 @@ __global__ void __launch_bounds__(kCheckThreads) closure_recheck_kernel(NewtonAr
 #pragma unroll
         for (int t = 0; t < N; ++t) gg[t] = g[t];
     }
-    const unsigned long long left = __ballot(valid && !conv);
-    const int lane = threadIdx.x & 63;
-    unsigned long long base = 0;
-    if (lane == 0 && left) base = atomicAdd(a.list_count, (unsigned long long)__popcll(left));
-    base = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(base >> 32)) << 32) |
-           (unsigned)__builtin_amdgcn_readfirstlane((unsigned)base);
-    if (valid && !conv) {
-        const unsigned long long below = lane ? (left & (~0ull >> (64 - lane))) : 0ull;
-        a.list_out[base + __popcll(below)] = (int)cell;
-    }
+    append_left(a, cell, valid && !conv);
     // ComputeDt of the finished cells, as the last step found it
-    double m = (conv && a.dt_min) ? a.dt_cell[cs] : 1e10;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off, 64));
-    if (lane == 0 && a.dt_min && m < 1e10) atomicMin(a.dt_min, (unsigned long long)__double_as_longlong(m));
+    const unsigned long long none[7] = {};
+    __shared__ double red[8 * (kCheckThreads / 64)];
+    add_counts(none, wave_min((conv && a.dt_min) ? a.dt_cell[cs] : 1e10), red, a.counter, a.dt_min);
 }
 
 // The same check for the workgroup kernel's sizes (n = S*M up to 128, any

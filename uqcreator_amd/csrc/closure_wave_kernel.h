@@ -37,6 +37,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "cell_queue.h"
 #include "tile_solve.h"
 #include "uqk_device.h"
 #include "uqk_internal.h"
@@ -91,6 +92,14 @@ template <int PREC> constexpr bool wave_reuses = PREC == 2 || PREC == 4;
 // the inverse from the registers, the lower triangle otherwise
 template <int PREC, int NT> constexpr int wave_tiles = PREC == 4 ? NT * NT : NT * (NT + 1) / 2;
 
+// basis pair (j <= i) of number e = i (i + 1) / 2 + j, from its root (e < 2^12)
+__device__ __forceinline__ void basis_pair(int e, int& j, int& i) {
+    i = (int)((__builtin_amdgcn_sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
+    i -= i * (i + 1) / 2 > e ? 1 : 0;
+    i += (i + 1) * (i + 2) / 2 <= e ? 1 : 0;
+    j = e - i * (i + 1) / 2;
+}
+
 // The system of a Newton step at the iterate whose Lambda lies at this lane's
 // point in Lk, into bh: the pair products (pairs x points)(points x state
 // pairs) on FP64 matrix steps; with RHS also the gradient g of this lane's
@@ -125,12 +134,8 @@ __device__ __forceinline__ void wave_system(const ClosureParams& c, const double
         for (int pg = 0; pg < W::PG; ++pg) acc[pg] = 0.0;
         const D *fj = nullptr, *wi = nullptr;
         if constexpr (!W::PAIR_TABLE) {
-            // pair number e = i (i + 1) / 2 + j, from its root
-            const int e = 16 * t + p16 < W::NPAIR ? 16 * t + p16 : 0;
-            int i = (int)((__builtin_amdgcn_sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
-            i -= i * (i + 1) / 2 > e ? 1 : 0;
-            i += (i + 1) * (i + 2) / 2 <= e ? 1 : 0;
-            const int j = e - i * (i + 1) / 2;
+            int j, i;
+            basis_pair(16 * t + p16 < W::NPAIR ? 16 * t + p16 : 0, j, i);
             fj = smem + j * QP + q4;
             wi = smem + W::PHIW + i * QP + q4;
         }
@@ -214,7 +219,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     static_assert(N < 64 && Q <= 64, "wave kernel needs n < 64 and Q <= 64");
     static_assert(M <= 16 && S <= 4, "the projection takes one 4 x 16 tile");
     extern __shared__ double smem[];
-    if (a.active && *a.active == 0) return;
+    // (both loads are sent before either is looked at)
+    const int active = a.active ? *a.active : 1;
+    const long ncells = a.cell_list ? (long)*a.cell_count : a.ncell;
+    if (!active || (long)blockIdx.x >= ncells) return;  // no cell for any wavefront of this workgroup
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int p16 = lane & 15, q4 = lane >> 4;
     double* phiT = smem;              // phiT[i*QP + k]  = phi(k, i), zero past Q
@@ -225,19 +233,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         phiT[t] = in ? a.phi[k * M + i] : 0.0;
         if (i < M) phiwT[t] = in ? a.phiw[k * M + i] : 0.0;
     }
-    // basis pair (j <= i) of number e
-    auto pair_of = [](int e, int& j, int& i) {
-        i = 0;
-        while ((i + 1) * (i + 2) / 2 <= e) ++i;
-        j = e - i * (i + 1) / 2;
-    };
     double* pairs = smem + W::PAIRS;
     if constexpr (W::PAIR_TABLE) {
         // operand (pair 16 t + l % 16, point 4 ks + l / 16) at (t KS + ks) 64 + l
         for (int t = threadIdx.x; t < W::PT * KS * 64; t += blockDim.x) {
             const int ln = t & 63, ks = (t >> 6) % KS, e = 16 * ((t >> 6) / KS) + (ln & 15), k = 4 * ks + (ln >> 4);
             int j, i;
-            pair_of(e < W::NPAIR ? e : 0, j, i);
+            basis_pair(e < W::NPAIR ? e : 0, j, i);
             pairs[t] = k < Q ? a.phi[k * M + j] * a.phiw[k * M + i] : 0.0;
         }
     }
@@ -251,9 +253,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             tr = tile / NT;
             tc = tile % NT;
         } else {
-            tr = 0;
-            while ((tr + 1) * (tr + 2) / 2 <= tile) ++tr;
-            tc = tile - tr * (tr + 1) / 2;
+            basis_pair(tile, tc, tr);
         }
         unsigned word = 0;
         for (int h = 0; h < 2; ++h) {
@@ -286,49 +286,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     const ClosureParams& c = a.c;
     const int SM = S * M;
 
-    // Work queue.  Position t of the 2^qbits queue is cell bitreverse(t)
-    // (skipped when >= ncell): neighbouring costly cells go to different
-    // waves.  After a residual check the queue runs over the *cell_count
-    // listed cells instead: position t is cell_list[bitreverse(t)] (skipped
-    // past the count).  Newton and failure counts are summed per wave and
-    // then per workgroup.  The next cell is taken from the queue while the
-    // current one starts, and its moments, duals and flags are loaded before
-    // the current cell's results are stored, so neither latency stands
-    // between cells.
-    unsigned long long w_fail = 0, w_newton = 0, w_grad = 0, w_took = 0, w_factor = 0, w_reuse = 0;
-    double w_dt = 1e10;  // min ComputeDt over this wave's cells (fused path)
-    const long nlist = a.cell_list ? (long)__builtin_amdgcn_readfirstlane((int)*a.cell_count) : 0;
-    int lbits = 0;
-    while ((1L << lbits) < nlist) ++lbits;
-    const int qb = a.cell_list ? lbits : a.qbits;
-    const long qsize = 1L << qb;
-    long qpos = 0, qend = 0;
-    // the next cell of the queue, -1 when it is exhausted (listed cells are
-    // valid by construction)
-    auto fetch = [&]() -> long {
-        for (;;) {
-            if (qpos == qend) {
-                long want = (qsize - qend) / (2 * a.waves);
-                if (want < 1) want = 1;
-                unsigned long long got = 0;
-                if (lane == 0) got = atomicAdd(a.counter, (unsigned long long)want);
-                const long base =
-                    (long)(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(got >> 32)) << 32) |
-                           (unsigned)__builtin_amdgcn_readfirstlane((unsigned)got));
-                if (base >= qsize) return -1;
-                qpos = base;
-                qend = base + want < qsize ? base + want : qsize;
-            }
-            const unsigned pos = (unsigned)qpos;
-            ++qpos;
-            const long qcell = qb ? (long)(__builtin_bitreverse32(pos) >> (32 - qb)) : 0;
-            if (a.cell_list) {
-                if (qcell >= nlist) continue;
-                return (long)__builtin_amdgcn_readfirstlane(a.cell_list[qcell]);
-            }
-            if (qcell < a.ncell) return qcell;
-        }
-    };
+    // The wavefront's cells (cell_queue.h): all of them, or the ones that the
+    // residual check listed.  The next cell is sent for while the current
+    // one starts, and its moments, duals and flags are loaded before the
+    // current cell's results are stored, so neither latency stands between
+    // cells.  Wavefront w of workgroup b is worker w gridDim + b: few cells
+    // go to as many workgroups.
+    unsigned long long w_count[7] = {};  // as the launch's counters
+    double w_dt = 1e10;                  // min ComputeDt over this wave's cells (fused path)
+    CellQueue queue((long)wave * gridDim.x + blockIdx.x, (long)gridDim.x * (blockDim.x >> 6), ncells, a.cell_list,
+                    a.counter);
     // a cell's inputs, loaded ahead (a lane's dual of the moments, the duals,
     // the learned start and the residual check's gradient); the kept-inverse
     // flag and the ComputeDt length are wave-uniform.  The kept inverse
@@ -348,7 +315,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         if constexpr (PREC == 2) kf_n = (a.pinv_mode == 1 && cl < a.pinv_slots) ? a.pinv_ok[cl] : 0;
     };
     constexpr int KT = PREC == 2 ? NT : 1, KQ = PREC == 2 ? W::NQ : 1;
-    long next = fetch();
+    long next = queue.first();
     prefetch(next);
     while (next >= 0) {
         const long cell = next;
@@ -375,10 +342,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         const double ue = on ? u_n : 0.0;
         double* lg = a.lam + cell * SM;
         if (on) lamA[dj] = l_n;
-        // phase: queue
-        next = fetch();
+        queue.ask();
         wave_sync();
-        // phase end: queue
 
         double Lk[S];  // Lambda at this lane's point for the last gradient
         double uproj = 0.0;  // <U phiW> of this lane's dual at the last gradient
@@ -577,12 +542,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             where = GIVEN;
             // phase end: start
         }
-        for (;;) {
+        for (bool first = true;; first = false) {
             double gt = 0.0, nt = 0.0;
             if (where != GIVEN) {
                 ++ngrad;
                 nt = gradient(at, gt);
             }
+            if (first) queue.resolve();
             if (where == END) break;
             if (where == TRIAL) {
                 // line search (closure.cpp:159-184): halve the step until
@@ -607,7 +573,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     // Hessian and runs the reference Newton step
                     take = nt < ng;
                     if (take) {
-                        ++w_reuse;
+                        ++w_count[6];
                         // contraction clearly worse than a (damped) Newton
                         // step's: factor afresh at the next Newton step
                         if (!(nt / ng <= 1.2 * (1.0 - c.alpha) + 1e-3)) refactor = true;
@@ -638,7 +604,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                         lamnew = t;
                         g = gt;
                         ng = nt;
-                        ++w_took;
+                        ++w_count[4];
                         ub_lam = true;
                     } else {
                         ub_lam = false;
@@ -730,7 +696,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     if (!spd) {
                         status = UQK_STATUS_NOT_SPD;
                     } else {
-                        ++w_factor;
+                        ++w_count[5];
                         if (c.max_iter == 1) {  // one-shot IPM (closure.cpp:151-154)
                             if (on) lam[dj] -= c.alpha * d;
                             ub_lam = false;
@@ -757,6 +723,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             at = lam;
         }
         // phase: outputs
+        next = queue.take();
         prefetch(next);
         // the cell's slot for the next launch: a usable inverse (1) -- the
         // one just stored, or the kept one while it is fresh -- or none (0)
@@ -790,24 +757,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             if (a.iters) a.iters[cell] = iters;
         }
         // status, iters and ngrad are wave-uniform: these sums stay scalar
-        w_fail += status != UQK_STATUS_CONVERGED ? 1ull : 0ull;
-        w_newton += (unsigned long long)iters;
-        w_grad += (unsigned long long)ngrad;
+        w_count[1] += status != UQK_STATUS_CONVERGED ? 1ull : 0ull;
+        w_count[2] += (unsigned long long)iters;
+        w_count[3] += (unsigned long long)ngrad;
         wave_sync();
         // phase end: outputs
     }
-    if (lane == 0) {
-        if (w_fail) atomicAdd(a.nfail, w_fail);
-        if (w_newton) atomicAdd(a.nfail + 1, w_newton);
-        if (w_grad) atomicAdd(a.nfail + 2, w_grad);
-        if (w_took && a.took) atomicAdd(a.took, w_took);
-        if (a.nfactor) {
-            if (w_factor) atomicAdd(a.nfactor, w_factor);
-            if (w_reuse) atomicAdd(a.nfactor + 1, w_reuse);
-        }
-        // positive doubles order as their bit patterns
-        if (a.dt_min && w_dt < 1e10) atomicMin(a.dt_min, (unsigned long long)__double_as_longlong(w_dt));
-    }
+    add_counts(w_count, w_dt, smem, a.counter, a.dt_min);
 }
 
 // ---------------------------------------------------------------------------
@@ -848,9 +804,7 @@ static void wave_go(const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st
     long want = (a.ncell + waves - 1) / waves;
     int blocks = (int)(want < (long)per_cu * num_cu ? want : (long)per_cu * num_cu);
     if (blocks < 1) blocks = 1;
-    NewtonArgs b = a;
-    set_queue(b, (long)blocks * waves);
-    hipLaunchKernelGGL((newton_wave_kernel<KIND, M, Q, PREC>), dim3(blocks), dim3(threads), shmem, st, b);
+    hipLaunchKernelGGL((newton_wave_kernel<KIND, M, Q, PREC>), dim3(blocks), dim3(threads), shmem, st, a);
     *err = hipGetLastError();
 }
 

@@ -17,7 +17,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kSweepThreads = 256;
 constexpr int kPartialBlocks = 8192;  // grid of the grid-stride sweeps and size of the partials
 
-int sweep_partial_blocks(long) { return kPartialBlocks; }
+int sweep_partial_blocks() { return kPartialBlocks; }
 
 // One thread per (cell, quadrature point): uq(s,k) = U_mat(sum_i lambda(s,i) phi(k,i)).
 #define UQK_SKIP_IF_INACTIVE(a) \
@@ -379,42 +379,63 @@ __global__ void __launch_bounds__(kSweepThreads) mean_var_kernel(SweepArgs a) {
     }
 }
 
-// t < t_end and steps < max_steps and no failed cell: the step runs
 // The end of a replayed step: residual and t (momentsolver.cpp:134-152), run
 // totals, and what the next step's launches need (zero closure counters, the
-// start value 1e10 of ComputeDt's MIN, the active flag; set_recon: the
-// step's closure left its outputs at the current lambda for every cell).
-__global__ void __launch_bounds__(kSweepThreads) step_end_kernel(RunState* rs, double* scalars,
-                                                                 unsigned long long* counters,
-                                                                 const double* partial, int npartial, int set_recon) {
-    if (!rs->active) return;
+// start value 1e10 of ComputeDt's MIN, the active flag: t < t_end and steps <
+// max_steps and no failed cell; set_recon: the step's closure left its outputs
+// at the current lambda for every cell).  One workgroup: what it costs is
+// latency, so all loads are sent at once (10.8 us per step with 256 threads
+// over 8,192 partials).
+constexpr int kEndThreads = 1024;
+__global__ void __launch_bounds__(kEndThreads) step_end_kernel(RunState* rs, double* scalars,
+                                                               unsigned long long* counters,
+                                                               const double* partial, int npartial, int set_recon) {
+    __shared__ unsigned long long total[kCounterLine];
+    __shared__ double red[kEndThreads / 64];
+    const int t = threadIdx.x;
+    const int active = rs->active;
+    const unsigned long long mine = t < kClosureCounters ? counters[t] : 0ull;
+    double v[kPartialBlocks / kEndThreads];
+#pragma unroll
+    for (int i = 0; i < kPartialBlocks / kEndThreads; ++i) {
+        const int at = t + i * kEndThreads;
+        v[i] = at < npartial ? partial[at] : 0.0;
+    }
+    if (!active) return;
+    if (t < kCounterLine) total[t] = 0ull;
+    __syncthreads();
+    if (mine) atomicAdd(&total[t % kCounterLine], mine);
     double m = 0.0;
-    for (int t = threadIdx.x; t < npartial; t += blockDim.x) m += partial[t];
-    m = block_sum(m);
-    if (threadIdx.x == 0) {
-        const double t = rs->t + scalars[0];
+#pragma unroll
+    for (int i = 0; i < kPartialBlocks / kEndThreads; ++i) m += v[i];
+    m = wave_sum(m);
+    if ((t & 63) == 0) red[t >> 6] = m;
+    if (t < kClosureCounters) counters[t] = 0ull;
+    __syncthreads();
+    if (t == 0) {
+        m = red[0];
+        for (int w = 1; w < kEndThreads / 64; ++w) m += red[w];
+        const double time = rs->t + scalars[0];
         const long long steps = rs->steps + 1;
-        const long long nfail = rs->nfail + (long long)counters[1];
-        rs->t = t;
+        const long long nfail = rs->nfail + (long long)total[1];
+        rs->t = time;
         rs->residual = m;
         rs->steps = steps;
         rs->nfail = nfail;
-        rs->newton += (long long)counters[2];
-        rs->gradients += (long long)counters[3];
-        rs->factorizations += (long long)counters[5];
-        rs->reuse_steps += (long long)counters[6];
-#pragma unroll
-        for (int i = 0; i < kClosureCounters; ++i) counters[i] = 0ull;
+        rs->newton += (long long)total[2];
+        rs->gradients += (long long)total[3];
+        rs->factorizations += (long long)total[5];
+        rs->reuse_steps += (long long)total[6];
         scalars[0] = 1e10;
-        rs->active = (t < rs->t_end && (rs->max_steps < 0 || steps < rs->max_steps) && nfail == 0) ? 1 : 0;
+        rs->active = (time < rs->t_end && (rs->max_steps < 0 || steps < rs->max_steps) && nfail == 0) ? 1 : 0;
         if (set_recon) rs->recon = 1;
     }
 }
 
 hipError_t launch_step_end(RunState* rs, double* scalars, unsigned long long* counters, const double* partial,
                            int set_recon, int npartial, hipStream_t st) {
-    hipLaunchKernelGGL(step_end_kernel, dim3(1), dim3(kSweepThreads), 0, st, rs, scalars, counters, partial,
-                       npartial, set_recon);
+    hipLaunchKernelGGL(step_end_kernel, dim3(1), dim3(kEndThreads), 0, st, rs, scalars, counters, partial, npartial,
+                       set_recon);
     return hipGetLastError();
 }
 
@@ -467,15 +488,28 @@ hipError_t launch_reconstruct(const SweepArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
+static int dt_blocks(long ncell) {
+    const long want = (ncell + kSweepThreads - 1) / kSweepThreads;
+    return (int)(want < 1 ? 1 : (want < kPartialBlocks ? want : kPartialBlocks));
+}
 template <int KIND> static void go_dt(const SweepArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(dt_partial_kernel<KIND>, dim3(kPartialBlocks), dim3(kSweepThreads), 0, st, a);
+    hipLaunchKernelGGL(dt_partial_kernel<KIND>, dim3(dt_blocks(a.ncell)), dim3(kSweepThreads), 0, st, a);
 }
 hipError_t launch_dt(int kind, const SweepArgs& a, hipStream_t st) {
     UQK_DISPATCH(kind, go_dt, a, st);
     SweepArgs b = a;
-    b.npartial = kPartialBlocks;
+    b.npartial = dt_blocks(a.ncell);
     hipLaunchKernelGGL(min_finish_kernel, dim3(1), dim3(kSweepThreads), 0, st, b);
     return hipGetLastError();
+}
+
+// Workgroups of the advance, each of which leaves one partial residual: as
+// many as the cells fill, up to kPartialBlocks (a small mesh that launches and
+// sums all of them spends 20 us of its step on that).
+int advance_partials(int S, int Q, long ncell) {
+    const long per = (long)advance_cells_per_wave(S, Q) * (kSweepThreads / 64);
+    const long want = (ncell + per - 1) / per;
+    return (int)(want < 1 ? 1 : (want < kPartialBlocks ? want : kPartialBlocks));
 }
 
 template <int KIND> static void go_advance(const SweepArgs& a, hipStream_t st) {
@@ -485,7 +519,7 @@ template <int KIND> static void go_advance(const SweepArgs& a, hipStream_t st) {
     // PhiW goes to LDS while a workgroup stays within 64 KB
     b.table_lds = shmem + sizeof(double) * a.Q * a.M <= 65536;
     if (b.table_lds) shmem += sizeof(double) * a.Q * a.M;
-    hipLaunchKernelGGL(advance_kernel<KIND>, dim3(kPartialBlocks), dim3(kSweepThreads), shmem, st, b);
+    hipLaunchKernelGGL(advance_kernel<KIND>, dim3(advance_partials(S, a.Q, a.ncell)), dim3(kSweepThreads), shmem, st, b);
 }
 hipError_t launch_advance(int kind, const SweepArgs& a, hipStream_t st) {
     UQK_DISPATCH(kind, go_advance, a, st);
@@ -494,7 +528,7 @@ hipError_t launch_advance(int kind, const SweepArgs& a, hipStream_t st) {
 
 hipError_t launch_residual(const SweepArgs& a, hipStream_t st) {
     SweepArgs b = a;
-    b.npartial = kPartialBlocks;
+    b.npartial = advance_partials(a.S, a.Q, a.ncell);
     hipLaunchKernelGGL(sum_finish_kernel, dim3(1), dim3(kSweepThreads), 0, st, b);
     return hipGetLastError();
 }

@@ -56,7 +56,6 @@ uqk::SweepArgs sweep_args(const uqk_ctx* ctx) {
     a.phiw = ctx->d_phiw;
     a.xi = ctx->d_xi;
     a.partial = ctx->d_partial;
-    a.npartial = uqk::sweep_partial_blocks(0);
     return a;
 }
 
@@ -179,7 +178,7 @@ bool wave_check(const uqk_ctx* ctx, bool per_cell_orders) {
            uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, 1, &wm, &wo);
 }
 
-// Launch the Newton closure kernel; leaves the failed-cell count in counters[1]
+// Launch the Newton closure kernel; leaves the failed-cell counts in counters
 // (counters: the context's d_counters unless the caller brings its own
 // kClosureCounters).
 // When uq_out/u_out are given and the specialised or the workgroup kernel runs
@@ -200,7 +199,6 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
     if (!counters) counters = ctx->d_counters;
     // (in a replayed run the previous step's step_end_kernel already cleared
     // the counters and set dt's start value: prezeroed)
-    // [0] queue head, [1] failed cells, [2] Newton steps, [3] gradients, [4] cells that took the learned start
     if (!prezeroed) UQK_HIP(ctx, uqk::launch_fill_u64(counters, uqk::kClosureCounters, ctx->stream));
     if (n <= 0) return 0;
     // learned warm start: the network's prediction (per-cell orders: masked
@@ -479,9 +477,13 @@ int collect_step_times(uqk_ctx* ctx) {
 
 int64_t finish_closure(uqk_ctx* ctx, const unsigned long long* counters = nullptr) {
     if (!counters) counters = ctx->d_counters;
-    UQK_HIP(ctx, hipMemcpyAsync(ctx->last_stats, counters + 1, sizeof(ctx->last_stats), hipMemcpyDeviceToHost,
-                                ctx->stream));  // counters 1..6
+    unsigned long long lines[uqk::kClosureCounters];
+    UQK_HIP(ctx, hipMemcpyAsync(lines, counters, sizeof(lines), hipMemcpyDeviceToHost, ctx->stream));
     UQK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for (int i = 0; i < 6; ++i) {  // counters 1..6
+        ctx->last_stats[i] = 0;
+        for (int l = 0; l < uqk::kCounterLines; ++l) ctx->last_stats[i] += lines[l * uqk::kCounterLine + 1 + i];
+    }
     float ms = 0.f;
     ctx->last_closure_ms = 0.0;
     if (ctx->timed) UQK_HIP(ctx, hipEventElapsedTime(&ms, ctx->tev0, ctx->tev1));
@@ -584,7 +586,7 @@ int uqk_create(const uqk_desc* desc, uqk_ctx** out) {
         UQK_HIP(ctx, hipMemcpy(ctx->d_xi, desc->xi, xb, hipMemcpyHostToDevice));
     }
     UQK_HIP(ctx, hipMalloc(&ctx->d_counters, uqk::kClosureCounters * sizeof(unsigned long long)));
-    UQK_HIP(ctx, hipMalloc(&ctx->d_partial, sizeof(double) * uqk::sweep_partial_blocks(0)));
+    UQK_HIP(ctx, hipMalloc(&ctx->d_partial, sizeof(double) * uqk::sweep_partial_blocks()));
     UQK_HIP(ctx, hipMalloc(&ctx->d_scalars, 4 * sizeof(double)));
     UQK_HIP(ctx, hipStreamCreate(&ctx->own_stream));
     ctx->stream = ctx->own_stream;
@@ -919,7 +921,8 @@ int64_t uqk_run_steps(uqk_ctx* ctx, const uqk_problem* prob, const uqk_mesh* mes
         ctx->check_mode = 0;
         if (rc) return rc;
         UQK_HIP(ctx, uqk::launch_step_end(ctx->d_run, ctx->d_scalars, ctx->d_counters, ctx->d_partial,
-                                          ctx->step_recon ? 1 : 0, uqk::sweep_partial_blocks(0), ctx->stream));
+                                          ctx->step_recon ? 1 : 0,
+                                          uqk::advance_partials(ctx->S, ctx->Q, mesh->n_cells), ctx->stream));
         return 0;
     };
     const int64_t limit = max_steps < 0 ? INT64_MAX : max_steps;

@@ -23,8 +23,7 @@ struct uqk_ctx {
     double* d_phi = nullptr;
     double* d_phiw = nullptr;
     double* d_xi = nullptr;
-    unsigned long long* d_counters = nullptr;  // [0] queue head, [1] failed cells, [2] Newton steps, [3] gradients,
-                                               // [4] cells that took the learned warm start
+    unsigned long long* d_counters = nullptr;  // kClosureCounters
     double* d_partial = nullptr;               // per-block partials
     double* d_scalars = nullptr;               // [0] dt, [1] residual
     hipStream_t own_stream = nullptr;

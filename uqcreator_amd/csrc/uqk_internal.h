@@ -101,12 +101,15 @@ struct RunState {
     int recon;
 };
 
-// Closure counters of a launch: [0] work-queue head, [1] failed cells, [2]
-// Newton steps, [3] gradient evaluations, [4] cells that started from the
-// learned warm start, [5] Cholesky factorisations, [6] steps on a kept
-// inverse, [7] unused, [8] cells the residual check left to the Newton
-// kernel; all zero at launch.
-constexpr int kClosureCounters = 9;
+// Closure counters of a launch, in kCounterLines cache lines whose entries
+// add up: [0] work-queue head, [1] failed cells, [2] Newton steps, [3]
+// gradient evaluations, [4] cells that started from the learned warm start,
+// [5] factorisations, [6] steps on a kept factor or inverse; in the first
+// line also [8] cells the residual check left to the Newton kernel.  All zero
+// at launch.
+constexpr int kCounterLines = 16;
+constexpr int kCounterLine = 16;
+constexpr int kClosureCounters = kCounterLines * kCounterLine;
 
 // Launch shape of the specialised closure kernel; 0 = automatic (as many
 // waves per workgroup as LDS allows, every resident workgroup slot filled).
@@ -212,7 +215,10 @@ hipError_t launch_residual(const SweepArgs& a, hipStream_t st);
 hipError_t launch_mean_var(int kind, const SweepArgs& a, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, int n, hipStream_t st);
 hipError_t launch_fill_f64(double* p, int n, double v, hipStream_t st);
-int sweep_partial_blocks(long ncell);
+// Largest number of partial results the sweeps leave, and the advance's for
+// a mesh (one per workgroup).
+int sweep_partial_blocks();
+int advance_partials(int S, int Q, long ncell);
 // End of a replayed step (momentsolver.cpp:134-152): residual = sum of the
 // advance's per-block partials, t += dt, the step's closure counts into the
 // run totals; then clears the closure counters, sets the fused dt's start value
