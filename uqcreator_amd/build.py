@@ -44,6 +44,10 @@ EXTRA_FLAGS = {
     "closure_wave.hip": ["-mllvm", "-disable-machine-licm"],
     "closure_wave_lag.hip": ["-mllvm", "-disable-machine-licm"],
     "closure_wave_reuse.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_tile_barrier.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_tile_euler1d.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_tile_euler2d.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_tile_shallow.hip": ["-mllvm", "-disable-machine-licm"],
 }
 
 

@@ -1,4 +1,6 @@
-// closure_fp64.hip -- batched FP64 Newton dual closure, one wavefront per cell.
+// closure_fp64.hip -- batched FP64 Newton dual closure, one wavefront per cell,
+// for systems too large for closure_tile_kernel.h and closure_block.hip (or
+// where the generic kernel is asked for at 64 duals and more).
 //
 // Restates Closure::SolveClosure / SolveClosureSafe (closure.cpp:133-193,
 // :297-339) for a whole batch of cells:

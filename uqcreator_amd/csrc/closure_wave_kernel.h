@@ -92,14 +92,6 @@ template <int PREC> constexpr bool wave_reuses = PREC == 2 || PREC == 4;
 // the inverse from the registers, the lower triangle otherwise
 template <int PREC, int NT> constexpr int wave_tiles = PREC == 4 ? NT * NT : NT * (NT + 1) / 2;
 
-// basis pair (j <= i) of number e = i (i + 1) / 2 + j, from its root (e < 2^12)
-__device__ __forceinline__ void basis_pair(int e, int& j, int& i) {
-    i = (int)((__builtin_amdgcn_sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
-    i -= i * (i + 1) / 2 > e ? 1 : 0;
-    i += (i + 1) * (i + 2) / 2 <= e ? 1 : 0;
-    j = e - i * (i + 1) / 2;
-}
-
 // The system of a Newton step at the iterate whose Lambda lies at this lane's
 // point in Lk, into bh: the pair products (pairs x points)(points x state
 // pairs) on FP64 matrix steps; with RHS also the gradient g of this lane's

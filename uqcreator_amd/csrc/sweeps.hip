@@ -303,7 +303,11 @@ __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per
                         const int nt = a.nt_cell ? a.nt_cell[c] : M;
                         const int bcc = a.bc[c];
                         const int f = ic * S + st;
-                        const double us = a.u[c * SM + f];  // reconstructed moments
+                        double us = a.u[c * SM + f];        // reconstructed moments
+                        if (a.cut && ic >= nt) {             // past the order that the refinement chose
+                            us = 0.0;
+                            a.cut[c * SM + f] = 0.0;
+                        }
                         double* un = a.u_out + c * SM;       // in: previous moments, out: new moments
                         const double old = un[f];
                         double v = us;

@@ -91,6 +91,14 @@ __device__ __forceinline__ void group_transpose(double (&d)[4]) {
     swap_rows(d[2], d[3]);
 }
 
+// basis pair (j <= i) of number e = i (i + 1) / 2 + j, from its root (e < 2^12)
+__device__ __forceinline__ void basis_pair(int e, int& j, int& i) {
+    i = (int)((__builtin_amdgcn_sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
+    i -= i * (i + 1) / 2 > e ? 1 : 0;
+    i += (i + 1) * (i + 2) / 2 <= e ? 1 : 0;
+    j = e - i * (i + 1) / 2;
+}
+
 // tile (tc, tr), tc <= tr, of the lower triangle
 __host__ __device__ constexpr int tile_lower(int tc, int tr) { return tr * (tr + 1) / 2 + tc; }
 
@@ -153,6 +161,7 @@ __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[NT * (NT + 1) / 2], int n, i
         double P[NT], W[NT];
 #pragma unroll
         for (int r = jb; r < NT; ++r) {
+            if (16 * r > n) break;  // (tiles past row n hold nothing)
             P[r] = T[tile_lower(jb, r)][e];
             if (r == jb && !(p >= j0 + (have < 4 ? have : 4))) P[r] = 0.0;  // finished rows
             if (have < 4 && q >= have) P[r] = 0.0;       // columns that are no pivots
@@ -161,12 +170,14 @@ __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[NT * (NT + 1) / 2], int n, i
         }
         if (4 * b + 4 < n) {
 #pragma unroll
-            for (int r = jb; r < NT; ++r)
+            for (int r = jb; r < NT; ++r) {
+                if (16 * r > n) break;
 #pragma unroll
                 for (int c = jb; c <= r; ++c)
                     if (16 * c < n)
                         T[tile_lower(c, r)] =
                             __builtin_amdgcn_mfma_f64_16x16x4f64(P[c], -W[r], T[tile_lower(c, r)], 0, 0, 0);
+            }
         }
     }
     return ok;
@@ -187,7 +198,8 @@ __device__ __forceinline__ double tile_back(const f64x4 (&T)[NT * (NT + 1) / 2],
         const int jb = b >> 2, e = b & 3, have = n - 4 * b;
         double s = 0.0;
 #pragma unroll
-        for (int r = jb; r < NT; ++r) s = fma(-T[tile_lower(jb, r)][e], X[r], s);
+        for (int r = jb; r < NT; ++r)
+            if (16 * r <= n) s = fma(-T[tile_lower(jb, r)][e], X[r], s);
         s = row_sum(s);
         const double x0 = lane_get(s, 0), x1 = lane_get(s, 16), x2 = lane_get(s, 32), x3 = lane_get(s, 48);
         const double v = p2 ? (p1 ? x3 : x2) : (p1 ? x1 : x0);

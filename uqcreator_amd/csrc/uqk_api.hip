@@ -186,12 +186,14 @@ bool wave_check(const uqk_ctx* ctx, bool per_cell_orders) {
 // is set.
 // With dt_out as well (the step), the fused kernels also reduce
 // Problem::ComputeDt over the cells into *dt_out and *fused_dt is set.
+// refining: the refinement follows, which may raise a cell's order, so only a
+// kernel that leaves all moments (the runtime-sized one) fuses.
 int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, double* lam, int32_t* status,
                    int32_t* iters, const int* active = nullptr, double* uq_out = nullptr, double* u_out = nullptr,
                    bool* fused = nullptr, double* dt_out = nullptr, const uqk::ProblemParams* dtp = nullptr,
                    const double* dx_param = nullptr, bool* fused_dt = nullptr,
                    unsigned long long* counters = nullptr, bool prezeroed = false, bool factors_per_cell = false,
-                   const int* recon_ok = nullptr) {
+                   const int* recon_ok = nullptr, bool refining = false) {
     if (fused) *fused = false;
     if (fused_dt) *fused_dt = false;
     ctx->timed = false;
@@ -309,9 +311,10 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
     if (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64 && block_ok)) {
         if (!block_ok) return fail(ctx, -3, "closure too large for the workgroup kernel");
         if (a.pinv_mode == 1 && ctx->factor_mode != 2) a.pinv_mode = 0;  // (the slots hold inverses)
-        const bool fuse = uq_out && u_out && ctx->c.max_iter != 1;
+        const bool fuse = uq_out && u_out && ctx->c.max_iter != 1 && !refining;
         a.uq_out = fuse ? uq_out : nullptr;
         a.u_out = fuse ? u_out : nullptr;
+        if (!fuse) a.dt_min = nullptr;
         const bool check = fuse && ctx->residual_check && !ctx->c.safe &&
                            uqk::closure_check_wave_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
         // learned start: the residual check chooses it for the cells that
@@ -344,12 +347,26 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
         ctx->last_kernel = UQK_KERNEL_BLOCK;
         ctx->timed = ev;
         if (fused) *fused = fuse;
-        if (fused_dt) *fused_dt = want_dt;
+        if (fused_dt) *fused_dt = want_dt && fuse;
         return 0;
     }
     if (lam_alt)
         if (int rc = uqk::enqueue_warm_select(ctx, n, u, lam, lam_alt, active, nt)) return rc;
     ctx->last_kernel = UQK_KERNEL_GENERIC;
+    if (uqk::newton_tile_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds)) {
+        const bool fuse = uq_out && u_out && ctx->c.max_iter != 1;
+        a.uq_out = fuse ? uq_out : nullptr;
+        a.u_out = fuse ? u_out : nullptr;
+        a.all_moments = refining;
+        if (!fuse) a.dt_min = nullptr;
+        if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev0, ctx->stream));
+        UQK_HIP(ctx, uqk::newton_tile_launch(ctx->kind, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream));
+        if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev1, ctx->stream));
+        ctx->timed = ev;
+        if (fused) *fused = fuse;
+        if (fused_dt) *fused_dt = want_dt && fuse;
+        return 0;
+    }
     a.uq_out = nullptr;
     a.u_out = nullptr;
     a.dt_min = nullptr;
@@ -394,7 +411,9 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
 // sets dt's start value and sums the residual (no fills, no residual kernel).
 // With refinement on (ctx->refine.nlev > 1) the levels move between uQ and the
 // reconstruction, as in momentsolver.cpp:99-124: the closure and uQ use the
-// old nTotal, the reconstruction and the advance the new one.
+// old nTotal, the reconstruction and the advance the new one (where the
+// closure kernel leaves the moments it leaves all of them, and the advance
+// cuts them at the new order).
 int enqueue_step(uqk_ctx* ctx, const uqk_problem* prob, const uqk_mesh* mesh, int32_t* nt, double* u,
                  double* lam, double* uq, double* u_scratch, int32_t* status, int32_t* iters, const int* active,
                  bool in_run = false) {
@@ -417,9 +436,9 @@ int enqueue_step(uqk_ctx* ctx, const uqk_problem* prob, const uqk_mesh* mesh, in
         ea0 = ctx->kev[ctx->kev_used + 2];
         ea1 = ctx->kev[ctx->kev_used + 3];
     }
-    int rc = launch_closure(ctx, n, nt, u, lam, status, iters, active, refining ? nullptr : uq,
-                            refining ? nullptr : u_scratch, &fused, ctx->d_scalars, &pp, mesh->dx_param, &fused_dt,
-                            nullptr, in_run, true, in_run ? &ctx->d_run->recon : nullptr);
+    int rc = launch_closure(ctx, n, nt, u, lam, status, iters, active, uq, u_scratch, &fused, ctx->d_scalars, &pp,
+                            mesh->dx_param, &fused_dt, nullptr, in_run, true, in_run ? &ctx->d_run->recon : nullptr,
+                            refining);
     ctx->cev0 = ctx->cev1 = nullptr;
     if (rc) return rc;
     uqk::SweepArgs a = sweep_args(ctx);
@@ -446,6 +465,7 @@ int enqueue_step(uqk_ctx* ctx, const uqk_problem* prob, const uqk_mesh* mesh, in
     if (!fused_dt) UQK_HIP(ctx, uqk::launch_dt(ctx->kind, a, ctx->stream));
     a.u = u_scratch;
     a.u_out = u;
+    a.cut = fused && refining ? u_scratch : nullptr;
     a.dt_dev = ctx->d_scalars;
     if (kt) UQK_HIP(ctx, hipEventRecord(ea0, ctx->stream));
     UQK_HIP(ctx, uqk::launch_advance(ctx->kind, a, ctx->stream));

@@ -29,6 +29,7 @@ struct NewtonArgs {
     const int* active;           // device flag: 0 skips the launch (graph replays past t_end)
     double* uq_out;              // wave kernel, when not null: U at the quadrature points of the
     double* u_out;               // returned lambda and its moments <U phiW> (fused uQ + reconstruction)
+    int all_moments;             // runtime-sized kernel: u_out past a cell's order too (not zero there)
     long waves;                  // resident waves of the launch (work-queue chunking), set by the launcher
     int qbits;                   // work queue of 2^qbits positions >= ncell, set by the launcher
     // with uq_out, when dt_min is not null: also min over cells and points of
@@ -144,6 +145,10 @@ long newton_wave_kept_floats(int S, int M);
 // CU at `waves` for the specialised kernel of (kind, M, Q, prec); false when
 // there is none.
 bool newton_wave_limits(int kind, int M, int Q, int prec, int max_lds, int waves, int* max_waves, int* occupancy);
+// runtime-sized kernel for n = S*M < 64, any Q that the LDS holds, per-cell
+// orders (closure_tile_kernel.h)
+bool newton_tile_fits(int S, int M, int Q, int max_lds);
+hipError_t newton_tile_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st);
 int newton_fp64_wave_doubles(int S, int M, int Q);
 // workgroup-per-cell kernel for n = S*M up to 256 (closure_block.hip)
 bool newton_block_fits(int S, int M, int Q, int max_lds);
@@ -187,6 +192,7 @@ struct SweepArgs {
     int npartial;
     double* scalar_out;          // final reduction result
     const int* active;           // device flag: 0 skips the launch
+    double* cut;                 // advance, when not null: u again, whose moments past a cell's order become zero
     int table_lds;               // advance: PhiW staged in LDS (set by the launcher)
 };
 
