@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
         }
         __syncthreads();
 
-        double Lk[S];  // Lambda at this thread's point (tid < Q) of the last gradient
+        double Lk[S], rk = 0.0;  // Lambda and density at this thread's point (tid < Q) of the last gradient
         double uproj = 0.0;  // <U phiW> of this thread's dual (tid < n) at the last gradient
         // <Ub phiW>: out(s, i) = sum_k Ub(s, k) phiW(k, i), state-major
         // (e = s nt + i), as FP64 MFMA tiles of the product (S x Q)(Q x nt):
@@ -225,6 +225,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
                 double Uv[S];
                 point_lambda(X);
                 closure_U<KIND>(c, Lk, Uv);
+                rk = Uv[0];
 #pragma unroll
                 for (int s = 0; s < S; ++s) Ub[s * Q + k] = Uv[s];
             }
@@ -261,7 +262,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
 #pragma unroll
                     for (int s = 0; s < S; ++s) Ld[s] += v[s * nt + i] * p;
                 }
-                closure_DU<KIND>(c, Lk, y);
+                closure_DU<KIND>(c, Lk, rk, y);
 #pragma unroll
                 for (int l = 0; l < S; ++l) {
                     double w = 0.0;
@@ -277,7 +278,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
 
         auto hessian = [&]() {
             // phase: hessian
-            if (tid < Q) closure_DU<KIND>(c, Lk, DUk + tid * P);
+            if (tid < Q) closure_DU<KIND>(c, Lk, rk, DUk + tid * P);
             __syncthreads();
             // every state block H_lm = Phi^T diag(DU_lm) PhiW (m <= l) on MFMA
             // tiles of 16 x 16, k in steps of 4, FP64 (PREC 0) or FP32 with
@@ -761,7 +762,12 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
         if (a.grad_at_lam) {
             // the residual check's gradient at lambda (its projection summed
             // in point order); Lambda at the points for the first Hessian
-            if (tid < Q) point_lambda(lam);
+            if (tid < Q) {
+                double Uv[S];
+                point_lambda(lam);
+                closure_U<KIND>(c, Lk, Uv);
+                rk = Uv[0];
+            }
             double sq = 0.0;
             if (tid < n) {
                 const int l = tid / nt, i = tid - l * nt;
@@ -827,9 +833,10 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
                     solve_kept();
                     if (tid < n) dv[tid] += d1;
                     __syncthreads();
-                    double Lk0[S];
+                    double Lk0[S], rk0;
 #pragma unroll
                     for (int s = 0; s < S; ++s) Lk0[s] = Lk[s];
+                    rk0 = rk;
                     const double nnew = trial(1.0);
                     if (nnew < ng) {
                         ++w_reuse;
@@ -851,6 +858,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
                     } else {
 #pragma unroll
                         for (int s = 0; s < S; ++s) Lk[s] = Lk0[s];
+                        rk = rk0;
                         // g stays: the swap at the next iteration's start
                         // brings it back
                         double* t = g;

@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) newton_fp64_kernel(NewtonArgs a) {
 
         // Hessian at the iterate whose Lambda(x_k) is in Lk (closure.cpp:255-271).
         auto hessian = [&]() {
-            for (int k = lane; k < Q; k += 64) closure_DU<KIND>(c, Lk + k * S, DUk + k * P);
+            for (int k = lane; k < Q; k += 64) closure_DU<KIND>(c, Lk + k * S, Uk[k * S], DUk + k * P);
             wave_sync();
             const int npair = nt * (nt + 1) / 2;
             for (int e = lane; e < npair; e += 64) {

@@ -13,8 +13,9 @@
 // What bounds it: the latency of a cell's chain, as in the wave kernel.  It
 // replaced a column-by-column Cholesky in LDS (closure_fp64.hip, which is
 // left with the systems of 64 duals and more): Euler 2D, 65,536 cells on
-// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 26.2 ms
-// against 51.7.
+// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 22.8 ms
+// against 52.6 (26.2 with DU through the exponential and with the lane's
+// numbers kept over the cell: 4 to 48 registers spilled).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -82,9 +83,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         // not kept in registers over the loop)
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));
-        const int p16 = lane & 15, q4 = lane >> 4;
-        const int s4 = (p16 & 3) < S ? (p16 & 3) : S - 1;  // this lane's state as an operand row
+        int p16 = lane & 15, q4 = lane >> 4;
+        int s4 = (p16 & 3) < S ? (p16 & 3) : S - 1;  // this lane's state as an operand row
         queue.ask();
+        // phase: inputs
         const int nt = a.nt_cell ? __builtin_amdgcn_readfirstlane(a.nt_cell[cell]) : M;
         const int n = S * nt;
         const double* ug = a.u + cell * SM;
@@ -102,10 +104,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         for (int t = lane; t < n; t += 64) lam[t] = lg[t];
         const double dx = a.uq_out && a.dt_min ? a.dx_param[cell] : 0.0;
         wave_sync();
+        // phase end: inputs
 
         double uproj[DT];
         // ||grad L|| at the duals X (LDS): U at the points in Ub, Lambda in DUb, gradient in gout
         auto gradient = [&](const double* X, double (&gout)[DT]) -> double {
+            // phase: gradient
             for (int p0 = 0; p0 < Q; p0 += 64) {
                 double t4[4] = {0.0, 0.0, 0.0, 0.0};
                 for (int ki = 0; 4 * ki < nt; ++ki) {
@@ -151,16 +155,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             }
             const double nrm = sqrt(wave_sum(sq));
             wave_sync();
+            // phase end: gradient
             return nrm;
         };
         // Newton direction at the iterate of the last gradient; false if the
         // Hessian is not positive definite
         auto direction = [&](const double (&g)[DT], double (&d)[DT]) -> bool {
+            // phase: hessian
             for (int k = lane; k < QP; k += 64) {
                 double L[S], y[P];
 #pragma unroll
                 for (int s = 0; s < S; ++s) L[s] = DUb[s * QP + k];
-                closure_DU<KIND>(c, L, y);
+                closure_DU<KIND>(c, L, Ub[k], y);  // (the last gradient was lam's)
 #pragma unroll
                 for (int p = 0; p < P; ++p) DUb[p * QP + k] = y[p];
             }
@@ -206,6 +212,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             for (int t = 0; t < DT; ++t)
                 if (on[t]) H[n * (n + 1) / 2 + q4 * nt + p16 + 16 * t] = g[t];
             wave_sync();
+            // phase end: hessian
+            // phase: load
             f64x4 T[TILES];
 #pragma unroll
             for (int tr = 0; tr < NT; ++tr)
@@ -219,8 +227,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                         const double v = H[in ? hi * (hi + 1) / 2 + lo : 0];
                         T[tile_lower(tc, tr)][e] = in ? v : 0.0;
                     }
+            // phase end: load
+            // phase: factor
             const bool spd = tile_ldl<NT>(T, n, p16, q4);
+            // phase end: factor
+            // phase: backsub
             yb[lane] = tile_back<NT>(T, n, p16, q4);
+            // phase end: backsub
             wave_sync();
 #pragma unroll
             for (int t = 0; t < DT; ++t) d[t] = on[t] ? yb[q4 * nt + p16 + 16 * t] : 0.0;
@@ -234,7 +247,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         bool ub_lam = false;  // Ub and uproj belong to lam
         enum { START, TRIAL, END };
         int where = START;
+        asm volatile("" : "+s"(where));  // (not cloned for its first pass)
         for (;;) {
+            // (and for each pass, for the same reason)
+            asm volatile("" : "+v"(lane));
+            p16 = lane & 15;
+            q4 = lane >> 4;
+            s4 = (p16 & 3) < S ? (p16 & 3) : S - 1;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) on[t] = q4 < S && p16 + 16 * t < nt;
             ++ngrad;
             const double nt_norm = gradient(where == TRIAL ? lamnew : lam, gt);
             if (where == END) break;
@@ -306,6 +327,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             if (!a.uq_out || ub_lam) break;
             where = END;
         }
+        // phase: outputs
         for (int t = lane; t < n; t += 64) lg[t] = lam[t];
         if (a.uq_out) {
             // uQ = U(lambda phi) (momentsolver.cpp:100) and u = <uQ phiW>
@@ -339,6 +361,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         w_count[2] += (unsigned long long)iters;
         w_count[3] += (unsigned long long)ngrad;
         wave_sync();
+        // phase end: outputs
     }
     add_counts(w_count, w_dt, smem, a.counter, a.dt_min);
 }

@@ -25,15 +25,20 @@
 //     explicit inverse where steps reuse it, in registers: tile_solve.h.
 //
 // What bounds it: the latency of one cell's chain of dependent steps at two
-// wavefronts per SIMD.  Cycles per call at n = 40, 25 points (Euler 2D, FP64):
-// factorisation 13.1 K and back substitution 3.4 K (register tiles spread
-// over the wave with one LDS round trip per two pivots: 23.4 K and 19.2 K),
-// Hessian 5.8 K (pairs over lanes, DU by v_readlane: 14.6 K), gradient 3.6 K
-// (4.3 K); 65,536 cells, 40 time steps: 26.3 ms against 39.1 (FP64), 22.9
-// against 30.8 (mixed).  At n = 45, 49 points, one closure of 100,003 cells:
-// 35.2 ms against 47.0 (FP64), 10.8 against 19.5 (mixed: a step on the kept
-// inverse is a matrix-vector product from registers, 1.2 K cycles, in place
+// wavefronts per SIMD, most of it instruction issue.  Cycles per call at n =
+// 40, 25 points (Euler 2D, FP64): factorisation 13.1 K and back substitution
+// 3.4 K (register tiles spread over the wave with one LDS round trip per two
+// pivots: 23.4 K and 19.2 K), Hessian 3.7 K (pairs over lanes, DU by
+// v_readlane, with an exponential and a logarithm: 14.6 K), gradient 3.6 K
+// (4.3 K); 65,536 cells, 40 time steps: 21.4 ms against 39.0 (FP64), 16.5
+// against 30.7 (mixed).  At n = 45, 49 points, one closure of 100,003 cells:
+// 30.4 ms against 47.4 (FP64), 10.2 against 19.5 (mixed: a step on the kept
+// inverse is a matrix-vector product from registers, 1.3 K cycles, in place
 // of two triangular solves from LDS, 13.9 K).
+// The next cell's moments, duals, density and kept inverse are asked for
+// while this cell still computes and are waited for before its results are
+// stored: loads come back in order behind the stores that precede them, and
+// asked for at the cell's end they cost 2.1 ms more over the mixed loop above.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -92,17 +97,17 @@ template <int PREC> constexpr bool wave_reuses = PREC == 2 || PREC == 4;
 // the inverse from the registers, the lower triangle otherwise
 template <int PREC, int NT> constexpr int wave_tiles = PREC == 4 ? NT * NT : NT * (NT + 1) / 2;
 
-// The system of a Newton step at the iterate whose Lambda lies at this lane's
-// point in Lk, into bh: the pair products (pairs x points)(points x state
+// The system of a Newton step at the iterate whose Lambda and density lie at
+// this lane's point in Lk and rk, into bh: the pair products (pairs x points)(points x state
 // pairs) on FP64 matrix steps; with RHS also the gradient g of this lane's
 // dual (the right-hand side).  smem: the workgroup's tables, bh: the wave's.
 template <int KIND, int M, int Q, bool RHS, class D>
-__device__ __forceinline__ void wave_system(const ClosureParams& c, const double* Lk, double g, D* smem, D* bh,
-                                            int lane, int p16, int q4) {
+__device__ __forceinline__ void wave_system(const ClosureParams& c, const double* Lk, double rk, double g, D* smem,
+                                            D* bh, int lane, int p16, int q4) {
     using W = WaveShape<KIND, M, Q>;
     constexpr int S = W::S, P = W::P, QP = W::QP, KS = W::KS;
     double y[P];
-    closure_DU<KIND>(c, Lk, y);
+    closure_DU<KIND>(c, Lk, rk, y);
     if (lane < QP) {
 #pragma unroll
         for (int p = 0; p < P; ++p) bh[p * QP + lane] = y[p];
@@ -164,14 +169,14 @@ typedef __attribute__((address_space(3))) double lds_double;
 typedef __attribute__((address_space(3))) unsigned lds_unsigned;
 template <int KIND, int M, int Q>
 __device__ __attribute__((noinline)) bool sweep_step(ClosureParams c, double L0, double L1, double L2, double L3,
-                                                     double g, lds_double* smem, lds_double* wb, float* Pg) {
+                                                     double rk, double g, lds_double* smem, lds_double* wb, float* Pg) {
     using W = WaveShape<KIND, M, Q>;
     constexpr int N = W::N, NT = W::NT, TILES = NT * (NT + 1) / 2, NQ = W::NQ;
     const int lane = threadIdx.x & 63, p16 = lane & 15, q4 = lane >> 4;
     lds_double *bh = wb + W::BH, *yb = wb + W::YB;
     const lds_unsigned* addr = (lds_unsigned*)(smem + W::ADDR);
     const double Lk[4] = {L0, L1, L2, L3};
-    wave_system<KIND, M, Q, true>(c, Lk, g, smem, bh, lane, p16, q4);
+    wave_system<KIND, M, Q, true>(c, Lk, rk, g, smem, bh, lane, p16, q4);
     f64x4 T[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -215,8 +220,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     const int active = a.active ? *a.active : 1;
     const long ncells = a.cell_list ? (long)*a.cell_count : a.ncell;
     if (!active || (long)blockIdx.x >= ncells) return;  // no cell for any wavefront of this workgroup
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p16 = lane & 15, q4 = lane >> 4;
+    int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    int p16 = lane & 15, q4 = lane >> 4;
     double* phiT = smem;              // phiT[i*QP + k]  = phi(k, i), zero past Q
     double* phiwT = smem + W::PHIW;   // phiwT[i*QP + k] = phiw(k, i)
     for (int t = threadIdx.x; t < W::PHIW; t += blockDim.x) {
@@ -273,8 +279,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
 
     // this lane's dual (s, i) = (q4, p16): its place in a cell's arrays and
     // its unknown in the system
-    const bool on = q4 < S && p16 < M;
-    const int dj = on ? p16 * S + q4 : 0, de = on ? q4 * M + p16 : 0;
+    bool on = q4 < S && p16 < M;
+    int dj = on ? p16 * S + q4 : 0, de = on ? q4 * M + p16 : 0;
+    // the lane's coordinates anew: the masks and LDS addresses that derive
+    // from them are then formed where they are used instead of being kept in
+    // registers over a loop
+    auto renew = [&]() {
+        asm volatile("" : "+v"(lane));
+        p16 = lane & 15;
+        q4 = lane >> 4;
+        on = q4 < S && p16 < M;
+        dj = on ? p16 * S + q4 : 0;
+        de = on ? q4 * M + p16 : 0;
+    };
     const ClosureParams& c = a.c;
     const int SM = S * M;
 
@@ -293,7 +310,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     // flag and the ComputeDt length are wave-uniform.  The kept inverse
     // itself is loaded ahead too: its registers are free once a cell's last
     // step is taken.
-    double u_n = 0.0, l_n = 0.0, la_n = 0.0, dx_n = 0.0, g_n = 0.0;
+    // They are sent for once the cell's first direction is known; the reuse
+    // across time steps has no registers for them then, and sends for them at
+    // the cell's end.
+    constexpr bool kEarly = PREC != 2;
+    // (with the check's gradient also the density at the point, of the uQ that
+    // the check or the last step left at lambda)
+    constexpr bool kDensity = KIND == UQK_EULER1D || KIND == UQK_EULER2D;
+    double u_n = 0.0, l_n = 0.0, la_n = 0.0, dx_n = 0.0, g_n = 0.0, rk_n = 0.0;
     int kf_n = 0;
     auto prefetch = [&](long cl) {
         if (cl < 0) return;
@@ -303,16 +327,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             if (a.lam_alt) la_n = a.lam_alt[cl * SM + dj];
             if (a.grad_at_lam) g_n = a.grad_at_lam[cl * SM + dj];
         }
+        if (kDensity && a.grad_at_lam) rk_n = a.uq_out[(cl * Q + (lane < Q ? lane : Q - 1)) * S];
         if (a.uq_out && a.dt_min) dx_n = a.dx_param[cl];
         if constexpr (PREC == 2) kf_n = (a.pinv_mode == 1 && cl < a.pinv_slots) ? a.pinv_ok[cl] : 0;
     };
     constexpr int KT = PREC == 2 ? NT : 1, KQ = PREC == 2 ? W::NQ : 1;
+    // waits for the inputs: what is stored next is then not waited for with
+    // them (loads and stores are counted in one order)
+    auto arrive = [&]() {
+        asm volatile("" : "+v"(u_n), "+v"(l_n), "+v"(la_n), "+v"(g_n), "+v"(rk_n), "+v"(dx_n), "+v"(kf_n));
+        kf_n = __builtin_amdgcn_readfirstlane(kf_n);
+    };
     long next = queue.first();
     prefetch(next);
+    arrive();
     while (next >= 0) {
         const long cell = next;
-        const double la_c = la_n, dx_c = dx_n, g_c = g_n;
-        const int kf_c = __builtin_amdgcn_readfirstlane(kf_n);
+
+        const double la_c = la_n, dx_c = dx_n, g_c = g_n, rk_c = rk_n;
+        const int kf_c = kf_n;
         // the kept inverse, sent for before Lambda at the points is formed
         // (lanes past row N - 1 repeat it; their sums are not used)
         float kept[KT][KQ];
@@ -337,7 +370,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         queue.ask();
         wave_sync();
 
-        double Lk[S];  // Lambda at this lane's point for the last gradient
+        double Lk[S], rk = rk_c;  // Lambda and density at this lane's point for the last gradient
         double uproj = 0.0;  // <U phiW> of this lane's dual at the last gradient
         // sum_k Ub(s, k) phiW(k, i) for this lane's dual (s, i): the product
         // (S x Q)(Q x M) in steps of four points; its lane layout is the duals'
@@ -387,6 +420,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             }
 #pragma unroll
             for (int s = 0; s < S; ++s) Lk[s] = L[s];
+            rk = Uv[0];
             wave_sync();
             const double acc = project_ub();
             uproj = acc;
@@ -478,7 +512,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             double Ld[S];
             point_lambda(yb, Ld);  // v^T phi_k
             double y[P];
-            closure_DU<KIND>(c, Lk, y);
+            closure_DU<KIND>(c, Lk, rk, y);
             wave_sync();
             if (lane < QP) {
 #pragma unroll
@@ -513,7 +547,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         }
         if constexpr (PREC == 4) reuse = c.max_iter != 1;
         f64x4 T_call[PREC == 4 ? TILES : 1];  // (kept across the call's steps)
-        double Lk0[S], g0 = 0.0;  // Lambda and gradient at lam while another point is tried
+        double Lk0[S], rk0 = 0.0, g0 = 0.0;  // Lambda, density and gradient at lam while another point is tried
         int status = -1, iters = 0, halvings = 0;
         int ngrad = 0;  // gradients evaluated here (the residual check counts the one it gives)
         // Ub and uproj hold U and <U phiW> at lam, the outputs' source
@@ -534,13 +568,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             where = GIVEN;
             // phase end: start
         }
-        for (bool first = true;; first = false) {
+        // (opaque, so that the loop is not cloned for its first pass)
+        int resolved = 0;
+        asm volatile("" : "+s"(where), "+s"(resolved));
+        for (;;) {
+            renew();
             double gt = 0.0, nt = 0.0;
             if (where != GIVEN) {
                 ++ngrad;
                 nt = gradient(at, gt);
             }
-            if (first) queue.resolve();
+            if (!resolved) {
+                queue.resolve();
+                resolved = 1;
+            }
             if (where == END) break;
             if (where == TRIAL) {
                 // line search (closure.cpp:159-184): halve the step until
@@ -572,6 +613,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     } else {
 #pragma unroll
                         for (int s = 0; s < S; ++s) Lk[s] = Lk0[s];
+                        rk = rk0;
                         refactor = true;
                     }
                 }
@@ -603,6 +645,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                         g = g0;
 #pragma unroll
                         for (int s = 0; s < S; ++s) Lk[s] = Lk0[s];
+                        rk = rk0;
                     }
                 } else {
                     if (where == START) {
@@ -615,6 +658,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                         g0 = g;
 #pragma unroll
                         for (int s = 0; s < S; ++s) Lk0[s] = Lk[s];
+                        rk0 = rk;
                         wave_sync();
                         where = ALT;
                         at = lamnew;
@@ -640,12 +684,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     }
 #pragma unroll
                     for (int s = 0; s < S; ++s) Lk0[s] = Lk[s];
+                    rk0 = rk;
                 } else {
                     bool spd;
                     if constexpr (PREC == 2) {
                         // phase: factor
                         spd = sweep_step<KIND, M, Q>(c, Lk[0], Lk[S > 1 ? 1 : 0], Lk[S > 2 ? 2 : 0],
-                                                     Lk[S > 3 ? 3 : 0], g, (lds_double*)smem, (lds_double*)wb,
+                                                     Lk[S > 3 ? 3 : 0], rk, g, (lds_double*)smem, (lds_double*)wb,
                                                      reuse ? a.pinv + cell * (long)W::KEPT : nullptr);
                         // phase end: factor
                         d = on ? yb[de] : 0.0;
@@ -658,14 +703,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
 #pragma unroll
                             for (int t = 0; t < KQ; ++t) kept[r][t] = 0.f;
                     } else {
-                        // the lane's coordinates anew: what derives from them
-                        // (masks and addresses of the step below) stays in
-                        // this branch instead of being kept for all cells, in
-                        // registers the rest needs
-                        int p16 = lane & 15, q4 = lane >> 4;
-                        asm volatile("" : "+v"(p16), "+v"(q4));
+                        renew();
                         // phase: hessian
-                        wave_system<KIND, M, Q, PREC == 0>(c, Lk, g, smem, bh, lane, p16, q4);
+                        wave_system<KIND, M, Q, PREC == 0>(c, Lk, rk, g, smem, bh, lane, p16, q4);
                         // phase end: hessian
                         if constexpr (PREC == 4) {
                             load_system(T_call);
@@ -698,6 +738,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     }
                 }
             }
+            if (kEarly && resolved < 2) {
+                next = queue.take();
+                prefetch(next);
+                resolved = 2;
+            }
             if (status < 0) {
                 step = 1.0;
                 halvings = 0;
@@ -715,8 +760,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             at = lam;
         }
         // phase: outputs
-        next = queue.take();
-        prefetch(next);
+        if constexpr (!kEarly) {
+            next = queue.take();
+            prefetch(next);
+        }
+        arrive();
         // the cell's slot for the next launch: a usable inverse (1) -- the
         // one just stored, or the kept one while it is fresh -- or none (0)
         if (PREC == 2 && reuse && lane == 0) a.pinv_ok[cell] = factored || !refactor ? 1 : 0;

@@ -299,9 +299,10 @@ template <int KIND>
 struct LinearStart {
     static constexpr int S = uqk::KindInfo<KIND>::S;
     double L[S][S];
-    __device__ bool factor(const uqk::ClosureParams& cp, const double* ds) {
+    // ds = DS(u_0), u00: the mean's first state (U's density at ds)
+    __device__ bool factor(const uqk::ClosureParams& cp, const double* ds, double u00) {
         double y[S * (S + 1) / 2];
-        uqk::closure_DU<KIND>(cp, ds, y);
+        uqk::closure_DU<KIND>(cp, ds, u00, y);
         for (int l = 0; l < S; ++l)
             for (int m = 0; m <= l; ++m) L[l][m] = y[l * (l + 1) / 2 + m];
         for (int j = 0; j < S; ++j) {
@@ -375,7 +376,7 @@ __device__ void stage_rows(RowScales<uqk::KindInfo<KIND>::S>& rs, long n, long r
             const long c = idx ? idx[r] : r;
             double D[S], ts[S], ds[S];
             LinearStart<KIND> lin;
-            ok = cell_scales<KIND>(u + (size_t)c * M * S, cp, D, ts, ds) && lin.factor(cp, ds);
+            ok = cell_scales<KIND>(u + (size_t)c * M * S, cp, D, ts, ds) && lin.factor(cp, ds, u[(size_t)c * M * S]);
             for (int s = 0; s < S; ++s) {
                 rs.D[t][s] = D[s];
                 rs.ts[t][s] = ts[s];

@@ -31,13 +31,6 @@ __device__ __forceinline__ double lane_get(double v, int lane) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// 1/h from v_rcp_f64 refined by two Newton steps
-__device__ __forceinline__ double recip_f64(double h) {
-    double r = __builtin_amdgcn_rcp(h);
-    r = fma(r, fma(-h, r, 1.0), r);
-    return fma(r, fma(-h, r, 1.0), r);
-}
-
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
     const long long x = __double_as_longlong(v);

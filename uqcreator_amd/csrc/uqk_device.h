@@ -40,8 +40,18 @@ template <> struct KindInfo<UQK_EULER2D> { static constexpr int S = 4; };
 template <> struct KindInfo<UQK_SHALLOW_WATER2D> { static constexpr int S = 3; };
 template <> struct KindInfo<UQK_SHALLOW_WATER2D_BARRIER> { static constexpr int S = 3; };
 
+// 1/h from v_rcp_f64 refined by two Newton steps
+__device__ __forceinline__ double recip_f64(double h) {
+    double r = __builtin_amdgcn_rcp(h);
+    r = fma(r, fma(-h, r, 1.0), r);
+    return fma(r, fma(-h, r, 1.0), r);
+}
+
 // ---------------------------------------------------------------------------
 // Entropy closures.  U(Lambda) = (grad s)^{-1}(Lambda) per quadrature point.
+// A division costs about 14 instructions, and the kernels that evaluate these
+// are bound by the instructions they issue: the quotients of one argument
+// share its reciprocal, and DU takes the density from U.
 // ---------------------------------------------------------------------------
 
 // Logistic map onto (u-, u+), evaluated on the branch whose exponential cannot
@@ -61,9 +71,14 @@ __device__ __forceinline__ double bb_du(double lam, double um, double up) {
     return ep * (up - um) / (1.0 + 2.0 * ep + exp(2.0 * lam));
 }
 
-// Euler 1D density from the duals (v0, v1, v2 < 0) (eulerclosure.cpp:7-12).
-__device__ __forceinline__ double e1_rho(double v0, double v1, double v2, double gm) {
-    return exp((2.0 * v0 * v2 - 2.0 * v2 * log(-v2) - 2.0 * v2 * gm - v1 * v1) / (2.0 * v2 * (gm - 1.0)));
+// Density of the Euler closures from the duals (v0, v, w < 0), q = |v|^2, r =
+// 1/w: exp((v0 - log(-w) - gamma - q / (2 w)) / (gamma - 1))
+// (eulerclosure.cpp:7-12; eulerclosure2d.cpp:7-17, whose (-v4)^(1 / (1 - gamma))
+// is taken into the exponential: equal up to rounding, no pow).
+__device__ __forceinline__ double euler_rho(double v0, double q, double w, double r, double gm) {
+    const double x = v0 - log(-w) - gm - 0.5 * q * r, g1 = gm - 1.0, k = recip_f64(g1);
+    const double e = x * k;
+    return exp(fma(fma(-e, g1, x), k, e));  // (the quotient corrected once: exp magnifies its error)
 }
 
 // Vector form of U (the one Closure::Gradient uses).
@@ -72,21 +87,19 @@ __device__ __forceinline__ void closure_U(const ClosureParams& c, const double* 
     if constexpr (KIND == UQK_BOUNDED_BARRIER) {
         out[0] = bb_u(L[0], c.u_minus, c.u_plus);
     } else if constexpr (KIND == UQK_EULER1D) {
-        double r = e1_rho(L[0], L[1], L[2], c.gamma);
-        out[0] = r;
-        out[1] = -(L[1] / L[2]) * r;
-        out[2] = ((L[1] * L[1] - 2.0 * L[2]) / (2.0 * L[2] * L[2])) * r;
+        // U = rho (1, -v/w, (v^2 - 2 w) / (2 w^2))
+        const double r = recip_f64(L[2]), q = L[1] * L[1];
+        const double rho = euler_rho(L[0], q, L[2], r, c.gamma);
+        out[0] = rho;
+        out[1] = -(L[1] * r) * rho;
+        out[2] = ((0.5 * q * r - 1.0) * r) * rho;
     } else if constexpr (KIND == UQK_EULER2D) {
-        // eulerclosure2d.cpp:7-17 (gamma stored negated there):
-        // exp(a / (1 + gm)) (-v4)^(1 / (1 + gm)) taken as one exponential,
-        // exp((a + log(-v4)) / (1 + gm)): equal up to rounding, no pow
-        const double gm = -c.gamma;
-        double v1 = L[0], v2 = L[1], v3 = L[2], v4 = L[3];
-        double e = exp(((v2 * v2 + v3 * v3 - 2.0 * v1 * v4 - 2.0 * v4 * gm) / (2.0 * v4) + log(-v4)) / (1.0 + gm));
-        out[0] = e;
-        out[1] = -(v2 * e / v4);
-        out[2] = -(v3 * e / v4);
-        out[3] = -(e * (-v2 * v2 - v3 * v3 + 2.0 * v4)) / (2.0 * v4 * v4);
+        const double r = recip_f64(L[3]), q = L[1] * L[1] + L[2] * L[2];
+        const double rho = euler_rho(L[0], q, L[3], r, c.gamma);
+        out[0] = rho;
+        out[1] = -(L[1] * r) * rho;
+        out[2] = -(L[2] * r) * rho;
+        out[3] = ((0.5 * q * r - 1.0) * r) * rho;
     } else if constexpr (KIND == UQK_SHALLOW_WATER2D) {
         // shallowwaterclosure2d.cpp:10-14
         double c0 = 2.0 * L[0] + L[1] * L[1] + L[2] * L[2];
@@ -123,49 +136,43 @@ __device__ __forceinline__ void closure_U_mat(const ClosureParams& c, const doub
 
 // Packed lower triangle of DU: entry p(l, m) = l*(l+1)/2 + m for m <= l holds
 // dU_l/dLambda_m.  The Hessian's upper triangle only reads these
-// (closure.cpp:265 with dposv 'U').
+// (closure.cpp:265 with dposv 'U').  The Euler closures take U's density, rho.
 template <int KIND>
-__device__ __forceinline__ void closure_DU(const ClosureParams& c, const double* L, double* y) {
+__device__ __forceinline__ void closure_DU(const ClosureParams& c, const double* L, double rho, double* y) {
     if constexpr (KIND == UQK_BOUNDED_BARRIER) {
         y[0] = bb_du(L[0], c.u_minus, c.u_plus);
-    } else if constexpr (KIND == UQK_EULER1D) {
-        // eulerclosure.cpp:37-56; DU(2,2) is the exact derivative unless du_exact == 0
-        const double gm = c.gamma;
-        double v0 = L[0], v1 = L[1], v2 = L[2];
-        double lg = log(-v2);
-        double E = exp((2.0 * v0 * v2 - 2.0 * v2 * lg - 2.0 * v2 * gm - v1 * v1) / (2.0 * v2 * (gm - 1.0)));
-        double d0 = E / (gm - 1.0);
-        double d1 = -(v1 / (v2 * (gm - 1.0))) * E;
-        double d2 = ((-2.0 * gm + 2.0 * v0 - 2.0 * lg - 2.0) / (2.0 * (gm - 1.0) * v2) -
-                     (-2.0 * gm * v2 + 2.0 * v0 * v2 - v1 * v1 - 2.0 * v2 * lg) / (2.0 * (gm - 1.0) * v2 * v2)) *
-                    E;
-        double a = (v1 * v1 - 2.0 * v2) / (2.0 * v2 * v2);
-        y[0] = d0;                                   // (0,0)
-        y[1] = -(v1 / v2) * d0;                      // (1,0)
-        y[2] = -(1.0 / v2) * E - (v1 / v2) * d1;     // (1,1)
-        y[3] = a * d0;                               // (2,0)
-        y[4] = a * d1 + (v1 / (v2 * v2)) * E;        // (2,1)
-        y[5] = c.du_exact ? (1.0 / (v2 * v2) - v1 * v1 / (v2 * v2 * v2)) * E + a * d2
-                          : (v1 * v1 * (v2 * v2 * v2) + 1.0 / (v2 * v2)) * E + a * d2;  // (2,2)
-    } else if constexpr (KIND == UQK_EULER2D) {
-        // eulerclosure2d.cpp:54-88
-        const double gm = -c.gamma;
-        double v1 = L[0], v2 = L[1], v3 = L[2], v4 = L[3];
-        double v22 = v2 * v2, v32 = v3 * v3, v42 = v4 * v4;
-        // the density factor as in closure_U (one exponential, no pow)
-        double e = exp(((v22 + v32 - 2.0 * v1 * v4 - 2.0 * v4 * gm) / (2.0 * v4) + log(-v4)) / (1.0 + gm)) / (1.0 + gm);
-        double vt = e * (v22 + v32 + 2.0 * v4 * gm) / (2.0 * v42 * v4);
-        y[0] = -e;                                                  // (0,0)
-        y[1] = v2 * e / v4;                                         // (1,0)
-        y[2] = -(e * (v22 + (gm + 1.0) * v4)) / v42;                // (1,1)
-        y[3] = v3 * e / v4;                                         // (2,0)
-        y[4] = -(v2 * v3 * e) / v42;                                // (2,1)
-        y[5] = -(e * (v32 + (gm + 1.0) * v4)) / v42;                // (2,2)
-        y[6] = -(0.5 * (v22 + v32 - 2.0 * v4) * e) / v42;           // (3,0)
-        y[7] = v2 * vt;                                             // (3,1)
-        y[8] = v3 * vt;                                             // (3,2)
-        y[9] = -(e * (v22 * v22 + v32 * v32 + 4.0 * v32 * v4 * gm - 4.0 * v42 * gm + 2.0 * v22 * (v32 + 2.0 * v4 * gm))) /
-               (4.0 * v42 * v42);                                   // (3,3)
+    } else if constexpr (KIND == UQK_EULER1D || KIND == UQK_EULER2D) {
+        // U = rho f, f = (1, -v/w, h) with h = (q/(2w) - 1)/w = E/rho (total
+        // energy over density); rho' = k rho f' with k = 1/(gamma - 1) and
+        // f' = (1, -v/w, h') = d(log rho)/dLambda / k, h' = (q/(2w) - 1)/w
+        // likewise; so DU = k rho f f^T + rho df/dLambda
+        // (eulerclosure.cpp:37-56, eulerclosure2d.cpp:54-88)
+        constexpr int D = KIND == UQK_EULER1D ? 1 : 2;
+        const double w = L[D + 1], r = recip_f64(w), k = recip_f64(c.gamma - 1.0);
+        double q = 0.0, m[D];  // m = -v/w, the velocity
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            m[i] = -(L[1 + i] * r);
+            q += L[1 + i] * L[1 + i];
+        }
+        const double h = (0.5 * q * r - 1.0) * r, kr = k * rho, rr = rho * r;
+        y[0] = kr;
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            const int l = 1 + i;
+            y[l * (l + 1) / 2] = kr * m[i];
+#pragma unroll
+            for (int j = 0; j <= i; ++j) y[l * (l + 1) / 2 + 1 + j] = kr * m[i] * m[j] - (i == j ? rr : 0.0);
+        }
+        constexpr int e = D + 1, at = e * (e + 1) / 2;
+        y[at] = kr * h;
+#pragma unroll
+        for (int j = 0; j < D; ++j) y[at + 1 + j] = kr * h * m[j] - rr * m[j];  // dh/dv = v/w^2 = -m/w
+        // dh/dw = 1/w^2 - q/w^3
+        if (KIND == UQK_EULER1D && !c.du_exact)
+            y[at + e] = (L[1] * L[1] * (w * w * w) + r * r) * rho + kr * h * h;  // as shipped
+        else
+            y[at + e] = kr * h * h + rr * r * (1.0 - q * r);
     } else if constexpr (KIND == UQK_SHALLOW_WATER2D) {
         // shallowwaterclosure2d.cpp:39-49
         const double g = c.g;
