@@ -119,8 +119,9 @@ int uqk_synchronize(uqk_ctx* ctx);
 
 /* Closure kernel selection: AUTO picks the compile-time specialised wave
  * kernel when one exists for (closure, M, Q) and the batch has one order,
- * else the workgroup-per-cell kernel for systems of 64..256 duals, else the
- * generic wave-per-cell kernel (any size, per-cell orders, FP64; below 64
+ * else the kernel for large systems (UQK_KERNEL_BLOCK; 64..128 duals: one
+ * wavefront per cell below 128, where LDS holds the tables, else a workgroup
+ * per cell), else the generic wave-per-cell kernel (any size, per-cell orders, FP64; below 64
  * duals in register tiles, where it outruns the workgroup kernel's mixed
  * precision, which UQK_KERNEL_BLOCK still selects). */
 enum { UQK_KERNEL_AUTO = 0, UQK_KERNEL_GENERIC = 1, UQK_KERNEL_WAVE = 2, UQK_KERNEL_BLOCK = 3 };

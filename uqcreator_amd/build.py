@@ -48,6 +48,11 @@ EXTRA_FLAGS = {
     "closure_tile_euler1d.hip": ["-mllvm", "-disable-machine-licm"],
     "closure_tile_euler2d.hip": ["-mllvm", "-disable-machine-licm"],
     "closure_tile_shallow.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wide_barrier.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wide_euler1d.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wide_euler2d.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wide_shallow.hip": ["-mllvm", "-disable-machine-licm"],
+    "closure_wide_shallow_barrier.hip": ["-mllvm", "-disable-machine-licm"],
 }
 
 
@@ -60,7 +65,8 @@ def sources():
 
 def _compile(src):
     obj = os.path.join(OUT, os.path.basename(src) + ".o")
-    cmd = [HIPCC] + HIP_FLAGS + EXTRA_FLAGS.get(os.path.basename(src), []) + ["-c", src, "-o", obj]
+    name = os.path.basename(src)
+    cmd = [HIPCC] + HIP_FLAGS + EXTRA_FLAGS.get(name, []) + ["-c", src, "-o", obj]
     if src.endswith(".cpp"):
         cmd = [HIPCC, "-x", "c++"] + [f for f in HIP_FLAGS if not f.startswith("--offload")] + ["-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -1,6 +1,6 @@
 // closure_block.hip -- batched FP64 Newton dual closure for large systems
-// (n = S * nTotal from 64 up to 128, e.g. 105 duals with 125 quadrature
-// points), one 256-thread workgroup per cell.
+// (n = S * nTotal up to 128) that closure_wide_kernel.h does not take: 128
+// duals, and tables that LDS does not hold.  One 256-thread workgroup per cell.
 //
 // Restates Closure::SolveClosure / SolveClosureSafe (closure.cpp:133-193,
 // :297-339), like closure_fp64.hip, with the work of a cell spread over four

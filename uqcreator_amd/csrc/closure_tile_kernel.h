@@ -13,9 +13,10 @@
 // What bounds it: the latency of a cell's chain, as in the wave kernel.  It
 // replaced a column-by-column Cholesky in LDS (closure_fp64.hip, which is
 // left with the systems of 64 duals and more): Euler 2D, 65,536 cells on
-// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 22.8 ms
+// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 22.1 ms
 // against 52.6 (26.2 with DU through the exponential and with the lane's
-// numbers kept over the cell: 4 to 48 registers spilled).
+// numbers kept over the cell: 4 to 48 registers spilled; 22.8 with reads of 8
+// bytes from LDS and tile rows skipped by branches).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -29,11 +30,11 @@ namespace uqk {
 // LDS doubles of the workgroup's tables and of a wavefront for table width M,
 // Q points and n duals at most
 struct TileLds {
-    int qp, ki, phiw, tables;            // row length, padded basis / 4, offset of phiw, size
+    int qp, ki, phiw, tables;            // row length (4 mod 8: tile_solve.h), padded basis / 4, offset of phiw, size
     int lam, lamnew, ub, du, yb, h, wave;  // offsets in a wavefront's part, and its size
     __host__ __device__ TileLds(int S, int M, int Q) {
         const int P = S * (S + 1) / 2, n = S * M;
-        qp = (Q + 3) / 4 * 4;
+        qp = (Q + 7) / 8 * 8 + 4;
         ki = (M + 3) / 4;
         phiw = 4 * ki * qp;
         tables = phiw + M * qp;
@@ -110,20 +111,33 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         // ||grad L|| at the duals X (LDS): U at the points in Ub, Lambda in DUb, gradient in gout
         auto gradient = [&](const double* X, double (&gout)[DT]) -> double {
             // phase: gradient
-            for (int p0 = 0; p0 < Q; p0 += 64) {
+            // W tiles of 16 points from p0 on
+            auto part = [&](int p0, auto width) {
+                constexpr int W = decltype(width)::value;
                 double t4[4] = {0.0, 0.0, 0.0, 0.0};
-                for (int ki = 0; 4 * ki < nt; ++ki) {
-                    const int i = 4 * ki + q4;
-                    const double xa = i < nt ? X[i * S + s4] : 0.0;
+                const double* ph[W];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        if (p0 + 16 * t < Q) {
-                            const int k = p0 + 16 * t + p16;
-                            t4[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(xa, phiT[i * QP + (k < Q ? k : Q - 1)], t4[t],
-                                                                       0, 0, 0);
-                        }
-                    }
+                for (int t = 0; t < W; ++t) {
+                    const int k = p0 + 16 * t + p16;
+                    ph[t] = phiT + q4 * QP + (k < Q ? k : Q - 1);
                 }
+                in_steps<1>(
+                    (nt + 3) / 4,
+                    [&](int ki) {
+                        Operands<W> o;
+                        const int i = 4 * ki + q4;
+                        o.a = i < nt ? X[i * S + s4] : 0.0;
+#pragma unroll
+                        for (int t = 0; t < W; ++t) o.b[t] = ph[t][4 * ki * QP];
+                        return o;
+                    },
+                    [&](const Operands<W>& o) {
+#pragma unroll
+                        for (int t = 0; t < W; ++t)
+                            t4[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(o.a, o.b[t], t4[t], 0, 0, 0);
+                    });
+#pragma unroll
+                for (int t = W; t < 4; ++t) t4[t] = t4[W - 1];  // (lanes past the tiles: finite)
                 group_transpose(t4);
                 double U[S];
                 closure_U<KIND>(c, t4, U);
@@ -135,6 +149,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                         DUb[s * QP + k] = t4[s];
                     }
                 }
+            };
+            for (int p0 = 0; p0 < Q; p0 += 64) {
+                if (Q - p0 > 32)
+                    part(p0, std::integral_constant<int, 4>());
+                else
+                    part(p0, std::integral_constant<int, 2>());
             }
             wave_sync();
             double sq = 0.0;
@@ -143,10 +163,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                 double acc = 0.0;
                 if (16 * t < (a.all_moments ? M : nt)) {
                     const int i = p16 + 16 * t < M ? p16 + 16 * t : M - 1;
-                    const double *ua = Ub + s4 * QP + q4, *wa = phiwT + i * QP + q4;
-#pragma unroll 4
-                    for (int k = 0; k < QP; k += 4)
-                        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(ua[k], wa[k], acc, 0, 0, 0);
+                    const double *ua = Ub + s4 * QP + 2 * q4, *wa = phiwT + i * QP + 2 * q4;
+                    in_steps<2>(
+                        QP / 8,
+                        [&](int k) {
+                            Operands<1, f64x2> o;
+                            o.a = two(ua + 8 * k);
+                            o.b[0] = two(wa + 8 * k);
+                            return o;
+                        },
+                        [&](const Operands<1, f64x2>& o) {
+#pragma unroll
+                            for (int h = 0; h < 2; ++h)
+                                acc = __builtin_amdgcn_mfma_f64_4x4x4f64(o.a[h], o.b[0][h], acc, 0, 0, 0);
+                        });
                 }
                 uproj[t] = acc;
                 const double g = on[t] ? acc - ue[t] : 0.0;
@@ -162,7 +192,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         // Hessian is not positive definite
         auto direction = [&](const double (&g)[DT], double (&d)[DT]) -> bool {
             // phase: hessian
-            for (int k = lane; k < QP; k += 64) {
+            for (int k = lane; k < QP - 4; k += 64) {
                 double L[S], y[P];
 #pragma unroll
                 for (int s = 0; s < S; ++s) L[s] = DUb[s * QP + k];
@@ -176,22 +206,37 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             for (int t = 0; 16 * t < npair; ++t) {
                 int j, i;
                 basis_pair(16 * t + p16 < npair ? 16 * t + p16 : 0, j, i);
-                const double *fj = phiT + j * QP + q4, *wi = phiwT + i * QP + q4;
+                const double *fj = phiT + j * QP + 2 * q4, *wi = phiwT + i * QP + 2 * q4;
                 const double* du[PG];
                 double acc[PG];
 #pragma unroll
                 for (int pg = 0; pg < PG; ++pg) {
                     const int p = 4 * pg + (p16 & 3);
-                    du[pg] = DUb + (p < P ? p : P - 1) * QP + q4;
+                    du[pg] = DUb + (p < P ? p : P - 1) * QP + 2 * q4;
                     acc[pg] = 0.0;
                 }
-#pragma unroll 4
-                for (int k = 0; k < QP; k += 4) {
-                    const double av = fj[k] * wi[k];
+                struct Step {
+                    f64x2 f, w, d[PG];
+                };
+                in_steps<2>(
+                    QP / 8,
+                    [&](int k) {
+                        Step o;
+                        o.f = two(fj + 8 * k);
+                        o.w = two(wi + 8 * k);
 #pragma unroll
-                    for (int pg = 0; pg < PG; ++pg)
-                        acc[pg] = __builtin_amdgcn_mfma_f64_4x4x4f64(av, du[pg][k], acc[pg], 0, 0, 0);
-                }
+                        for (int pg = 0; pg < PG; ++pg) o.d[pg] = two(du[pg] + 8 * k);
+                        return o;
+                    },
+                    [&](const Step& o) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const double av = o.f[h] * o.w[h];
+#pragma unroll
+                            for (int pg = 0; pg < PG; ++pg)
+                                acc[pg] = __builtin_amdgcn_mfma_f64_4x4x4f64(av, o.d[pg][h], acc[pg], 0, 0, 0);
+                        }
+                    });
                 // this lane's products: pair 16 t + 4 (p16 / 4) + q4, state pairs 4 pg + p16 % 4
                 const int e = 16 * t + 4 * (p16 >> 2) + q4;
                 if (e < npair) {
@@ -229,11 +274,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                     }
             // phase end: load
             // phase: factor
-            const bool spd = tile_ldl<NT>(T, n, p16, q4);
+            bool spd = false;
+            static_for<NT>([&](auto last) {  // (as many tile rows as the order takes)
+                constexpr int R = decltype(last)::value + 1;
+                if (n >> 4 == R - 1) {
+                    spd = tile_ldl<R>(T, n, p16, q4);
+                    yb[lane] = tile_back<R>(T, n, p16, q4);
+                }
+            });
             // phase end: factor
-            // phase: backsub
-            yb[lane] = tile_back<NT>(T, n, p16, q4);
-            // phase end: backsub
             wave_sync();
 #pragma unroll
             for (int t = 0; t < DT; ++t) d[t] = on[t] ? yb[q4 * nt + p16 + 16 * t] : 0.0;

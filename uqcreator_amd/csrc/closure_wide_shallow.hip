@@ -1,0 +1,11 @@
+// closure_wide_shallow.hip -- the shallow-water 2D instantiations of the one-wavefront
+// Newton closure for 64 duals and more (closure_wide_kernel.h).
+#include "closure_wide_kernel.h"
+
+namespace uqk {
+
+hipError_t newton_wide_shallow(const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st, const LaunchShape& shape) {
+    return wide_kind<UQK_SHALLOW_WATER2D>(a, max_lds, num_cu, st, shape);
+}
+
+}  // namespace uqk

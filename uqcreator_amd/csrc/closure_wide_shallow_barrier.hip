@@ -1,0 +1,11 @@
+// closure_wide_shallow_barrier.hip -- the shallow-water 2D barrier instantiations of the one-wavefront
+// Newton closure for 64 duals and more (closure_wide_kernel.h).
+#include "closure_wide_kernel.h"
+
+namespace uqk {
+
+hipError_t newton_wide_shallow_barrier(const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st, const LaunchShape& shape) {
+    return wide_kind<UQK_SHALLOW_WATER2D_BARRIER>(a, max_lds, num_cu, st, shape);
+}
+
+}  // namespace uqk

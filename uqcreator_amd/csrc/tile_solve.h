@@ -18,6 +18,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "uqk_device.h"
 
 namespace uqk {
@@ -84,12 +86,85 @@ __device__ __forceinline__ void group_transpose(double (&d)[4]) {
     swap_rows(d[2], d[3]);
 }
 
-// basis pair (j <= i) of number e = i (i + 1) / 2 + j, from its root (e < 2^12)
+// basis pair (j <= i) of number e = i (i + 1) / 2 + j, from its root (e < 2^14)
 __device__ __forceinline__ void basis_pair(int e, int& j, int& i) {
     i = (int)((__builtin_amdgcn_sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
-    i -= i * (i + 1) / 2 > e ? 1 : 0;
-    i += (i + 1) * (i + 2) / 2 <= e ? 1 : 0;
-    j = e - i * (i + 1) / 2;
+    const int below = (int)__umul24(i, i + 1) >> 1;  // (24-bit products: the 32-bit one takes four times as long)
+    const int low = below > e ? 1 : 0, high = below + i + 1 <= e ? 1 : 0;
+    j = e - (below - (low ? i : 0) + (high ? i + 1 : 0));
+    i += high - low;
+}
+
+// Stands where paths join that matrix instructions precede on some of them.
+// What reads their results has to come 9 (4 x 4 x 4) or 18 (16 x 16 x 4) issue
+// slots later at most; the compiler counts these slots along one of the paths
+// to a join only, and where a shorter one exists the read can come too early
+// (seen as the old low half of a result).
+template <int SLOTS>
+__device__ __forceinline__ void settle() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop %0" : : "n"(SLOTS < 16 ? SLOTS - 1 : 15));
+    if constexpr (SLOTS > 16) asm volatile("s_nop %0" : : "n"(SLOTS - 17));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// mma(load(0)), mma(load(1)), .. for `steps` steps, U of them in flight: the
+// next U are loaded while these are multiplied (what an LDS round trip costs
+// a wavefront with no other beside it, or few).  Steps are loaded up to U past
+// the last, so the operands' rows need that much readable LDS behind them.
+// (Written out, because loops over matrix instructions are not unrolled with a
+// remainder.)
+template <int U, class Load, class Mma>
+__device__ __forceinline__ void in_steps(int steps, Load load, Mma mma) {
+    decltype(load(0)) x[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = load(u);
+    int s = 0;
+    for (; s + 2 * U < steps; s += 2 * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) y[u] = load(s + U + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mma(x[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = load(s + 2 * U + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mma(y[u]);
+    }
+    if (s + U < steps) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) y[u] = load(s + U + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mma(x[u]);
+        s += U;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u < steps) mma(y[u]);
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u < steps) mma(x[u]);
+    }
+    settle<9>();
+}
+// Operands of a matrix step, and of two steps: eight points, of which lane
+// group q holds 2 q and 2 q + 1 (one ds_read_b128 each; 16 rows of 4 mod 8
+// doubles at these four columns fall on all 64 banks once: 8.8 cycles per
+// double and lane with four wavefronts, where ds_read_b64 of rows 4 mod 8 at
+// columns q takes 64 and of odd rows 16).
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+template <int N, class T = double>
+struct Operands {
+    T a, b[N];
+};
+__device__ __forceinline__ f64x2 two(const double* x) { return *reinterpret_cast<const f64x2*>(x); }
+
+// f(integral_constant<0>) .. f(integral_constant<N - 1>)
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        static_for<N, I + 1>(f);
+    }
 }
 
 // tile (tc, tr), tc <= tr, of the lower triangle
@@ -141,9 +216,12 @@ __device__ __forceinline__ bool pivot_inverse(double pv, int j0, int have, int p
 
 // In place on the lower tiles of [H; g^T] (n pivots; row n holds the right
 // hand side): column block b becomes W = V^T, the block-unit upper factor of
-// H = V^T B V (B the 4 x 4 pivot blocks).  NT tiles of 16 hold n + 1 rows.
-template <int NT>
-__device__ __forceinline__ bool tile_ldl(f64x4 (&T)[NT * (NT + 1) / 2], int n, int p, int q) {
+// H = V^T B V (B the 4 x 4 pivot blocks).  The first NT tile rows hold n + 1
+// rows; there is no branch between the matrix instructions of a step, whose
+// tiles past the last pivot are updated for nothing where n is not a constant
+// (settle).
+template <int NT, int TILES>
+__device__ __forceinline__ bool tile_ldl(f64x4 (&T)[TILES], int n, int p, int q) {
     bool ok = true;
 #pragma unroll
     for (int b = 0; b < 4 * NT; ++b) {
@@ -154,34 +232,32 @@ __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[NT * (NT + 1) / 2], int n, i
         double P[NT], W[NT];
 #pragma unroll
         for (int r = jb; r < NT; ++r) {
-            if (16 * r > n) break;  // (tiles past row n hold nothing)
             P[r] = T[tile_lower(jb, r)][e];
             if (r == jb && !(p >= j0 + (have < 4 ? have : 4))) P[r] = 0.0;  // finished rows
             if (have < 4 && q >= have) P[r] = 0.0;       // columns that are no pivots
             W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(bv, P[r], 0.0, 0, 0, 0);
             T[tile_lower(jb, r)][e] = W[r];
         }
-        if (4 * b + 4 < n) {
+        if (!__builtin_constant_p(n) || 4 * b + 4 < n) {
 #pragma unroll
-            for (int r = jb; r < NT; ++r) {
-                if (16 * r > n) break;
+            for (int r = jb; r < NT; ++r)
 #pragma unroll
                 for (int c = jb; c <= r; ++c)
-                    if (16 * c < n)
+                    if (!__builtin_constant_p(n) || 16 * c < n)
                         T[tile_lower(c, r)] =
                             __builtin_amdgcn_mfma_f64_16x16x4f64(P[c], -W[r], T[tile_lower(c, r)], 0, 0, 0);
-            }
         }
     }
+    if (!__builtin_constant_p(n)) settle<18>();
     return ok;
 }
 
 // The solution from the factor that tile_ldl left: x_{4b+k} = W(n, k) -
 // sum_{r > 4b+3} W(r, k) x_r, four unknowns per step, the sum over the rows
-// of a lane group by DPP.  Lane l gets x_l (zero past n).
-template <int NT>
-__device__ __forceinline__ double tile_back(const f64x4 (&T)[NT * (NT + 1) / 2], int n, int p, int q) {
-    double X[NT];
+// of a lane group by DPP.  X[r] of lane 16 q + p is x_{16 r + p} (-1 at n,
+// zero past it).
+template <int NT, int TILES>
+__device__ __forceinline__ void tile_back_rows(const f64x4 (&T)[TILES], int n, int p, int q, double (&X)[NT]) {
 #pragma unroll
     for (int r = 0; r < NT; ++r) X[r] = 16 * r + p == n ? -1.0 : 0.0;
     const bool p1 = p & 1, p2 = p & 2;
@@ -192,12 +268,19 @@ __device__ __forceinline__ double tile_back(const f64x4 (&T)[NT * (NT + 1) / 2],
         double s = 0.0;
 #pragma unroll
         for (int r = jb; r < NT; ++r)
-            if (16 * r <= n) s = fma(-T[tile_lower(jb, r)][e], X[r], s);
+            s = fma(-T[tile_lower(jb, r)][e], X[r], s);
         s = row_sum(s);
         const double x0 = lane_get(s, 0), x1 = lane_get(s, 16), x2 = lane_get(s, 32), x3 = lane_get(s, 48);
         const double v = p2 ? (p1 ? x3 : x2) : (p1 ? x1 : x0);
         if ((p >> 2) == e && (p & 3) < have) X[jb] = v;
     }
+}
+
+// The same for n < 64: lane l gets x_l (zero past n).
+template <int NT, int TILES>
+__device__ __forceinline__ double tile_back(const f64x4 (&T)[TILES], int n, int p, int q) {
+    double X[NT];
+    tile_back_rows<NT>(T, n, p, q, X);
     double d = X[0];
 #pragma unroll
     for (int r = 1; r < NT; ++r) d = q == r ? X[r] : d;
@@ -251,8 +334,8 @@ __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, in
 // of the matrix steps at NT = 3): the panel's rows above the pivots are the
 // transposed pivot rows, turned over through LDS (scr, 64 (NT - 1) doubles).
 // -H^-1 in the lower triangle, and H^-1 g in row n where row n held g.
-template <int NT, class D>
-__device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[NT * (NT + 1) / 2], int n, int p, int q, D* scr) {
+template <int NT, int TILES, class D>
+__device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p, int q, D* scr) {
     bool ok = true;
 #pragma unroll
     for (int b = 0; b < 4 * NT; ++b) {
@@ -298,6 +381,7 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[NT * (NT + 1) / 2], 
             }
         }
     }
+    if (!__builtin_constant_p(n)) settle<18>();
     return ok;
 }
 

@@ -101,6 +101,15 @@ int check_mesh(uqk_ctx* ctx, const uqk_mesh* m) {
     return 0;
 }
 
+// Whether a kernel for large systems takes the shape (UQK_KERNEL_BLOCK): one
+// wavefront per cell below 128 duals, else a workgroup per cell.
+bool wide_fits(const uqk_ctx* ctx) {
+    return uqk::newton_wide_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+}
+bool large_fits(const uqk_ctx* ctx) {
+    return wide_fits(ctx) || uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+}
+
 // Kept inverse factors of the mixed wave kernel across time steps: grows
 // the per-cell slots (flags cleared) to n cells.  Allocates only outside
 // graph capture.
@@ -114,7 +123,7 @@ int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
         uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, 1, &wm, &wo))
         return uqk::newton_wave_reuse_fits(ctx->kind, ctx->M, ctx->Q, (int)ctx->max_lds) ? 1 : 0;
     if (ctx->kernel == UQK_KERNEL_WAVE) return 0;
-    const bool block_ok = uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+    const bool block_ok = large_fits(ctx);
     if (block_ok && (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64)))
         return 2;
     return 0;
@@ -124,8 +133,9 @@ int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
 // capture only; a change of mode starts with no kept factor.
 int ensure_factor_buffers(uqk_ctx* ctx, long n_cells, int mode) {
     const long n = (long)ctx->S * ctx->M;
-    // mode 1: the FP32 inverse; mode 2: the FP32 factor (packed U)
-    const long nn = mode == 1 ? uqk::newton_wave_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
+    // mode 1: the FP32 inverse; mode 2: the same in tiles, or the FP32 factor (packed U)
+    const long nn = mode == 1 ? uqk::newton_wave_kept_floats(ctx->S, ctx->M)
+                    : wide_fits(ctx) ? uqk::newton_wide_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
     if (ctx->pinv_cell_cap >= n_cells && ctx->factor_mode == mode) return 0;
     if (ctx->capturing) return fail(ctx, -1, "kept factors: buffers must exist before graph capture");
     hipFree(ctx->pinv_cell);
@@ -307,7 +317,7 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
         a.grad_at_lam = nullptr;
         a.dt_cell = nullptr;
     }
-    const bool block_ok = uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+    const bool block_ok = large_fits(ctx);
     if (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64 && block_ok)) {
         if (!block_ok) return fail(ctx, -3, "closure too large for the workgroup kernel");
         if (a.pinv_mode == 1 && ctx->factor_mode != 2) a.pinv_mode = 0;  // (the slots hold inverses)
@@ -341,7 +351,8 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
             a.grad_at_lam = ctx->check_grad;
             a.dt_cell = ca.dt_cell;
         }
-        UQK_HIP(ctx, uqk::newton_block_launch(ctx->kind, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream, ctx->shape));
+        UQK_HIP(ctx, (wide_fits(ctx) ? uqk::newton_wide_launch : uqk::newton_block_launch)(
+                         ctx->kind, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream, ctx->shape));
         if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev1, ctx->stream));
         ctx->step_recon = a.dt_cell != nullptr;
         ctx->last_kernel = UQK_KERNEL_BLOCK;
@@ -1119,7 +1130,7 @@ int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda,
                       uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, 4, &wmax,
                                               &occ);
     const bool block = !wave && (ctx->kernel == UQK_KERNEL_AUTO || ctx->kernel == UQK_KERNEL_BLOCK) &&
-                       uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+                       large_fits(ctx);
     if (!wave && !block) return fail(ctx, -3, "uqk_autotune: no specialised closure kernel for this shape");
     if (block) wmax = 4;
     const size_t bytes = sizeof(double) * (size_t)n * ctx->S * ctx->M;
@@ -1136,7 +1147,7 @@ int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda,
         if (wave)
             uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, waves, &wm, &oc);
         else
-            oc = uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
+            oc = wide_fits(ctx) ? 1 : uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
         for (int per_cu = 1; per_cu <= oc && rc == 0; ++per_cu) {
             ctx->shape.waves = waves;
             ctx->shape.blocks_per_cu = per_cu;
