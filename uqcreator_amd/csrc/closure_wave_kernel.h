@@ -32,7 +32,7 @@
 // v_readlane, with an exponential and a logarithm: 14.6 K), gradient 3.6 K
 // (4.3 K); 65,536 cells, 40 time steps: 21.4 ms against 39.0 (FP64), 16.5
 // against 30.7 (mixed).  At n = 45, 49 points, one closure of 100,003 cells:
-// 30.4 ms against 47.4 (FP64), 10.2 against 19.5 (mixed: a step on the kept
+// 29.9 ms against 47.4 (FP64), 10.0 against 19.5 (mixed: a step on the kept
 // inverse is a matrix-vector product from registers, 1.3 K cycles, in place
 // of two triangular solves from LDS, 13.9 K).
 // The next cell's moments, duals, density and kept inverse are asked for
@@ -55,7 +55,13 @@ struct WaveShape {
     static constexpr int N = S * M;              // duals per cell
     static constexpr int P = S * (S + 1) / 2;    // distinct DU entries
     static constexpr int KS = (Q + 3) / 4;       // four points per matrix step
-    static constexpr int QP = 4 * KS;            // row length of the tables and of U
+    // row length of the tables and of U: 4 mod 8, as tile_solve.h's f64x2 reads like it
+    static constexpr int QP = 4 * KS + (KS % 2 ? 0 : 4);
+    // the point that lane group q has in step ks: two steps share eight points,
+    // of which a group takes two neighbours (one read); a last odd step has four
+    __host__ __device__ static constexpr int point(int ks, int q) {
+        return (ks | 1) < KS ? 8 * (ks / 2) + 2 * q + (ks & 1) : 4 * ks + q;
+    }
     static constexpr int NPAIR = M * (M + 1) / 2;
     static constexpr int PT = (NPAIR + 15) / 16; // tiles of 16 basis pairs
     static constexpr int PG = (P + 3) / 4;       // groups of four state pairs
@@ -97,6 +103,21 @@ template <int PREC> constexpr bool wave_reuses = PREC == 2 || PREC == 4;
 // the inverse from the registers, the lower triangle otherwise
 template <int PREC, int NT> constexpr int wave_tiles = PREC == 4 ? NT * NT : NT * (NT + 1) / 2;
 
+__device__ __forceinline__ f64x2 two(const __attribute__((address_space(3))) double* x) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) f64x2*>(x);
+}
+// a row of LDS (of points) as the operands of all KS steps: WaveShape::point
+template <int KS, class D>
+__device__ __forceinline__ void row_steps(const D* row, int q4, double (&v)[KS]) {
+#pragma unroll
+    for (int ks = 0; ks + 1 < KS; ks += 2) {
+        const f64x2 x = two(row + 4 * ks + 2 * q4);
+        v[ks] = x[0];
+        v[ks + 1] = x[1];
+    }
+    if constexpr (KS % 2) v[KS - 1] = row[4 * (KS - 1) + q4];
+}
+
 // The system of a Newton step at the iterate whose Lambda and density lie at
 // this lane's point in Lk and rk, into bh: the pair products (pairs x points)(points x state
 // pairs) on FP64 matrix steps; with RHS also the gradient g of this lane's
@@ -117,9 +138,7 @@ __device__ __forceinline__ void wave_system(const ClosureParams& c, const double
 #pragma unroll
     for (int pg = 0; pg < W::PG; ++pg) {
         const int p = 4 * pg + (p16 & 3);
-        const D* src = bh + (p < P ? p : P - 1) * QP + q4;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) du[pg][ks] = src[4 * ks];
+        row_steps<KS>(bh + (p < P ? p : P - 1) * QP, q4, du[pg]);
     }
     wave_sync();
     // products of tile t: lane holds (pair 16 t + 4 (p16 / 4) + q4, state pair 4 pg + p16 % 4)
@@ -129,12 +148,12 @@ __device__ __forceinline__ void wave_system(const ClosureParams& c, const double
         double acc[W::PG];
 #pragma unroll
         for (int pg = 0; pg < W::PG; ++pg) acc[pg] = 0.0;
-        const D *fj = nullptr, *wi = nullptr;
+        double fj[KS], wi[KS];
         if constexpr (!W::PAIR_TABLE) {
             int j, i;
             basis_pair(16 * t + p16 < W::NPAIR ? 16 * t + p16 : 0, j, i);
-            fj = smem + j * QP + q4;
-            wi = smem + W::PHIW + i * QP + q4;
+            row_steps<KS>(smem + j * QP, q4, fj);
+            row_steps<KS>(smem + W::PHIW + i * QP, q4, wi);
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -142,7 +161,7 @@ __device__ __forceinline__ void wave_system(const ClosureParams& c, const double
             if constexpr (W::PAIR_TABLE)
                 av = smem[W::PAIRS + (t * KS + ks) * 64 + lane];
             else
-                av = fj[4 * ks] * wi[4 * ks];
+                av = fj[ks] * wi[ks];
 #pragma unroll
             for (int pg = 0; pg < W::PG; ++pg)
                 acc[pg] = __builtin_amdgcn_mfma_f64_4x4x4f64(av, du[pg][ks], acc[pg], 0, 0, 0);
@@ -233,9 +252,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     }
     double* pairs = smem + W::PAIRS;
     if constexpr (W::PAIR_TABLE) {
-        // operand (pair 16 t + l % 16, point 4 ks + l / 16) at (t KS + ks) 64 + l
+        // operand (pair 16 t + l % 16, point(ks, l / 16)) at (t KS + ks) 64 + l
         for (int t = threadIdx.x; t < W::PT * KS * 64; t += blockDim.x) {
-            const int ln = t & 63, ks = (t >> 6) % KS, e = 16 * ((t >> 6) / KS) + (ln & 15), k = 4 * ks + (ln >> 4);
+            const int ln = t & 63, ks = (t >> 6) % KS, e = 16 * ((t >> 6) / KS) + (ln & 15), k = W::point(ks, ln >> 4);
             int j, i;
             basis_pair(e < W::NPAIR ? e : 0, j, i);
             pairs[t] = k < Q ? a.phi[k * M + j] * a.phiw[k * M + i] : 0.0;
@@ -375,6 +394,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         // sum_k Ub(s, k) phiW(k, i) for this lane's dual (s, i): the product
         // (S x Q)(Q x M) in steps of four points; its lane layout is the duals'
         auto project_ub = [&]() -> double {
+            // (points in order: the residual check's sum to the last bit)
             const double* ua = Ub + ((p16 & 3) < S ? (p16 & 3) : S - 1) * QP + q4;
             const double* wa = phiwT + (p16 < M ? p16 : M - 1) * QP + q4;
             double acc = 0.0;
