@@ -7,15 +7,17 @@
 //   mean / variance of the solution      (momentsolver.cpp:302-328)
 #include <hip/hip_runtime.h>
 
+#include "tile_solve.h"
 #include "uqk_device.h"
 #include "uqk_internal.h"
 
 namespace uqk {
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSweepThreads = 256;
 constexpr int kPartialBlocks = 8192;  // grid of the grid-stride sweeps and size of the partials
+// grid of the advance: its workgroups load the projection's table once each
+constexpr int kAdvanceBlocks = 2048;
 
 int sweep_partial_blocks() { return kPartialBlocks; }
 
@@ -172,12 +174,27 @@ __host__ __device__ inline int advance_wave_doubles(int S, int Q) {
 // the edges share one projection); the shallow-water bed friction enters as
 // -area * S(u) at the point before the projection; the projection
 // rhs(s, i) = sum_k G(s, k) phiW(k, i) of all the wave's cells is one FP64
-// MFMA tile row block (rows: cell slot x state), and the lanes holding the
-// tile's elements update the moments.  The residual |u_new(0,0) - u_old(0,0)|
-// * area is accumulated per block.
-// (four waves per SIMD: the kernel waits on memory and square roots, and the
-// register budget of four waves holds it without spilling)
-template <int KIND>
+// matrix product (rows: cell slot x state), and the lanes holding its elements
+// update the moments.  The residual |u_new(0,0) - u_old(0,0)| * area is
+// accumulated per block.
+// What bounds it: the wait for memory at four wavefronts per SIMD (60% of
+// their time), and the fluxes' instructions (half of the SIMDs' time).  uQ is
+// read from HBM once (62 MB of 65,536 cells at 25 points and four states).
+// Reciprocals and roots as refined estimates and the cell's own state formed
+// once for its edges, edge data in one load per vector or (ONE) in scalar
+// registers, 2,048 workgroups instead of 8,192 that each load the projection's
+// table: 94 -> 79 us there, 777 -> 466 us for 65,536 cells at 125 points and
+// three states, whose projection took 16-row products for 3 rows.
+// a read-only value at a uniform address, through the scalar cache
+template <class T> __device__ __forceinline__ T uniform_load(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)p;
+}
+
+// ONE: a wavefront has one cell (Q > 32).  The cell, its edges and their
+// normals are then uniform, in scalar registers.
+// (four waves per SIMD: the kernel waits on memory, and the register budget
+// of four waves holds it)
+template <int KIND, bool ONE>
 __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(4))) advance_kernel(SweepArgs a) {
     constexpr int S = KindInfo<KIND>::S;
     UQK_SKIP_IF_INACTIVE(a)
@@ -185,7 +202,7 @@ __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int M = a.M, Q = a.Q, SM = S * M, E = a.nedge, D = a.dim;
-    const int CPW = advance_cells_per_wave(S, Q);
+    const int CPW = ONE ? 1 : advance_cells_per_wave(S, Q);
     double* Gs = smem + wave * advance_wave_doubles(S, Q);
     const bool wlds = a.table_lds != 0;
     double* wt = smem + (blockDim.x >> 6) * advance_wave_doubles(S, Q);
@@ -197,78 +214,113 @@ __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
     const bool fric = (S == 3 && a.p.problem == UQK_SHALLOW_WATER2D_PROBLEM && a.p.friction > 0.0);
     // this lane's cell slot and first point
-    const int slot = CPW > 1 ? lane / Q : 0;
-    const int k0 = CPW > 1 ? lane - slot * Q : lane;
+    const int slot = ONE ? 0 : lane / Q;
+    const int k0 = ONE ? lane : lane - slot * Q;
     const bool lane_on = slot < CPW && k0 < Q;
     double res = 0.0;
     const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
     for (long cell0 = ((long)blockIdx.x * (blockDim.x >> 6) + wave) * CPW; cell0 < a.ncell; cell0 += nwaves * CPW) {
-        const long cell = cell0 + slot;
+        const long cell = ONE ? (long)__builtin_amdgcn_readfirstlane((int)cell0) : cell0 + slot;
         const bool on = lane_on && cell < a.ncell;
-        const int bc = on ? a.bc[cell] : UQK_BC_DIRICHLET;
+        int bc = UQK_BC_DIRICHLET;
+        if constexpr (ONE)
+            bc = uniform_load(a.bc + cell);
+        else if (on)
+            bc = a.bc[cell];
         if (on && bc != UQK_BC_DIRICHLET) {
             const double* uqj = a.uq + cell * S * Q;
             const bool wall = (bc == UQK_BC_NOSLIP || bc == UQK_BC_SWWALL);
-            const double area = a.area[cell];
+            const double area = ONE ? uniform_load(a.area + cell) : a.area[cell];
+            int nb[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                nb[e] = 0;
+                if (e < E) nb[e] = ONE ? uniform_load(a.nbr + cell * E + e) : a.nbr[cell * E + e];
+            }
             for (int k = k0; k < Q; k += 64) {
-                double uj[S], gj[S], Gsum[S];
+                double uj[S], Gsum[S], v[S], vn[S];
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
                     uj[s] = uqj[k * S + s];
                     Gsum[s] = 0.0;
                 }
-                if constexpr (S >= 3) {
-                    if (wall) {
-                        // ghost state: velocity reflected to the tangential
-                        // part (expliciteuler.cpp:25-58)
-                        const double bx = a.bnormal[cell * D + 0], by = a.bnormal[cell * D + 1];
-                        const double rho = uj[0], vx = uj[1] / rho, vy = uj[2] / rho;
-                        const double vn = bx * vx + by * vy;
-                        const double tx = vx - vn * bx, ty = vy - vn * by;
+                // an edge's other state, with ONE sent for before the edge before
+                // it is used (without, the registers are worth more: 98 us
+                // against 109 with it, 65,536 cells of four states at 25 points;
+                // the reference reads the never-written uQ[nCells], zero)
+                auto other = [&](int j, double (&x)[S]) {
+                    const double* src = j != a.ncell ? a.uq + (long)j * Q * S : uqj;
 #pragma unroll
-                        for (int s = 0; s < S; ++s) gj[s] = uj[s];
-                        if constexpr (S == 4) {
-                            if (bc == UQK_BC_NOSLIP) gj[3] += rho * 0.5 * ((tx * tx + ty * ty) - (vx * vx + vy * vy));
-                        }
-                        gj[1] = rho * tx;
-                        gj[2] = rho * ty;
-                    }
-                }
+                    for (int s = 0; s < S; ++s) x[s] = src[k * S + s];
+                };
+                if constexpr (ONE) other(nb[0], v);
+                const PointState pj = point_state<S>(a.p, uj);
+#pragma unroll 1
                 for (int e = 0; e < E; ++e) {
-                    const int nb = a.nbr[cell * E + e];
+                    const int nbe = e < 2 ? (e == 0 ? nb[0] : nb[1]) : (e == 2 ? nb[2] : nb[3]);
+                    if constexpr (!ONE) other(nbe, vn);
+                    if (ONE && e + 1 < E) other(e == 0 ? nb[1] : e == 1 ? nb[2] : nb[3], vn);
                     const double* nu = a.unit_normal + (cell * E + e) * D;
                     const double* nv = a.normal + (cell * E + e) * D;
-                    const double nux = nu[0], nuy = D > 1 ? nu[1] : 0.0, nx = nv[0], ny = D > 1 ? nv[1] : 0.0;
-                    double l[S], r[S], G[S];
-                    if (wall && nb == a.ncell) {
-                        // the flux is G(ghost, ghost)
-#pragma unroll
-                        for (int s = 0; s < S; ++s) l[s] = r[s] = S >= 3 ? gj[s] : uj[s];
-                    } else if (nb == a.ncell) {
-                        // the reference reads the never-written uQ[nCells] (zero)
-#pragma unroll
-                        for (int s = 0; s < S; ++s) {
-                            l[s] = uj[s];
-                            r[s] = 0.0;
+                    double nux, nuy = 0.0, nx, ny = 0.0;
+                    if constexpr (ONE) {
+                        nux = uniform_load(nu);
+                        nx = uniform_load(nv);
+                        if (D > 1) {
+                            nuy = uniform_load(nu + 1);
+                            ny = uniform_load(nv + 1);
                         }
+                    } else if (D > 1) {
+                        const f64x2 u2 = two(nu), v2 = two(nv);
+                        nux = u2[0];
+                        nuy = u2[1];
+                        nx = v2[0];
+                        ny = v2[1];
                     } else {
-#pragma unroll
-                        for (int s = 0; s < S; ++s) {
-                            l[s] = uj[s];
-                            r[s] = a.uq[((long)nb * Q + k) * S + s];
-                        }
+                        nux = nu[0];
+                        nx = nv[0];
                     }
-                    point_flux<S>(a.p, l, r, nux, nuy, nx, ny, G);
+                    const bool edge = nbe == a.ncell;
+                    double l[S], r[S], G[S];
+                    PointState pl = pj;
 #pragma unroll
-                    for (int s = 0; s < S; ++s) Gsum[s] += G[s];
+                    for (int s = 0; s < S; ++s) {
+                        l[s] = uj[s];
+                        r[s] = edge ? 0.0 : ONE ? v[s] : vn[s];
+                    }
+                    if (edge && wall) {
+                        // ghost state: velocity reflected to the tangential
+                        // part (expliciteuler.cpp:25-58); the flux is G(ghost, ghost)
+                        if constexpr (S >= 3) {
+                            const double bx = a.bnormal[cell * D + 0], by = a.bnormal[cell * D + 1];
+                            const double rho = uj[0], vx = uj[1] / rho, vy = uj[2] / rho;
+                            const double vn = bx * vx + by * vy;
+                            const double tx = vx - vn * bx, ty = vy - vn * by;
+                            if constexpr (S == 4) {
+                                if (bc == UQK_BC_NOSLIP) l[3] += rho * 0.5 * ((tx * tx + ty * ty) - (vx * vx + vy * vy));
+                            }
+                            l[1] = rho * tx;
+                            l[2] = rho * ty;
+                        }
+#pragma unroll
+                        for (int s = 0; s < S; ++s) r[s] = l[s];
+                        pl = point_state<S>(a.p, l);
+                    }
+                    point_flux<S>(a.p, l, pl, r, point_state<S>(a.p, r), nux, nuy, nx, ny, G);
+#pragma unroll
+                    for (int s = 0; s < S; ++s) {
+                        Gsum[s] += G[s];
+                        v[s] = vn[s];
+                    }
                 }
                 if (fric) {
                     // bed friction S_s = -cf |v| q_s / h (s = 1, 2) at this point
                     const double cf =
                         a.p.friction * (1.0 + (a.p.friction_dim >= 0 ? a.xi[k * a.d + a.p.friction_dim] : 0.0));
-                    const double sp = sqrt(uj[1] * uj[1] + uj[2] * uj[2]) / uj[0];
+                    const double hi = recip_any(uj[0]);
+                    const double sp = sqrt_f64(uj[1] * uj[1] + uj[2] * uj[2]) * hi;
 #pragma unroll
-                    for (int s = 1; s < S; ++s) Gsum[s] += area * (cf * sp * uj[s] / uj[0]);
+                    for (int s = 1; s < S; ++s) Gsum[s] += area * (cf * sp * uj[s] * hi);
                 }
 #pragma unroll
                 for (int s = 0; s < S; ++s) Gs[(slot * Q + k) * S + s] = Gsum[s];
@@ -276,45 +328,67 @@ __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per
         }
         wave_sync();
         // projection and update: D = A B with A(r, k) = G(cell slot r / S,
-        // state r % S, point k) and B(k, i) = phiW(k, i), 16 x 16 x 4 FP64
-        // MFMA steps (lane l: row/column l % 16, k = 4 ks + l / 16); element e
-        // of lane l is D(4 e + l / 16, l % 16)
-        const int r16 = lane & 15, kq4 = lane >> 4;
-        const int ks_n = (Q + 3) >> 2;
-        const int ar_slot = r16 / S, ar_s = r16 - ar_slot * S;
-        const long ar_cell = cell0 + ar_slot;
-        const bool ar_on = ar_slot < CPW && ar_cell < a.ncell && a.bc[ar_cell] != UQK_BC_DIRICHLET;
-        for (int ti = 0; 16 * ti < M; ++ti) {
-            const int ic = 16 * ti + r16;
-            f64x4 pacc = {0.0, 0.0, 0.0, 0.0};
-            for (int ks = 0; ks < ks_n; ++ks) {
-                const int k = 4 * ks + kq4;
-                const double av = (ar_on && k < Q) ? Gs[(ar_slot * Q + k) * S + ar_s] : 0.0;
-                const double bv = (ic < M && k < Q) ? phiw[k * M + ic] : 0.0;
-                pacc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, pacc, 0, 0, 0);
+        // state r % S, point k) and B(k, i) = phiW(k, i); the lanes that hold
+        // D(r, i) update the moment
+        const int p16 = lane & 15, q4 = lane >> 4;
+        const int ar = ONE ? p16 & 3 : p16, ar_slot = ar / S < CPW ? ar / S : 0;
+        const double* ga = Gs + ar_slot * Q * S + ar % S;
+        const bool ar_on = ONE ? ar < S && bc != UQK_BC_DIRICHLET
+                               : ar / S < CPW && cell0 + ar_slot < a.ncell &&
+                                     a.bc[cell0 + ar_slot] != UQK_BC_DIRICHLET;
+        // row r, column ic of D, with the moment's value us and its old one
+        auto update = [&](int row, int ic, double acc, double us, double old) {
+            const int cs = row / S, st = row - cs * S, f = ic * S + st;
+            const long c = cell0 + cs;
+            if (cs >= CPW || c >= a.ncell || ic >= M) return;
+            const int nt = !a.nt_cell ? M : ONE ? uniform_load(a.nt_cell + cell) : a.nt_cell[c];
+            const int bcc = ONE ? bc : a.bc[c];
+            const double ac = ONE ? uniform_load(a.area + cell) : a.area[c];
+            double v = us;
+            if (a.cut && ic >= nt) {  // past the order that the refinement chose
+                v = 0.0;
+                a.cut[c * SM + f] = 0.0;
             }
-            if (ic < M) {
+            if (bcc != UQK_BC_DIRICHLET && ic < nt) v -= (dt / ac) * acc;
+            a.u_out[c * SM + f] = v;
+            if (f == 0) res += fabs(v - old) * ac;
+        };
+        for (int ti = 0; 16 * ti < M; ++ti) {
+            const int ic = 16 * ti + p16;
+            const double* wb = phiw + (ic < M ? ic : M - 1);
+            auto load = [&](int ks) {
+                Operands<1> o;
+                const int k = 4 * ks + q4, kk = k < Q ? k : Q - 1;
+                const double x = ga[kk * S];
+                o.a = ar_on && k < Q ? x : 0.0;
+                o.b[0] = wb[kk * M];
+                return o;
+            };
+            // u: reconstructed moments; u_out: in the previous moments, out the new
+            if constexpr (ONE) {
+                // S <= 4 rows: 4 x 4 x 4 products (16 x 16 x 4 ones take four
+                // times as long); lane 16 q + p gets D(q, 16 ti + p)
+                const long f = cell0 * SM + ic * S + q4;
+                const bool has = q4 < S && ic < M && cell0 < a.ncell;
+                const double us = has ? a.u[f] : 0.0, old = has ? a.u_out[f] : 0.0;
+                double acc = 0.0;
+                in_steps<4>((Q + 3) / 4, load, [&](const Operands<1>& o) {
+                    acc = __builtin_amdgcn_mfma_f64_4x4x4f64(o.a, o.b[0], acc, 0, 0, 0);
+                });
+                update(q4, ic, acc, us, old);
+            } else {
+                f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+                for (int ks = 0; ks < (Q + 3) / 4; ++ks) {
+                    const Operands<1> o = load(ks);
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a, o.b[0], acc, 0, 0, 0);
+                }
+                settle<18>();
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = 4 * e + kq4;
-                    const int cs = row / S, st = row - cs * S;
-                    const long c = cell0 + cs;
-                    if (cs < CPW && c < a.ncell) {
-                        const int nt = a.nt_cell ? a.nt_cell[c] : M;
-                        const int bcc = a.bc[c];
-                        const int f = ic * S + st;
-                        double us = a.u[c * SM + f];        // reconstructed moments
-                        if (a.cut && ic >= nt) {             // past the order that the refinement chose
-                            us = 0.0;
-                            a.cut[c * SM + f] = 0.0;
-                        }
-                        double* un = a.u_out + c * SM;       // in: previous moments, out: new moments
-                        const double old = un[f];
-                        double v = us;
-                        if (bcc != UQK_BC_DIRICHLET && ic < nt) v = us - (dt / a.area[c]) * pacc[e];
-                        un[f] = v;
-                        if (f == 0) res += fabs(v - old) * a.area[c];
-                    }
+                for (int e = 0; e < 4; ++e) {  // element e at (4 e + q, 16 ti + p)
+                    const int row = 4 * e + q4, cs = row / S;
+                    const long f = (cell0 + cs) * SM + ic * S + row - cs * S;
+                    const bool has = cs < CPW && cell0 + cs < a.ncell && ic < M;
+                    update(row, ic, acc[e], has ? a.u[f] : 0.0, has ? a.u_out[f] : 0.0);
                 }
             }
         }
@@ -513,7 +587,7 @@ hipError_t launch_dt(int kind, const SweepArgs& a, hipStream_t st) {
 int advance_partials(int S, int Q, long ncell) {
     const long per = (long)advance_cells_per_wave(S, Q) * (kSweepThreads / 64);
     const long want = (ncell + per - 1) / per;
-    return (int)(want < 1 ? 1 : (want < kPartialBlocks ? want : kPartialBlocks));
+    return (int)(want < 1 ? 1 : (want < kAdvanceBlocks ? want : kAdvanceBlocks));
 }
 
 template <int KIND> static void go_advance(const SweepArgs& a, hipStream_t st) {
@@ -523,7 +597,11 @@ template <int KIND> static void go_advance(const SweepArgs& a, hipStream_t st) {
     // PhiW goes to LDS while a workgroup stays within 64 KB
     b.table_lds = shmem + sizeof(double) * a.Q * a.M <= 65536;
     if (b.table_lds) shmem += sizeof(double) * a.Q * a.M;
-    hipLaunchKernelGGL(advance_kernel<KIND>, dim3(advance_partials(S, a.Q, a.ncell)), dim3(kSweepThreads), shmem, st, b);
+    const dim3 blocks(advance_partials(S, a.Q, a.ncell));
+    if (advance_cells_per_wave(S, a.Q) == 1)
+        hipLaunchKernelGGL((advance_kernel<KIND, true>), blocks, dim3(kSweepThreads), shmem, st, b);
+    else
+        hipLaunchKernelGGL((advance_kernel<KIND, false>), blocks, dim3(kSweepThreads), shmem, st, b);
 }
 hipError_t launch_advance(int kind, const SweepArgs& a, hipStream_t st) {
     UQK_DISPATCH(kind, go_advance, a, st);

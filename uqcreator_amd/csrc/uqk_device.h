@@ -198,12 +198,58 @@ __device__ __forceinline__ void closure_DU(const ClosureParams& c, const double*
 }
 
 // ---------------------------------------------------------------------------
+// 1/x and sqrt(x) to an ulp: v_rcp_f64 and v_rsq_f64 with two refinements,
+// in place of the correctly rounded divide and root, which take four times
+// the instructions (and most of the time of the point fluxes).  Zero,
+// infinities and NaN as 1/x and sqrt(x) have them.
+__device__ __forceinline__ double recip_any(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    double e = fma(-x, r, 1.0);
+    const double r1 = fma(r, e, r);
+    e = fma(-x, r1, 1.0);
+    const double r2 = fma(r1, e, r1);
+    return __builtin_isfinite(r2) ? r2 : r;
+}
+__device__ __forceinline__ double sqrt_f64(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    double g = x * r, h = 0.5 * r;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x == 0.0 || x == __builtin_inf() ? x : g;
+}
+
+// Velocity, pressure and wave speed at a point (euler2d.cpp:88-112,
+// shallowwater2d.cpp:21-65), what both sides of an edge bring into its flux.
+struct PointState {
+    double vx, vy, p, c;
+};
+template <int S> __device__ __forceinline__ PointState point_state(const ProblemParams& p, const double* u) {
+    PointState q{0.0, 0.0, 0.0, 0.0};
+    if constexpr (S >= 3) {
+        const double ri = recip_any(u[0]);
+        q.vx = u[1] * ri;
+        q.vy = u[2] * ri;
+        if constexpr (S == 4) {
+            q.p = (p.gamma - 1.0) * (u[3] - 0.5 * u[0] * (q.vx * q.vx + q.vy * q.vy));
+            q.c = sqrt_f64(p.gamma * q.p * ri);
+        } else {
+            q.p = 0.5 * p.g * u[0] * u[0];
+            q.c = sqrt_f64(p.g * u[0]);
+        }
+    }
+    return q;
+}
+
 // Point fluxes G(u, v, nUnit, n): the outward flux of the cell holding u
-// through an edge with unit normal nu and scaled normal n.
+// through an edge with unit normal nu and scaled normal n; a and b are the
+// point_states of u and v.
 // ---------------------------------------------------------------------------
 template <int S>
-__device__ __forceinline__ void point_flux(const ProblemParams& p, const double* u, const double* v, double nux,
-                                           double nuy, double nx, double ny, double* out) {
+__device__ __forceinline__ void point_flux(const ProblemParams& p, const double* u, const PointState& a,
+                                           const double* v, const PointState& b, double nux, double nuy, double nx,
+                                           double ny, double* out) {
     if (p.problem == UQK_BURGERS) {
         if (p.flux == UQK_FLUX_REFERENCE) {
             // burgers.cpp:21-28
@@ -217,67 +263,37 @@ __device__ __forceinline__ void point_flux(const ProblemParams& p, const double*
         return;
     }
     if constexpr (S >= 3) {
-        double nn = sqrt(nx * nx + ny * ny);
-        double Fu[S], Fv[S];  // F . n
-        double unu, unv, au, av;
-        if (p.problem == UQK_EULER2D_PROBLEM) {
-            if constexpr (S == 4) {
-                const double gm = p.gamma;
-                double ri = 1.0 / u[0];
-                double uu = u[1] * ri, vu = u[2] * ri;
-                double pu = (gm - 1.0) * (u[3] - 0.5 * u[0] * (uu * uu + vu * vu));
-                au = sqrt(gm * pu * ri);
-                double rv = 1.0 / v[0];
-                double uv = v[1] * rv, vv = v[2] * rv;
-                double pv = (gm - 1.0) * (v[3] - 0.5 * v[0] * (uv * uv + vv * vv));
-                av = sqrt(gm * pv * rv);
-                unu = nux * uu + nuy * vu;
-                unv = nux * uv + nuy * vv;
-                // euler2d.cpp:95-112
-                Fu[0] = u[1] * nx + u[2] * ny;
-                Fu[1] = (u[1] * uu + pu) * nx + u[2] * uu * ny;
-                Fu[2] = u[1] * vu * nx + (u[2] * vu + pu) * ny;
-                Fu[3] = (u[3] + pu) * uu * nx + (u[3] + pu) * vu * ny;
-                Fv[0] = v[1] * nx + v[2] * ny;
-                Fv[1] = (v[1] * uv + pv) * nx + v[2] * uv * ny;
-                Fv[2] = v[1] * vv * nx + (v[2] * vv + pv) * ny;
-                Fv[3] = (v[3] + pv) * uv * nx + (v[3] + pv) * vv * ny;
-            }
-        } else {
-            if constexpr (S == 3) {
-                // shallowwater2d.cpp:21-65
-                const double g = p.g;
-                double uu = u[1] / u[0], vu = u[2] / u[0], uv = v[1] / v[0], vv = v[2] / v[0];
-                au = sqrt(g * u[0]);
-                av = sqrt(g * v[0]);
-                unu = nux * uu + nuy * vu;
-                unv = nux * uv + nuy * vv;
-                Fu[0] = u[1] * nx + u[2] * ny;
-                Fu[1] = (u[1] * u[1] / u[0] + 0.5 * g * u[0] * u[0]) * nx + u[1] * u[2] / u[0] * ny;
-                Fu[2] = u[1] * u[2] / u[0] * nx + (u[2] * u[2] / u[0] + 0.5 * g * u[0] * u[0]) * ny;
-                Fv[0] = v[1] * nx + v[2] * ny;
-                Fv[1] = (v[1] * v[1] / v[0] + 0.5 * g * v[0] * v[0]) * nx + v[1] * v[2] / v[0] * ny;
-                Fv[2] = v[1] * v[2] / v[0] * nx + (v[2] * v[2] / v[0] + 0.5 * g * v[0] * v[0]) * ny;
-            }
+        // F . n = (rho un, q1 un + p nx, q2 un + p ny, (E + p) un), un the
+        // velocity along the scaled normal (euler2d.cpp:95-112,
+        // shallowwater2d.cpp:21-65); the reciprocals and square roots are
+        // those of point_state, the cell's own once for all its edges
+        const double nn = sqrt_f64(nx * nx + ny * ny);
+        const double wu = a.vx * nx + a.vy * ny, wv = b.vx * nx + b.vy * ny;
+        double Fu[S], Fv[S];
+        Fu[0] = u[1] * nx + u[2] * ny;
+        Fv[0] = v[1] * nx + v[2] * ny;
+        Fu[1] = fma(u[1], wu, a.p * nx);
+        Fv[1] = fma(v[1], wv, b.p * nx);
+        Fu[2] = fma(u[2], wu, a.p * ny);
+        Fv[2] = fma(v[2], wv, b.p * ny);
+        if constexpr (S == 4) {
+            Fu[3] = (u[3] + a.p) * wu;
+            Fv[3] = (v[3] + b.p) * wv;
         }
+        const double unu = nux * a.vx + nuy * a.vy, unv = nux * b.vx + nuy * b.vy;
         if (p.flux == UQK_FLUX_REFERENCE) {
             // HLL with Davis wave speeds (euler2d.cpp:52-87)
-            double lmin = unu - au, lmax = unv + av;
-            if (lmin >= 0) {
+            const double lmin = unu - a.c, lmax = unv + b.c;
+            const double f = recip_any(lmax - lmin), ll = lmax * lmin * nn;
 #pragma unroll
-                for (int s = 0; s < S; ++s) out[s] = Fu[s];
-            } else if (lmax <= 0) {
-#pragma unroll
-                for (int s = 0; s < S; ++s) out[s] = Fv[s];
-            } else {
-                double f = 1.0 / (lmax - lmin);
-#pragma unroll
-                for (int s = 0; s < S; ++s) out[s] = f * ((lmax * Fu[s] - lmin * Fv[s]) + lmax * lmin * (v[s] - u[s]) * nn);
+            for (int s = 0; s < S; ++s) {
+                const double h = f * ((lmax * Fu[s] - lmin * Fv[s]) + ll * (v[s] - u[s]));
+                out[s] = lmin >= 0 ? Fu[s] : lmax <= 0 ? Fv[s] : h;
             }
         } else {
-            double smax = fmax(fabs(unu) + au, fabs(unv) + av);
+            const double smax = 0.5 * fmax(fabs(unu) + a.c, fabs(unv) + b.c) * nn;
 #pragma unroll
-            for (int s = 0; s < S; ++s) out[s] = 0.5 * (Fu[s] + Fv[s]) - 0.5 * smax * (v[s] - u[s]) * nn;
+            for (int s = 0; s < S; ++s) out[s] = 0.5 * (Fu[s] + Fv[s]) - smax * (v[s] - u[s]);
         }
     }
 }
@@ -288,16 +304,10 @@ template <int S>
 __device__ __forceinline__ double point_dt(const ProblemParams& p, const double* u, double dx) {
     if (p.problem == UQK_BURGERS) return p.cfl * dx / fabs(u[0]);
     if constexpr (S >= 3) {
-        double ri = 1.0 / u[0];
-        double vx = u[1] * ri, vy = u[2] * ri, a;
-        if constexpr (S == 4) {
-            double pr = (p.gamma - 1.0) * (u[3] - 0.5 * u[0] * (vx * vx + vy * vy));
-            a = sqrt(p.gamma * pr * ri);
-        } else {
-            a = sqrt(p.g * u[0]);
-        }
-        return (p.cfl / dx) * fmin(fmin(fabs(1.0 / (vy - a)), fabs(1.0 / (vy + a))),
-                                   fmin(fabs(1.0 / (vx + a)), fabs(1.0 / (vx - a))));
+        // min |1 / w| over the wave speeds w as 1 / max |w|: one reciprocal
+        const PointState q = point_state<S>(p, u);
+        return (p.cfl / dx) * recip_any(fmax(fmax(fabs(q.vy - q.c), fabs(q.vy + q.c)),
+                                             fmax(fabs(q.vx + q.c), fabs(q.vx - q.c))));
     }
     return 1e10;
 }
