@@ -43,6 +43,7 @@ constexpr int kLayers = 5;  // four hidden + head
 constexpr int kTile = 64;   // GEMM workgroup tile (rows and columns)
 constexpr int kKs = 32;     // GEMM K step (one MFMA 16x16x32)
 constexpr int kLdsStride = 40;  // bf16 per LDS tile row (32 + 8 pad)
+constexpr long kNetSmallRows = 4096;  // rows up to which the fused network takes 16 per workgroup
 constexpr long kPredictChunk = 1L << 16;  // rows per inference pass of the warm start
 
 enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2, EPI_ATOMIC = 3 };
@@ -63,15 +64,25 @@ struct GemmArgs {
     int k_split;              // K range per blockIdx.z (a multiple of 32)
 };
 
+// 2 / d for d >= 1 (an exponential plus one), rounded as the division: v_rcp's
+// estimate and one remainder give the same for all 835,318,475 floats of
+// [1, 1e30], in four instructions in place of ten.  Above, where 1 - 2 / d is
+// 1 either way, d counts as 1e30.
+__device__ __forceinline__ float two_over(float d) {
+    d = fminf(d, 1e30f);
+    const float r = __builtin_amdgcn_rcpf(d), q = 2.0f * r;
+    return fmaf(fmaf(-d, q, 2.0f), r, q);
+}
+
 __device__ __forceinline__ float gelu_f(float z) {
     const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-    const float th = 1.0f - 2.0f / (expf(2.0f * u) + 1.0f);
+    const float th = 1.0f - two_over(expf(2.0f * u) + 1.0f);
     return 0.5f * z * (1.0f + th);
 }
 
 __device__ __forceinline__ float gelu_prime_f(float z) {
     const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-    const float th = 1.0f - 2.0f / (expf(2.0f * u) + 1.0f);
+    const float th = 1.0f - two_over(expf(2.0f * u) + 1.0f);
     return 0.5f * (1.0f + th) + 0.5f * z * (1.0f - th * th) * 0.7978845608028654f * (1.0f + 0.134145f * z * z);
 }
 
@@ -157,6 +168,138 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
                     atomicAdd(&g.f[(size_t)m * g.ldf + n], v);
                 }
             }
+}
+
+// The whole network for 16 RT rows per workgroup: the activations stay in LDS
+// (two buffers, a row of the widest layer and 8 padding), the weights come
+// from L2 as operands, each wavefront's next 32 inputs of up to four tiles of
+// 16 outputs loaded while the last are multiplied.  The products, their order
+// over the inputs and the rounding of the activations are those of
+// gemm_bf16_kernel, bit for bit.
+// What bounds it: the GELUs (an exponential and a division each, in FP32) and
+// the matrix steps, about as much time; layer by layer the activations went
+// out and back (67 MB per layer of 65,536 rows and 256 outputs) through tiles
+// of 64 x 64 with two barriers per 32 inputs.  65,536 rows, 256 hidden: 101 us
+// (five GEMMs of 37 us but the last); a batch of 1,024: 28 us (five of 7).
+struct NetArgs {
+    int rows, ld;
+    int dims[kLayers + 1];
+    long off[kLayers];
+    const __bf16 *x, *w;       // inputs; weights W_l (N x K) at off[l]
+    const float* p;            // FP32 parameters (the biases, after W_l)
+    float* y;
+    float* z[kLayers - 1];     // pre-activations and activations for the
+    __bf16* act[kLayers];      // backward pass (may be null)
+};
+__device__ __forceinline__ void matrix_settle() {  // before results are read where paths join (tile_solve.h)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int RT>
+__global__ __launch_bounds__(256) void net_kernel(NetArgs a) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 net_lds[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, p16 = lane & 15, q4 = lane >> 4;
+    const long r0 = (long)blockIdx.x * (16 * RT);
+    __bf16 *cur = net_lds, *nxt = net_lds + 16 * RT * a.ld;
+    for (int t = threadIdx.x; t < 16 * RT * (a.dims[0] / 8); t += 256) {
+        const int row = t / (a.dims[0] / 8), c = t - row * (a.dims[0] / 8);
+        bf16x8 v = {};
+        if (r0 + row < a.rows) v = *reinterpret_cast<const bf16x8*>(a.x + (r0 + row) * a.dims[0] + 8 * c);
+        *reinterpret_cast<bf16x8*>(cur + row * a.ld + 8 * c) = v;
+    }
+    for (int l = 0; l < kLayers; ++l) {
+        const int K = a.dims[l], N = a.dims[l + 1];
+        const __bf16* W = a.w + a.off[l];
+        const float* bias = a.p + a.off[l] + (long)N * K;
+        __syncthreads();
+        // output tiles t0, t0 + 4, .. (NJ of them)
+        auto part = [&](int t0, auto count) {
+            constexpr int NJ = decltype(count)::value;
+            f32x4 acc[RT][NJ];
+            bf16x8 bn[NJ];
+            const __bf16* wp[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                wp[j] = W + (size_t)(16 * (t0 + 4 * j) + p16) * K + 8 * q4;
+                bn[j] = *reinterpret_cast<const bf16x8*>(wp[j]);
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[r][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            for (int k0 = 0; k0 < K; k0 += kKs) {
+                bf16x8 b[NJ], x[RT];
+                const int kn = k0 + kKs < K ? k0 + kKs : 0;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    b[j] = bn[j];
+                    bn[j] = *reinterpret_cast<const bf16x8*>(wp[j] + kn);
+                }
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+                    x[r] = *reinterpret_cast<const bf16x8*>(cur + (16 * r + p16) * a.ld + k0 + 8 * q4);
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[r], b[j], acc[r][j], 0, 0, 0);
+            }
+            matrix_settle();
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float bv = bias[16 * (t0 + 4 * j) + p16];
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[r][j][i] += bv;
+            }
+            // element i: row 16 r + 4 q + i, output 16 (t0 + 4 j) + p
+            if (l + 1 < kLayers) {
+                __bf16* out = nxt + 4 * q4 * a.ld + 16 * t0 + p16;
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            out[(16 * r + i) * a.ld + 64 * j] = (__bf16)gelu_f(acc[r][j][i]);
+            }
+            float* zo = l + 1 < kLayers ? a.z[l] : a.y;
+            if (zo) {
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const long m = r0 + 16 * r + 4 * q4 + i;
+                        if (m >= a.rows) continue;
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) zo[m * N + 16 * (t0 + 4 * j) + p16] = acc[r][j][i];
+                    }
+            }
+        };
+        const int tiles = N / 16;
+        for (int t0 = wave; t0 < tiles;) {
+            if (t0 + 12 < tiles) {
+                part(t0, std::integral_constant<int, 4>());
+                t0 += 16;
+            } else {
+                part(t0, std::integral_constant<int, 1>());
+                t0 += 4;
+            }
+        }
+        __bf16* x = cur;
+        cur = nxt;
+        nxt = x;
+        // the backward pass takes the activations (rows of 8, from LDS)
+        if (l + 1 < kLayers && a.z[l]) {
+            __syncthreads();
+            for (int t = threadIdx.x; t < 16 * RT * (N / 8); t += 256) {
+                const int row = t / (N / 8), c = t - row * (N / 8);
+                if (r0 + row < a.rows)
+                    *reinterpret_cast<bf16x8*>(a.act[l + 1] + (r0 + row) * N + 8 * c) =
+                        *reinterpret_cast<const bf16x8*>(cur + row * a.ld + 8 * c);
+            }
+        }
+    }
 }
 
 // db[n] += sum over rows of x[row*ld + n] (x FP32 or BF16): a block of 256
@@ -671,6 +814,36 @@ int ensure_rows(uqk_mlp* n, long rows) {
 
 // forward over rows already staged in act[0]; store_z keeps what backward needs
 int forward(uqk_mlp* n, long rows, bool store_z) {
+    // the fused network where its activations leave two workgroups per CU:
+    // 64 rows per workgroup for many rows, 16 for a training batch (which
+    // would fill a few CUs only, and with more rows read the weights too often)
+    int widest = 0;
+    for (int l = 0; l <= kLayers; ++l) widest = std::max(widest, n->dims[l]);
+    const int rt = rows > kNetSmallRows ? 4 : 1;
+    const size_t lds = sizeof(__bf16) * 2 * 16 * rt * (size_t)(widest + 8);
+    bool whole = rows > 0 && lds <= 80 * 1024;
+    for (int l = 0; l <= kLayers; ++l) whole = whole && n->dims[l] % kKs == 0;
+    if (whole) {
+        NetArgs a{};
+        a.rows = (int)rows;
+        a.ld = widest + 8;
+        for (int l = 0; l <= kLayers; ++l) a.dims[l] = n->dims[l];
+        for (int l = 0; l < kLayers; ++l) a.off[l] = n->off[l];
+        a.x = n->act[0];
+        a.w = n->ph;
+        a.p = n->p;
+        a.y = n->y;
+        for (int l = 0; l + 1 < kLayers; ++l) {
+            a.z[l] = store_z ? n->z[l] : nullptr;
+            a.act[l + 1] = n->act[l + 1];
+        }
+        if (rt == 4)
+            hipLaunchKernelGGL(net_kernel<4>, dim3(blocks(rows, 64)), dim3(256), lds, n->ctx->stream, a);
+        else
+            hipLaunchKernelGGL(net_kernel<1>, dim3(blocks(rows, 16)), dim3(256), lds, n->ctx->stream, a);
+        MLP_HIP(n, hipGetLastError());
+        return 0;
+    }
     for (int l = 0; l < kLayers; ++l) {
         GemmArgs a{};
         a.M = (int)rows;
