@@ -49,22 +49,48 @@ __global__ void __launch_bounds__(kSweepThreads) eval_uq_kernel(SweepArgs a) {
     for (int s = 0; s < S; ++s) out[s] = Uv[s];
 }
 
-// One thread per output moment (cell, i, s): u(s,i) = sum_k uq(s,k) phiw(k,i) for i < nt.
+// u(s, i) = sum_k uq(s, k) phiw(k, i) for i < nt: a wavefront's 16 / S cells
+// as one FP64 matrix product (rows: cell slot x state), 16 moments at a time;
+// uQ is read once, a cell's four points of a step together, and two passes'
+// steps are in flight.  It is bound by that read (65,536 cells at 25 points,
+// four states: 27 us; one thread per moment, every uQ read M times through
+// L1, 65 us).
+template <int S>
 __global__ void __launch_bounds__(kSweepThreads) reconstruct_kernel(SweepArgs a) {
+    constexpr int CPW = 16 / S;
     UQK_SKIP_IF_INACTIVE(a)
-    const int S = a.S, M = a.M, Q = a.Q;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.ncell * S * M) return;
-    long cell = t / (S * M);
-    int e = (int)(t - cell * S * M);
-    int i = e / S, s = e - i * S;
-    int nt = a.nt_cell ? a.nt_cell[cell] : M;
-    double acc = 0.0;
-    if (i < nt) {
-        const double* q = a.uq + cell * S * Q;
-        for (int k = 0; k < Q; ++k) acc += q[k * S + s] * a.phiw[k * M + i];
+    const int M = a.M, Q = a.Q;
+    const int lane = threadIdx.x & 63, p16 = lane & 15, q4 = lane >> 4;
+    const long cell0 = ((long)blockIdx.x * (kSweepThreads / 64) + (threadIdx.x >> 6)) * CPW;
+    if (cell0 >= a.ncell) return;
+    const int slot = p16 / S < CPW ? p16 / S : 0;
+    const long ca = cell0 + slot < a.ncell ? cell0 + slot : a.ncell - 1;
+    const double* ua = a.uq + ca * S * Q + p16 % S;
+    for (int ti = 0; 16 * ti < M; ++ti) {
+        const int ic = 16 * ti + p16;
+        const double* wb = a.phiw + (ic < M ? ic : M - 1);
+        f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+        in_steps<4>(
+            (Q + 3) / 4,
+            [&](int ks) {
+                Operands<1> o;
+                const int k = 4 * ks + q4, kk = k < Q ? k : Q - 1;
+                const double x = ua[kk * S], w = wb[kk * M];
+                o.a = k < Q ? x : 0.0;
+                o.b[0] = k < Q ? w : 0.0;
+                return o;
+            },
+            [&](const Operands<1>& o) { acc = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a, o.b[0], acc, 0, 0, 0); });
+        settle<18>();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // element e at (4 e + q, 16 ti + p)
+            const int row = 4 * e + q4, cs = row / S;
+            const long c = cell0 + cs;
+            if (cs >= CPW || c >= a.ncell || ic >= M) continue;
+            const int nt = a.nt_cell ? a.nt_cell[c] : M;
+            a.u_out[c * S * M + ic * S + row % S] = ic < nt ? acc[e] : 0.0;
+        }
     }
-    a.u_out[t] = acc;
 }
 
 // MomentSolver refinement (momentsolver.cpp:104-117) with ComputeRefIndicator
@@ -399,59 +425,80 @@ __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per
     if (threadIdx.x == 0) a.partial[blockIdx.x] = res;
 }
 
+// sum over the SUB lanes (32 or 64) that share a cell, in every lane
+template <int SUB> __device__ __forceinline__ double sub_sum(double v) {
+    v = row_sum(v);
+    if constexpr (SUB == 64) return group_sum(v);
+    const long long x = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(x >> 32), false, false);
+    return __longlong_as_double(((long long)hi[0] << 32) | (unsigned)lo[0]) +
+           __longlong_as_double(((long long)hi[1] << 32) | (unsigned)lo[1]);
+}
+
 // E and Var of each state from the closure at lambda (WriteMeanAndVar,
-// momentsolver.cpp:302-328): one wavefront per cell, lanes over quadrature
-// points (up to 128 per cell), the two weighted sums as wave reductions.  The
-// cell's duals are read by all lanes at once (one cache line, broadcast).
-template <int KIND>
+// momentsolver.cpp:302-328): lanes over quadrature points (up to 128 per
+// cell), the two weighted sums over them by DPP and row swaps.  A wavefront
+// has two cells where they have 32 points or fewer, else one.  Bound by the
+// loads of the duals and the closure's exponentials: 65,536 cells at 25
+// points, four states: 42 us (108 with one cell per wavefront, U formed
+// for a second point that no lane had, and sums through LDS).
+template <int KIND, int SUB>
 __global__ void __launch_bounds__(kSweepThreads) mean_var_kernel(SweepArgs a) {
     constexpr int S = KindInfo<KIND>::S;
-    constexpr int KP = 2;  // quadrature points per lane
-    const int lane = threadIdx.x & 63;
-    const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
-    for (long cell = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); cell < a.ncell; cell += nwaves) {
+    constexpr int KP = SUB == 64 ? 2 : 1;  // quadrature points per lane
+    constexpr int CPW = 64 / SUB;
+    const int lane = threadIdx.x & (SUB - 1), half = (threadIdx.x & 63) / SUB;
+    const long step = (long)gridDim.x * (blockDim.x >> 6) * CPW;
+    for (long cell0 = ((long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * CPW; cell0 < a.ncell;
+         cell0 += step) {
+        const bool has = cell0 + half < a.ncell;
+        const long cell = has ? cell0 + half : cell0;
         const int nt = a.nt_cell ? a.nt_cell[cell] : a.M;
         const double* lam = a.lam + cell * S * a.M;
         double Uv[KP][S], w0[KP];
 #pragma unroll
         for (int h = 0; h < KP; ++h) {
-            const int k = lane + 64 * h;
-            double L[S];
+            const int k = lane + SUB * h;
 #pragma unroll
-            for (int s = 0; s < S; ++s) L[s] = 0.0;
+            for (int s = 0; s < S; ++s) Uv[h][s] = 0.0;  // (U of Lambda = 0 may be NaN)
             w0[h] = 0.0;
             if (k < a.Q) {
+                double L[S];
+#pragma unroll
+                for (int s = 0; s < S; ++s) L[s] = 0.0;
+                const double* ph = a.phi + k * a.M;
+#pragma unroll 4
                 for (int i = 0; i < nt; ++i) {
-                    const double p = a.phi[k * a.M + i];
+                    const double p = ph[i];
 #pragma unroll
                     for (int s = 0; s < S; ++s) L[s] += lam[i * S + s] * p;
                 }
                 w0[h] = a.phiw[k * a.M + 0];
-            }
-            closure_U<KIND>(a.c, L, Uv[h]);
-            if (k >= a.Q) {
-#pragma unroll
-                for (int s = 0; s < S; ++s) Uv[h][s] = 0.0;  // U of Lambda = 0 may be NaN
+                closure_U<KIND>(a.c, L, Uv[h]);
             }
         }
-        double E[S];
+        double E[S], V[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             double e = 0.0;
 #pragma unroll
             for (int h = 0; h < KP; ++h) e += Uv[h][s] * w0[h];
-            E[s] = wave_sum(e);
+            E[s] = sub_sum<SUB>(e);
         }
-        double* out = a.mv_out + cell * 2 * S;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             double v = 0.0;
 #pragma unroll
             for (int h = 0; h < KP; ++h) v += (Uv[h][s] - E[s]) * (Uv[h][s] - E[s]) * w0[h];
-            v = wave_sum(v);
-            if (lane == 0) {
+            V[s] = sub_sum<SUB>(v);
+        }
+        if (lane == 0 && has) {
+            double* out = a.mv_out + cell * 2 * S;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
                 out[s] = E[s];
-                out[S + s] = v;
+                out[S + s] = V[s];
             }
         }
     }
@@ -560,9 +607,14 @@ hipError_t launch_refine(const RefineArgs& a, hipStream_t st) {
 
 hipError_t launch_reconstruct(const SweepArgs& a, hipStream_t st) {
     if (a.ncell <= 0) return hipSuccess;
-    long total = a.ncell * a.S * a.M;
-    int blocks = (int)((total + kSweepThreads - 1) / kSweepThreads);
-    hipLaunchKernelGGL(reconstruct_kernel, dim3(blocks), dim3(kSweepThreads), 0, st, a);
+    const long per = (kSweepThreads / 64) * (16 / a.S);
+    const dim3 blocks((unsigned)((a.ncell + per - 1) / per));
+    switch (a.S) {
+        case 1: hipLaunchKernelGGL(reconstruct_kernel<1>, blocks, dim3(kSweepThreads), 0, st, a); break;
+        case 3: hipLaunchKernelGGL(reconstruct_kernel<3>, blocks, dim3(kSweepThreads), 0, st, a); break;
+        case 4: hipLaunchKernelGGL(reconstruct_kernel<4>, blocks, dim3(kSweepThreads), 0, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
@@ -616,10 +668,13 @@ hipError_t launch_residual(const SweepArgs& a, hipStream_t st) {
 }
 
 template <int KIND> static void go_mean_var(const SweepArgs& a, hipStream_t st) {
-    const long waves = kSweepThreads / 64;
-    const long want = (a.ncell + waves - 1) / waves;
-    const int blocks = (int)(want < kPartialBlocks ? want : kPartialBlocks);
-    hipLaunchKernelGGL(mean_var_kernel<KIND>, dim3(blocks), dim3(kSweepThreads), 0, st, a);
+    const long per = (kSweepThreads / 64) * (a.Q <= 32 ? 2 : 1);
+    const long want = (a.ncell + per - 1) / per;
+    const dim3 blocks((unsigned)(want < kPartialBlocks ? want : kPartialBlocks));
+    if (a.Q <= 32)
+        hipLaunchKernelGGL((mean_var_kernel<KIND, 32>), blocks, dim3(kSweepThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL((mean_var_kernel<KIND, 64>), blocks, dim3(kSweepThreads), 0, st, a);
 }
 hipError_t launch_mean_var(int kind, const SweepArgs& a, hipStream_t st) {
     if (a.ncell <= 0) return hipSuccess;
