@@ -128,11 +128,9 @@ class C3:
         fm = flop_model(4, self.b.M, self.b.Q)
         S, M, Q = 4, self.b.M, self.b.Q
         # the closure's timing window: the residual check (from the last
-        # step's moments after the run's first step), the Newton kernel and,
-        # in the mixed time loop with kept inverses, the inverse kernel
+        # step's moments after the run's first step) and the Newton kernel
         kname = ("closure_recheck_kernel<2,10,25> (closure_check_kernel<2,10,25> in the first step) + " +
-                 ("newton_wave_kernel<2,10,25,2> + factor_inverse_kernel<40>" if lagged > 0 else
-                  "newton_wave_kernel<2,10,25,%d>" % precision))
+                 "newton_wave_kernel<2,10,25,%d>" % (2 if lagged > 0 else 0))
         roof_c = closure_roofline(kname, closure_ms / timed_steps, newton / args.steps, grads / args.steps, fm,
                                   precision == native.MIXED, factors / args.steps, lagged / args.steps)
         adv_ms = advance_ms / timed_steps

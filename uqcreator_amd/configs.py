@@ -168,9 +168,9 @@ def _legs(make_closure, prob, m, u, lam0, nt, steps, params, closure_from_lam0, 
         if nt is None:
             fm = roofline.flop_model(S, M, Q)
             block = cl.last_kernel() == native.KERNEL_BLOCK
-            # (the workgroup kernel's mixed time loop is its kept-factor instantiation, <KIND, 2>)
+            # (the mixed time loop of large systems is the instantiation that keeps inverses, <.., 1>)
             r["roofline_closure"] = roofline.closure_roofline(
-                kernels["closure"] % (2 if block and prec == native.MIXED else prec), cms, newton / steps,
+                kernels["closure"] % int(block and prec == native.MIXED), cms, newton / steps,
                 grads / steps, fm, prec == native.MIXED, factors / steps, lagged / steps)
         print("case:", leg, "loop", {k: r[k] for k in ("value", "ms_per_step", "newton_steps_per_cell_step",
                                                        "mean_var_rel_l2_vs_fp64")}, file=sys.stderr, flush=True)
@@ -182,7 +182,7 @@ def _legs(make_closure, prob, m, u, lam0, nt, steps, params, closure_from_lam0, 
 
 def c4(steps, pairs=5_000_000, adam_steps=19200):
     """Per-cell orders 1..6 on the 2D Euler NACA setup (7x7 points, n up to
-    112: the workgroup kernel)."""
+    112: the kernel for large systems)."""
     b, m, u, lam0, nt = workloads.euler2d_c4()
     prob = native.problem(native.EULER2D_PROBLEM, flux=native.FLUX_LAX_FRIEDRICHS, cfl=0.4)
 
@@ -196,7 +196,7 @@ def c4(steps, pairs=5_000_000, adam_steps=19200):
     del du, dl
     info["pairs"] = npairs
     legs = _legs(make, prob, m, u, lam0, nt, steps, params, True,
-                 {"closure": "newton_block_kernel<2,%d>", "advance": "advance_kernel"})
+                 {"closure": "newton_wide_kernel<2,8,%d>", "advance": "advance_kernel"})
     out = {"case": "c4", "workload": "2D Euler NACA0012 O-grid 512x128, per-cell orders 1..6 (nTotal 3..28, "
                                      "seeded), 7x7 Gauss, Rusanov flux, CFL 0.4",
            "n_cells": m.n_cells, "warm_start_training": info, "legs": legs,
@@ -232,7 +232,7 @@ def c5(steps, pairs=5_000_000, adam_steps=19200):
     del du, dl
     info["pairs"] = npairs
     legs = _legs(make, prob, m, u, lam0, None, steps, params, False,
-                 {"closure": "newton_block_kernel<4,%d>", "advance": "advance_kernel"})
+                 {"closure": "newton_wide_kernel<4,7,%d>", "advance": "advance_kernel"})
     out = {"case": "c5", "workload": "shallow-water dam break 1024x1024, barrier 0.01, total degree 4 (35 x 3 = "
                                      "105 duals), 5^3 Gauss, HLL flux, friction 0.01 (1 + xi3), CFL 0.45",
            "n_cells": m.n_cells, "warm_start_training": info, "legs": legs,

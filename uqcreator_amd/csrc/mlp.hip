@@ -86,20 +86,19 @@ __device__ __forceinline__ float gelu_prime_f(float z) {
     return 0.5f * (1.0f + th) + 0.5f * z * (1.0f - th * th) * 0.7978845608028654f * (1.0f + 0.134145f * z * z);
 }
 
-// Stage a 64 x 32 tile of an operand into LDS as [row][k] (row = m or n).
-// Not transposed: rows r0.. of P[row*ld + k]; transposed: P[k*ld + row].
+// A thread's part of a 64 x 32 tile of an operand (row = m or n), and its
+// place in LDS as [row][k].  Not transposed: rows r0.. of P[row*ld + k];
+// transposed: P[k*ld + row].
 template <bool T>
-__device__ __forceinline__ void stage(__bf16* S, const __bf16* P, int ld, int r0, int R, int k0) {
+__device__ __forceinline__ bf16x8 load_tile(const __bf16* P, int ld, int r0, int R, int k0) {
     const int t = threadIdx.x;
+    bf16x8 v = {};
     if constexpr (!T) {
         const int row = t >> 2, kc = (t & 3) * 8;
-        bf16x8 v = {};
         if (r0 + row < R) v = *reinterpret_cast<const bf16x8*>(P + (size_t)(r0 + row) * ld + k0 + kc);
-        *reinterpret_cast<bf16x8*>(S + row * kLdsStride + kc) = v;
     } else {
         const int kk = t >> 3, rc = (t & 7) * 8;
         const __bf16* src = P + (size_t)(k0 + kk) * ld + r0 + rc;
-        bf16x8 v = {};
         if (r0 + rc + 8 <= R) {
             v = *reinterpret_cast<const bf16x8*>(src);
         } else {
@@ -107,14 +106,31 @@ __device__ __forceinline__ void stage(__bf16* S, const __bf16* P, int ld, int r0
             for (int j = 0; j < 8; ++j)
                 if (r0 + rc + j < R) v[j] = src[j];
         }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) S[(rc + j) * kLdsStride + kk] = v[j];
     }
+    return v;
+}
+template <bool T> __device__ __forceinline__ void store_tile(__bf16* S, bf16x8 v) {
+    const int t = threadIdx.x;
+    if constexpr (!T) {
+        *reinterpret_cast<bf16x8*>(S + (t >> 2) * kLdsStride + (t & 3) * 8) = v;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) S[((t & 7) * 8 + j) * kLdsStride + (t >> 3)] = v[j];
+    }
+}
+
+__device__ __forceinline__ void matrix_settle() {  // before results are read where paths join (tile_solve.h)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // C (M x N) = op(A) op(B)^T over K with a fused epilogue.  256 threads, a
 // 64 x 64 tile per workgroup, each wave a 32 x 32 quarter (2 x 2 MFMA tiles).
-// blockIdx.z splits K (ATOMIC epilogue only).
+// blockIdx.z splits K (ATOMIC epilogue only).  The operands are sent for four
+// steps of 32 ahead: a training batch leaves a tenth of the chip's workgroups,
+// each of which otherwise waits for memory once per step (1,024 rows, 256
+// hidden: weight gradient 16.7 us, input gradient 11.5 us).
 template <bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(16))) __bf16 As[kTile * kLdsStride];
@@ -129,23 +145,44 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kb; k0 < ke; k0 += kKs) {
-        stage<TA>(As, g.A, g.lda, m0, g.M, k0);
-        stage<TB>(Bs, g.B, g.ldb, n0, g.N, k0);
-        __syncthreads();
-        bf16x8 a[2], b[2];
+    constexpr int PF = 4;
+    bf16x8 pa[PF], pb[PF];
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
-            a[r] = *reinterpret_cast<const bf16x8*>(As + (wr + r * 16 + (lane & 15)) * kLdsStride + 8 * (lane >> 4));
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-            b[c] = *reinterpret_cast<const bf16x8*>(Bs + (wc + c * 16 + (lane & 15)) * kLdsStride + 8 * (lane >> 4));
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
-        __syncthreads();
+    for (int u = 0; u < PF; ++u) {
+        pa[u] = pb[u] = bf16x8{};
+        if (kb + u * kKs < ke) {
+            pa[u] = load_tile<TA>(g.A, g.lda, m0, g.M, kb + u * kKs);
+            pb[u] = load_tile<TB>(g.B, g.ldb, n0, g.N, kb + u * kKs);
+        }
     }
+    for (int k4 = kb; k4 < ke; k4 += PF * kKs) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int k0 = k4 + u * kKs;
+            if (k0 >= ke) break;
+            store_tile<TA>(As, pa[u]);
+            store_tile<TB>(Bs, pb[u]);
+            if (k0 + PF * kKs < ke) {
+                pa[u] = load_tile<TA>(g.A, g.lda, m0, g.M, k0 + PF * kKs);
+                pb[u] = load_tile<TB>(g.B, g.ldb, n0, g.N, k0 + PF * kKs);
+            }
+            __syncthreads();
+            bf16x8 a[2], b[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                a[r] = *reinterpret_cast<const bf16x8*>(As + (wr + r * 16 + (lane & 15)) * kLdsStride + 8 * (lane >> 4));
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                b[c] = *reinterpret_cast<const bf16x8*>(Bs + (wc + c * 16 + (lane & 15)) * kLdsStride + 8 * (lane >> 4));
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
+            __syncthreads();
+        }
+    }
+    matrix_settle();
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -191,11 +228,6 @@ struct NetArgs {
     float* z[kLayers - 1];     // pre-activations and activations for the
     __bf16* act[kLayers];      // backward pass (may be null)
 };
-__device__ __forceinline__ void matrix_settle() {  // before results are read where paths join (tile_solve.h)
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 15");
-    __builtin_amdgcn_sched_barrier(0);
-}
 template <int RT>
 __global__ __launch_bounds__(256) void net_kernel(NetArgs a) {
     extern __shared__ __attribute__((aligned(16))) __bf16 net_lds[];
@@ -324,21 +356,27 @@ __global__ __launch_bounds__(256) void colsum_kernel(const T* x, int ld, int row
 // FP32 (bias gradient) and BF16 (products) copies; loss accumulated in FP64.
 __global__ void loss_kernel(const float* y, const float* t, int rows, int NO, int n_real, float* dyf, __bf16* dyh,
                             double* loss) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double part[4];
     double e2 = 0.0;
-    if (i < (size_t)rows * NO) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < (size_t)rows * NO;
+         i += (size_t)gridDim.x * blockDim.x) {
         const int n = (int)(i % NO);
         float d = 0.f;
         if (n < n_real) {
             const float e = y[i] - t[i];
-            e2 = (double)e * e;
+            e2 += (double)e * e;
             d = 2.0f * e / ((float)rows * (float)n_real);
         }
         dyf[i] = d;
         dyh[i] = (__bf16)d;
     }
+    // one atomic per workgroup (they take 12 ns each on one address: 1,024
+    // wavefronts of a batch of 1,024 rows took 15 us)
     e2 = uqk::wave_sum(e2);
-    if ((threadIdx.x & 63) == 0 && e2 != 0.0) atomicAdd(loss, e2 / ((double)rows * n_real));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = e2;
+    __syncthreads();
+    e2 = (part[0] + part[1]) + (part[2] + part[3]);
+    if (threadIdx.x == 0 && e2 != 0.0) atomicAdd(loss, e2 / ((double)rows * n_real));
 }
 
 // Adam (Kingma and Ba 2015) on the FP32 masters, BF16 copies refreshed.
@@ -876,7 +914,7 @@ int forward(uqk_mlp* n, long rows, bool store_z) {
 int backward(uqk_mlp* n, long rows, int n_real) {
     hipStream_t st = n->ctx->stream;
     hipLaunchKernelGGL(fill_f32_kernel, dim3(blocks(n->np)), dim3(256), 0, st, n->g, n->np, 0.f);
-    hipLaunchKernelGGL(loss_kernel, dim3(blocks(rows * n->NO)), dim3(256), 0, st, n->y, n->t, (int)rows, n->NO,
+    hipLaunchKernelGGL(loss_kernel, dim3(std::min(blocks(rows * n->NO), 128u)), dim3(256), 0, st, n->y, n->t, (int)rows, n->NO,
                        n_real, n->dyf, n->dyh, n->d_loss);
     const __bf16* dcur = n->dyh;
     int ldcur = n->NO;

@@ -8,7 +8,6 @@ import numpy as np
 
 # dense peaks of one MI355X
 FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3
 HBM_PEAK_GBS = 8000.0
 
 
@@ -40,13 +39,12 @@ def advance_bytes_per_cell(S, M, Q, edges, dim):
 def closure_roofline(kernel, kernel_ms, newton, grads, fm, precision_mixed, factors=None, lagged=0.0,
                      reuse="inverse"):
     """Roofline of a closure launch: algorithmic flops over its HIP-event
-    time; the peak is time-weighted over the units the flops run on (Hessian
-    on FP64 or FP32 MFMA, the rest FP64).  factors / lagged: factored Newton
+    time against the FP64 peak, on which all of them run (the mixed closure's
+    Hessian too; precision_mixed changes nothing any more).  factors / lagged: factored Newton
     steps and steps on a kept factorisation (mixed closure; by default every
     Newton step is factored).  reuse: "inverse" (the time loop keeps an
-    inverse per factorisation -- the wave kernel's H^-1, the workgroup
-    kernel's U^-1 formed at its first use -- F_inv + F_lag) or "factor" (a
-    single call solves with its last factor, F_tri)."""
+    inverse per factorisation, F_inv + F_lag) or "factor" (a single call solves
+    with its last factor, F_tri)."""
     if factors is None:
         factors = newton
     f_hess = factors * fm["F_H"]
@@ -57,10 +55,8 @@ def closure_roofline(kernel, kernel_ms, newton, grads, fm, precision_mixed, fact
         else:
             f_fp64 += lagged * fm["F_tri"]
     flops = f_hess + f_fp64
-    hess_peak = FP32_PEAK_TFLOPS if precision_mixed else FP64_PEAK_TFLOPS
-    t_min = f_hess / (hess_peak * 1e12) + f_fp64 / (FP64_PEAK_TFLOPS * 1e12)
     achieved = flops / (kernel_ms * 1e-3) / 1e12 if kernel_ms > 0 else 0.0
-    peak = flops / t_min / 1e12 if t_min > 0 else FP64_PEAK_TFLOPS
+    peak = FP64_PEAK_TFLOPS
     return {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
             "traffic": None, "kernel": kernel, "kernel_ms": kernel_ms, "flops_per_launch": flops,
             "hessian_flops_per_launch": f_hess, "newton_steps_per_launch": newton,
