@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(kCheckThreads) closure_check_kernel(NewtonArgs
         for (int i = 0; i < M; ++i) {
             const double f = tphi[k * M + i];
 #pragma unroll
-            for (int s = 0; s < S; ++s) L[s] += lam[i * S + s] * f;
+            for (int s = 0; s < S; ++s) L[s] = fma(lam[i * S + s], f, L[s]);
         }
         closure_U<KIND>(c, L, U);
         if (valid) {

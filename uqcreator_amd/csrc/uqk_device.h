@@ -76,7 +76,8 @@ __device__ __forceinline__ double bb_du(double lam, double um, double up) {
 // (eulerclosure.cpp:7-12; eulerclosure2d.cpp:7-17, whose (-v4)^(1 / (1 - gamma))
 // is taken into the exponential: equal up to rounding, no pow).
 __device__ __forceinline__ double euler_rho(double v0, double q, double w, double r, double gm) {
-    const double x = v0 - log(-w) - gm - 0.5 * q * r, g1 = gm - 1.0, k = recip_f64(g1);
+#pragma clang fp contract(off)
+    const double x = fma(-0.5 * q, r, (v0 - log(-w)) - gm), g1 = gm - 1.0, k = recip_f64(g1);
     const double e = x * k;
     return exp(fma(fma(-e, g1, x), k, e));  // (the quotient corrected once: exp magnifies its error)
 }
@@ -84,6 +85,9 @@ __device__ __forceinline__ double euler_rho(double v0, double q, double w, doubl
 // Vector form of U (the one Closure::Gradient uses).
 template <int KIND>
 __device__ __forceinline__ void closure_U(const ClosureParams& c, const double* L, double* out) {
+    // (every fused multiply-add is written out: the residual checks and the
+    // Newton kernels get the same bits)
+#pragma clang fp contract(off)
     if constexpr (KIND == UQK_BOUNDED_BARRIER) {
         out[0] = bb_u(L[0], c.u_minus, c.u_plus);
     } else if constexpr (KIND == UQK_EULER1D) {
@@ -92,24 +96,24 @@ __device__ __forceinline__ void closure_U(const ClosureParams& c, const double* 
         const double rho = euler_rho(L[0], q, L[2], r, c.gamma);
         out[0] = rho;
         out[1] = -(L[1] * r) * rho;
-        out[2] = ((0.5 * q * r - 1.0) * r) * rho;
+        out[2] = (fma(0.5 * q, r, -1.0) * r) * rho;
     } else if constexpr (KIND == UQK_EULER2D) {
-        const double r = recip_f64(L[3]), q = L[1] * L[1] + L[2] * L[2];
+        const double r = recip_f64(L[3]), q = fma(L[1], L[1], L[2] * L[2]);
         const double rho = euler_rho(L[0], q, L[3], r, c.gamma);
         out[0] = rho;
         out[1] = -(L[1] * r) * rho;
         out[2] = -(L[2] * r) * rho;
-        out[3] = ((0.5 * q * r - 1.0) * r) * rho;
+        out[3] = (fma(0.5 * q, r, -1.0) * r) * rho;
     } else if constexpr (KIND == UQK_SHALLOW_WATER2D) {
         // shallowwaterclosure2d.cpp:10-14
-        double c0 = 2.0 * L[0] + L[1] * L[1] + L[2] * L[2];
+        double c0 = fma(L[2], L[2], fma(L[1], L[1], 2.0 * L[0]));
         out[0] = 0.5 * c0 / c.g;
         out[1] = 0.5 * L[1] * c0 / c.g;
-        out[2] = 0.5 * (2.0 * L[0] * L[2] + L[1] * L[1] * L[2] + L[2] * L[2] * L[2]) / c.g;
+        out[2] = 0.5 * fma(L[2] * L[2], L[2], fma(L[1] * L[1], L[2], 2.0 * L[0] * L[2])) / c.g;
     } else {
         // entropy |q|^2/(2h) + g h^2/2 - eps log h: h solves g h - eps/h = c
-        double cc = L[0] + 0.5 * (L[1] * L[1] + L[2] * L[2]);
-        double r = sqrt(cc * cc + 4.0 * c.g * c.barrier);
+        double cc = fma(0.5, fma(L[1], L[1], L[2] * L[2]), L[0]);
+        double r = sqrt(fma(cc, cc, 4.0 * c.g * c.barrier));
         double h = cc > 0.0 ? (cc + r) / (2.0 * c.g) : (2.0 * c.barrier) / (r - cc);
         out[0] = h;
         out[1] = h * L[1];
@@ -226,13 +230,14 @@ struct PointState {
     double vx, vy, p, c;
 };
 template <int S> __device__ __forceinline__ PointState point_state(const ProblemParams& p, const double* u) {
+#pragma clang fp contract(off)
     PointState q{0.0, 0.0, 0.0, 0.0};
     if constexpr (S >= 3) {
         const double ri = recip_any(u[0]);
         q.vx = u[1] * ri;
         q.vy = u[2] * ri;
         if constexpr (S == 4) {
-            q.p = (p.gamma - 1.0) * (u[3] - 0.5 * u[0] * (q.vx * q.vx + q.vy * q.vy));
+            q.p = (p.gamma - 1.0) * fma(-0.5 * u[0], fma(q.vx, q.vx, q.vy * q.vy), u[3]);
             q.c = sqrt_f64(p.gamma * q.p * ri);
         } else {
             q.p = 0.5 * p.g * u[0] * u[0];
