@@ -130,7 +130,7 @@ __device__ __forceinline__ void matrix_settle() {  // before results are read wh
 // blockIdx.z splits K (ATOMIC epilogue only).  The operands are sent for four
 // steps of 32 ahead: a training batch leaves a tenth of the chip's workgroups,
 // each of which otherwise waits for memory once per step (1,024 rows, 256
-// hidden: weight gradient 16.7 us, input gradient 11.5 us).
+// hidden: weight gradient 16.8 -> 12.7 us, input gradient 11.5 -> 11.0 us).
 template <bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(16))) __bf16 As[kTile * kLdsStride];

@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(kSweepThreads) eval_uq_kernel(SweepArgs a) {
 // as one FP64 matrix product (rows: cell slot x state), 16 moments at a time;
 // uQ is read once, a cell's four points of a step together, and two passes'
 // steps are in flight.  It is bound by that read (65,536 cells at 25 points,
-// four states: 27 us; one thread per moment, every uQ read M times through
+// four states: 19 us; one thread per moment, every uQ read M times through
 // L1, 65 us).
 template <int S>
 __global__ void __launch_bounds__(kSweepThreads) reconstruct_kernel(SweepArgs a) {
