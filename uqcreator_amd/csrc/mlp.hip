@@ -62,6 +62,7 @@ struct GemmArgs {
     float* f;                 // LINEAR: y;      ATOMIC: f += acc
     int ldf;
     int k_split;              // K range per blockIdx.z (a multiple of 32)
+    float* db;                // ATOMIC: db[m] += sum over k of A (may be null)
 };
 
 // 2 / d for d >= 1 (an exponential plus one), rounded as the division: v_rcp's
@@ -145,6 +146,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the sums over k of A (the bias gradient): a product with ones, in the
+    // workgroups and wavefronts of the first columns
+    const bool sums = EPI == EPI_ATOMIC && g.db && blockIdx.y == 0 && wc == 0;
+    f32x4 sum[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
     constexpr int PF = 4;
     bf16x8 pa[PF], pb[PF];
 #pragma unroll
@@ -179,10 +187,23 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c)
                     acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
+            if (EPI == EPI_ATOMIC && sums) {
+#pragma unroll
+                for (int r = 0; r < 2; ++r) sum[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], ones, sum[r], 0, 0, 0);
+            }
             __syncthreads();
         }
     }
     matrix_settle();
+    if (EPI == EPI_ATOMIC && sums && (lane & 15) == 0) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + wr + r * 16 + 4 * (lane >> 4) + i;
+                if (m < g.M) atomicAdd(&g.db[m], sum[r][i]);
+            }
+    }
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -334,21 +355,20 @@ __global__ __launch_bounds__(256) void net_kernel(NetArgs a) {
     }
 }
 
-// db[n] += sum over rows of x[row*ld + n] (x FP32 or BF16): a block of 256
+// db[n] += sum over rows of x[row*ld + n]: a block of 256
 // threads covers kColsumRows rows of 256 columns, eight loads in flight per
 // thread, one atomic per column and block.
 constexpr int kColsumRows = 32;
 inline dim3 colsum_grid(long rows, int N) {
     return dim3((unsigned)((rows + kColsumRows - 1) / kColsumRows), (unsigned)((N + 255) / 256));
 }
-template <class T>
-__global__ __launch_bounds__(256) void colsum_kernel(const T* x, int ld, int rows, int N, float* db) {
+__global__ __launch_bounds__(256) void colsum_kernel(const float* x, int ld, int rows, int N, float* db) {
     const int n = blockIdx.y * 256 + threadIdx.x;
     if (n >= N) return;
     const int r0 = blockIdx.x * kColsumRows, r1 = min(rows, r0 + kColsumRows);
     float s = 0.f;
 #pragma unroll 8
-    for (int r = r0; r < r1; ++r) s += (float)x[(size_t)r * ld + n];
+    for (int r = r0; r < r1; ++r) s += x[(size_t)r * ld + n];
     atomicAdd(&db[n], s);
 }
 
@@ -936,13 +956,11 @@ int backward(uqk_mlp* n, long rows, int n_real) {
         a.f = gW;
         a.ldf = K;
         a.k_split = ksplit;
+        // db_l: with the weight gradient; the head's from its FP32 residuals
+        if (l < kLayers - 1) a.db = gb;
         if (int rc = gemm(n, EPI_ATOMIC, true, true, a, splits)) return rc;
         if (l == kLayers - 1)
-            hipLaunchKernelGGL(colsum_kernel<float>, colsum_grid(rows, N), dim3(256), 0, st, n->dyf, n->NO, (int)rows, N,
-                               gb);
-        else
-            hipLaunchKernelGGL(colsum_kernel<__bf16>, colsum_grid(rows, N), dim3(256), 0, st, dcur, ldcur, (int)rows, N,
-                               gb);
+            hipLaunchKernelGGL(colsum_kernel, colsum_grid(rows, N), dim3(256), 0, st, n->dyf, n->NO, (int)rows, N, gb);
         if (l == 0) break;
         // dz_{l-1} = (dz_l W_l) * gelu'(z_{l-1})
         GemmArgs b{};
