@@ -38,9 +38,9 @@ enum {
 /* Arithmetic of the Newton steps. */
 enum {
     UQK_FP64 = 0,   /* everything in FP64, a factorisation per step (the plain path) */
-    UQK_MIXED = 1   /* steps on kept FP32 factorisations (uqk_set_factor_reuse), the
-                       workgroup kernel's Hessian on FP32 MFMA; factorisation,
-                       gradient, residual and accept test in FP64                  */
+    UQK_MIXED = 1   /* steps on kept FP32 inverses (uqk_set_factor_reuse);
+                       Hessian, factorisation, gradient, residual and accept test
+                       in FP64 (the workgroup kernel's Hessian on FP32 MFMA)       */
 };
 
 /* Per-cell closure status (replaces the reference's exit(EXIT_FAILURE)). */
@@ -122,8 +122,8 @@ int uqk_synchronize(uqk_ctx* ctx);
  * else the kernel for large systems (UQK_KERNEL_BLOCK; 64..128 duals: one
  * wavefront per cell below 128, where LDS holds the tables, else a workgroup
  * per cell), else the generic wave-per-cell kernel (any size, per-cell orders, FP64; below 64
- * duals in register tiles, where it outruns the workgroup kernel's mixed
- * precision, which UQK_KERNEL_BLOCK still selects). */
+ * duals in register tiles, where it outruns the mixed precision of the
+ * kernel for large systems, which UQK_KERNEL_BLOCK still selects). */
 enum { UQK_KERNEL_AUTO = 0, UQK_KERNEL_GENERIC = 1, UQK_KERNEL_WAVE = 2, UQK_KERNEL_BLOCK = 3 };
 int uqk_set_closure_kernel(uqk_ctx* ctx, int32_t kernel);
 /* Kernel used by the last closure call (UQK_KERNEL_GENERIC / _WAVE / _BLOCK). */
@@ -252,11 +252,12 @@ int uqk_last_closure_stats(const uqk_ctx* ctx, int64_t* newton_steps, int64_t* g
 /* Reuse of the factorisation in the mixed closure (no counterpart in the
  * reference; on by default for UQK_MIXED contexts).  In the time loop, after
  * a cell's FP64 factorisation of its Hessian in one step, the library keeps
- * P = H^{-1} of the factored matrix: the wave kernel (uniform orders,
- * n < 64) as an explicit inverse (computed in FP64 with the step, kept in
- * FP32), the workgroup kernel (n up to 128, per-cell orders too) as
- * the factor U rounded to FP32 and tagged with the cell's order, replaced
- * by U^{-1} (P = U^{-1} U^{-T}) the first time a later step uses it.  The
+ * P = H^{-1} of the factored matrix as an explicit inverse (computed in
+ * FP64 with the step, kept in FP32): the wave kernel (uniform orders, n < 64)
+ * and the kernel for 64 to 127 duals (per-cell orders too, tagged with the
+ * cell's order); the workgroup kernel keeps the factor U rounded to FP32,
+ * replaced by U^{-1} (P = U^{-1} U^{-T}) the first time a later step uses it.
+ * The
  * cell's Newton steps in later time steps take d = P g refined once with
  * the FP64 Hessian-vector product (d += P (g - H d)) and keep it when the
  * full step lowers ||grad L|| (the FP64 accept test); otherwise, and after
@@ -308,11 +309,12 @@ int uqk_kernel_times(const uqk_ctx* ctx, double* closure_ms, double* advance_ms,
 /* Launch shape of the specialised closure kernels: wavefronts (cells in
  * flight) per workgroup of the one-wavefront kernel (1, 2, 4; 0 = as many as
  * LDS allows) and persistent workgroups per CU of either kernel (0 = every
- * resident slot; the workgroup kernel for n = S*M >= 64 takes only this). */
+ * resident slot; the kernel for large systems, n = S*M >= 64, has one resident
+ * workgroup per CU). */
 int uqk_set_launch_shape(uqk_ctx* ctx, int32_t waves, int32_t blocks_per_cu);
 int uqk_get_launch_shape(const uqk_ctx* ctx, int32_t* waves, int32_t* blocks_per_cu);
 /* Times the specialised closure kernel the context runs (the one-wavefront
- * kernel, or the workgroup kernel for n = S*M >= 64) on n cells (device u and
+ * kernel, or the kernel for large systems, n = S*M >= 64) on n cells (device u and
  * starting lambda; lambda is not modified) for every launch shape the LDS and
  * the occupancy allow, keeps the fastest for ctx, and appends it as one JSON
  * line

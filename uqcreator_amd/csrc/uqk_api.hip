@@ -114,8 +114,9 @@ bool large_fits(const uqk_ctx* ctx) {
 // the per-cell slots (flags cleared) to n cells.  Allocates only outside
 // graph capture.
 // Kept factorisations of the time loop's mixed closure, by the kernel the
-// launch takes: 1 the wave kernel's kept inverses, 2 the workgroup kernel's
-// kept FP32 factors, 0 none.
+// launch takes: 1 the wave kernel's kept inverses, 2 those of the kernels for
+// large systems (below 128 duals inverses in tiles, else the workgroup kernel's
+// kept FP32 factors), 0 none.
 int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
     if (ctx->precision != UQK_MIXED || !ctx->factor_reuse || ctx->c.max_iter == 1) return 0;
     int wm = 0, wo = 0;
@@ -238,7 +239,7 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
     a.took = counters + 4;
     a.nfactor = counters + 5;
     // mixed precision: kept factorisations (per cell in the time loop: the
-    // wave kernel's inverses or the workgroup kernel's FP32 factors; in
+    // wave kernel's inverses or those of the kernel for large systems; in
     // registers for a single closure call);
     // the buffers exist before a graph is captured
     const int fmode = factors_per_cell ? factor_mode(ctx, nt != nullptr) : 0;
@@ -1123,7 +1124,7 @@ int uqk_get_launch_shape(const uqk_ctx* ctx, int32_t* waves, int32_t* blocks_per
 int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda, const char* json_path) {
     if (!ctx || n <= 0 || !u || !lambda) return -1;
     // the kernel the context runs: the one-wavefront kernel where it fits,
-    // else the workgroup kernel (n = S*M >= 64), whose only launch parameter
+    // else the kernel for large systems (n = S*M >= 64), whose launch parameter
     // is the number of persistent workgroups per CU (one wave count: 4)
     int wmax = 0, occ = 0;
     const bool wave = ctx->kernel != UQK_KERNEL_BLOCK &&
