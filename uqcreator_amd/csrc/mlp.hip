@@ -370,21 +370,30 @@ __global__ __launch_bounds__(256) void net_kernel(NetArgs a) {
     }
 }
 
-// db[n] += sum over rows of x[row*ld + n]: a block of 256
-// threads covers kColsumRows rows of 256 columns, eight loads in flight per
-// thread, one atomic per column and block.
-constexpr int kColsumRows = 32;
+// db[n] += sum over rows of x[row*ld + n]: 16 wavefronts of a workgroup take 64
+// rows each of 64 columns, their sums are added in order, and one atomic per
+// column and 1,024 rows follows (a training batch of that size then gives the
+// same bits in every run).
+constexpr int kColsumRows = 1024;
 inline dim3 colsum_grid(long rows, int N) {
-    return dim3((unsigned)((rows + kColsumRows - 1) / kColsumRows), (unsigned)((N + 255) / 256));
+    return dim3((unsigned)((rows + kColsumRows - 1) / kColsumRows), (unsigned)((N + 63) / 64));
 }
-__global__ __launch_bounds__(256) void colsum_kernel(const float* x, int ld, int rows, int N, float* db) {
-    const int n = blockIdx.y * 256 + threadIdx.x;
-    if (n >= N) return;
-    const int r0 = blockIdx.x * kColsumRows, r1 = min(rows, r0 + kColsumRows);
+__global__ __launch_bounds__(1024) void colsum_kernel(const float* x, int ld, int rows, int N, float* db) {
+    __shared__ float part[16][64];
+    const int c = threadIdx.x & 63, g = threadIdx.x >> 6, n = blockIdx.y * 64 + c;
+    const int r0 = blockIdx.x * kColsumRows + 64 * g, r1 = min(rows, r0 + 64);
     float s = 0.f;
-#pragma unroll 8
-    for (int r = r0; r < r1; ++r) s += x[(size_t)r * ld + n];
-    atomicAdd(&db[n], s);
+    if (n < N) {
+#pragma unroll 16
+        for (int r = r0; r < r1; ++r) s += x[(size_t)r * ld + n];
+    }
+    part[g][c] = s;
+    __syncthreads();
+    if (g == 0 && n < N) {
+#pragma unroll
+        for (int k = 1; k < 16; ++k) s += part[k][c];
+        atomicAdd(&db[n], s);
+    }
 }
 
 // dy = 2 (y - t) / (rows * n_real) for the first n_real outputs, 0 beyond;
@@ -975,7 +984,7 @@ int backward(uqk_mlp* n, long rows, int n_real) {
         if (l < kLayers - 1) a.db = gb;
         if (int rc = gemm(n, EPI_ATOMIC, true, true, a, splits)) return rc;
         if (l == kLayers - 1)
-            hipLaunchKernelGGL(colsum_kernel, colsum_grid(rows, N), dim3(256), 0, st, n->dyf, n->NO, (int)rows, N, gb);
+            hipLaunchKernelGGL(colsum_kernel, colsum_grid(rows, N), dim3(1024), 0, st, n->dyf, n->NO, (int)rows, N, gb);
         if (l == 0) break;
         // dz_{l-1} = (dz_l W_l) * gelu'(z_{l-1})
         GemmArgs b{};
