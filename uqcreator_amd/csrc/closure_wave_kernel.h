@@ -209,7 +209,8 @@ __device__ __attribute__((noinline)) bool sweep_step(ClosureParams c, double L0,
     }
     wave_sync();
     if (spd && Pg) {
-        // (r, c) of the lower tiles to both of its places
+        // (r, c) of the lower tiles to both of its places, and zero to the
+        // places past N that fill a row's runs (later steps read whole runs)
 #pragma unroll
         for (int r = 0; r < NT; ++r)
 #pragma unroll
@@ -217,11 +218,9 @@ __device__ __attribute__((noinline)) bool sweep_step(ClosureParams c, double L0,
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int R = 16 * r + p16, C = 16 * cc + 4 * e + q4;
-                    const float v = -(float)T[tile_lower(cc, r)][e];
-                    if (R < N && C < N) {
-                        Pg[(R * 4 + q4) * NQ + 4 * cc + e] = v;
-                        if (cc < r) Pg[(C * 4 + (p16 & 3)) * NQ + 4 * r + (p16 >> 2)] = v;
-                    }
+                    const float v = R < N && C < N ? -(float)T[tile_lower(cc, r)][e] : 0.f;
+                    if (R < N && C < 4 * NQ) Pg[(R * 4 + q4) * NQ + 4 * cc + e] = v;
+                    if (cc < r && C < N && R < 4 * NQ) Pg[(C * 4 + (p16 & 3)) * NQ + 4 * r + (p16 >> 2)] = v;
                 }
     }
     return spd;
