@@ -1,5 +1,5 @@
 // tile_solve.h -- factorisation, solve and inversion of a symmetric positive
-// definite system of n < 64 unknowns by one wavefront, entirely in registers.
+// definite system by one wavefront, entirely in registers.
 //
 // The matrix lies in 16 x 16 tiles in the accumulator layout of
 // v_mfma_f64_16x16x4f64: element e (0..3) of lane 16 q + p of tile (tc, tr)
@@ -8,11 +8,10 @@
 // 4 b + q of row p), and this register is, as it stands, the A operand (rows
 // p, k = q) and the B operand (k = q, columns p) of a rank-4 update.  So four
 // pivots are eliminated per step without moving the panel:
-//   B   = the 4 x 4 pivot block, inverted by every lane from v_readlane'd
-//         scalars (two 2 x 2 blocks, so two reciprocals are in sequence, not
-//         four);
-//   W   = P B^-1, one v_mfma_f64_4x4x4_4b per 16 rows of the panel P;
-//   H  -= P W^T on the tiles that are left, one v_mfma_f64_16x16x4 each.
+//   B   = L D L^T, the 4 x 4 pivot block, factored by every lane from
+//         v_readlane'd scalars (three reciprocals in sequence);
+//   V   = P L^-T, one v_mfma_f64_4x4x4_4b per 16 rows of the panel P;
+//   H  -= V D^-1 V^T on the tiles that are left, one v_mfma_f64_16x16x4 each.
 // There is no LDS round trip and no lane mask per entry.
 #pragma once
 
@@ -170,11 +169,20 @@ __device__ __forceinline__ void static_for(F f) {
 // tile (tc, tr), tc <= tr, of the lower triangle
 __host__ __device__ constexpr int tile_lower(int tc, int tr) { return tr * (tr + 1) / 2 + tc; }
 
-// B^-1 of the 4 x 4 pivot block at row/column j0 (0, 4, 8, 12) of a diagonal
-// tile whose panel register is pv; lane 16 q + p gets B^-1(p % 4, q).  Of
-// the four pivots only `have` are real, the others read as identity.  False
-// if a leading minor is not positive.
-__device__ __forceinline__ bool pivot_inverse(double pv, int j0, int have, int p, int q, double& bv) {
+// The 4 x 4 pivot block B = L D L^T at row/column j0 (0, 4, 8, 12) of a
+// diagonal tile whose panel register is pv, formed by every lane from
+// v_readlane'd scalars: lane 16 q + p gets li = L^-1(p % 4, q), lt = L^-1(q, p
+// % 4) and di = 1/D(q).  Of the four pivots only `have` are real, the others
+// read as identity.  False if a pivot is not positive.
+// The factors and not B^-1, because the update with V = P L^-T, H -= V D^-1
+// V^T, stands as much ill-conditioning as the Cholesky factorisation does;
+// with H -= P B^-1 P^T the Newton iteration met pivots that rounding had made
+// negative in 23 of 40 Euler closures that Cholesky solves (n = 40, a start of
+// a far too small density).  No product of two pivots either: it underflows
+// where the density does.  Both cost nothing: 65,536 cells of n = 40, 40 time
+// steps in FP64, 20.1 ms against 20.5 with the inverse from two 2 x 2 blocks.
+__device__ __forceinline__ bool pivot_factors(double pv, int j0, int have, int p, int q, double& li, double& lt,
+                                              double& di) {
     double b00 = lane_get(pv, j0), b10 = lane_get(pv, j0 + 1), b20 = lane_get(pv, j0 + 2), b30 = lane_get(pv, j0 + 3);
     double b11 = lane_get(pv, 16 + j0 + 1), b21 = lane_get(pv, 16 + j0 + 2), b31 = lane_get(pv, 16 + j0 + 3);
     double b22 = lane_get(pv, 32 + j0 + 2), b32 = lane_get(pv, 32 + j0 + 3), b33 = lane_get(pv, 48 + j0 + 3);
@@ -183,43 +191,32 @@ __device__ __forceinline__ bool pivot_inverse(double pv, int j0, int have, int p
         if (have < 3) b22 = 1.0, b20 = b21 = 0.0;
         if (have < 2) b11 = 1.0, b10 = 0.0;
     }
-    // E = [b00 b10; b10 b11] = L D L^T; 1/d1 = b00 / det, so that both
-    // reciprocals start at once
-    const double det = fma(b00, b11, -b10 * b10);
-    const double r0 = recip_f64(b00), e11 = b00 * recip_f64(det), l = b10 * r0;
-    const double e01 = -l * e11, e00 = fma(-l, e01, r0);
-    // X = E^-1 F, F = [b20 b30; b21 b31]; S = G - F^T X
-    const double x00 = fma(e00, b20, e01 * b21), x10 = fma(e01, b20, e11 * b21);
-    const double x01 = fma(e00, b30, e01 * b31), x11 = fma(e01, b30, e11 * b31);
-    const double s00 = fma(-b20, x00, fma(-b21, x10, b22));
-    const double s10 = fma(-b20, x01, fma(-b21, x11, b32));
-    const double s11 = fma(-b30, x01, fma(-b31, x11, b33));
-    const double dets = fma(s00, s11, -s10 * s10);
-    const double t0 = recip_f64(s00), i33 = s00 * recip_f64(dets), m = s10 * t0;
-    const double i23 = -m * i33, i22 = fma(-m, i23, t0);
-    // Y = X S^-1
-    const double y00 = fma(x00, i22, x01 * i23), y01 = fma(x00, i23, x01 * i33);
-    const double y10 = fma(x10, i22, x11 * i23), y11 = fma(x10, i23, x11 * i33);
-    const double i00 = fma(y00, x00, fma(y01, x01, e00)), i01 = fma(y00, x10, fma(y01, x11, e01));
-    const double i11 = fma(y10, x10, fma(y11, x11, e11));
-    const int pm = p & 3;
-    // row pm of the symmetric inverse: columns q
-    const bool p1 = pm & 1, p2 = pm & 2, q1 = q & 1, q2 = q & 2;
-    const double c0 = q1 ? (p1 ? i11 : i01) : (p1 ? i01 : i00);      // p, q < 2
-    const double c2 = q1 ? (p1 ? i33 : i23) : (p1 ? i23 : i22);      // p, q >= 2
-    // -Y(a, b): row a < 2 and column 2 + b
-    const bool a1 = p2 ? q1 : p1, d1 = p2 ? p1 : q1;
-    const double c1 = -(d1 ? (a1 ? y11 : y01) : (a1 ? y10 : y00));
-    bv = p2 == q2 ? (p2 ? c2 : c0) : c1;
-    return b00 > 0.0 && det > 0.0 && s00 > 0.0 && dets > 0.0;
+    const double r0 = recip_f64(b00), l10 = b10 * r0, l20 = b20 * r0, l30 = b30 * r0;
+    const double d1 = fma(-l10, b10, b11), c21 = fma(-l20, b10, b21), c31 = fma(-l30, b10, b31);
+    const double r1 = recip_f64(d1), l21 = c21 * r1, l31 = c31 * r1;
+    const double d2 = fma(-l21, c21, fma(-l20, b20, b22)), c32 = fma(-l31, c21, fma(-l30, b20, b32));
+    const double r2 = recip_f64(d2), l32 = c32 * r2;
+    const double d3 = fma(-l32, c32, fma(-l31, c31, fma(-l30, b30, b33)));
+    const double r3 = recip_f64(d3);
+    // L^-1: i10 = -l10, i21 = -l21, i32 = -l32
+    const double i20 = fma(l21, l10, -l20), i31 = fma(l32, l21, -l31);
+    const double i30 = fma(-l32, i20, fma(l31, l10, -l30));
+    const bool p1 = p & 1, p2 = p & 2, q1 = q & 1, q2 = q & 2;
+    const double c0 = p2 ? (p1 ? i30 : i20) : (p1 ? -l10 : 1.0);
+    const double c1 = p2 ? (p1 ? i31 : -l21) : (p1 ? 1.0 : 0.0);
+    const double c2 = p2 ? (p1 ? -l32 : 1.0) : 0.0, c3 = p1 && p2 ? 1.0 : 0.0;
+    li = q2 ? (q1 ? c3 : c2) : (q1 ? c1 : c0);
+    lt = __builtin_amdgcn_mfma_f64_4x4x4f64(li, (p & 3) == q ? 1.0 : 0.0, 0.0, 0, 0, 0);  // (transposed)
+    di = q2 ? (q1 ? r3 : r2) : (q1 ? r1 : r0);
+    return b00 > 0.0 && d1 > 0.0 && d2 > 0.0 && d3 > 0.0;
 }
 
 // In place on the lower tiles of [H; g^T] (n pivots; row n holds the right
-// hand side): column block b becomes W = V^T, the block-unit upper factor of
-// H = V^T B V (B the 4 x 4 pivot blocks).  The first NT tile rows hold n + 1
-// rows; there is no branch between the matrix instructions of a step, whose
-// tiles past the last pivot are updated for nothing where n is not a constant
-// (settle).
+// hand side): column block b becomes V D^-1, that of the unit lower factor of
+// H = L D L^T, and the block's own rows its L^-1, transposed.  The first NT
+// tile rows hold n + 1 rows; there is no branch between the matrix
+// instructions of a step, whose tiles past the last pivot are updated for
+// nothing where n is not a constant (settle).
 template <int NT, int TILES>
 __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[TILES], int n, int p, int q) {
     bool ok = true;
@@ -227,16 +224,17 @@ __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[TILES], int n, int p, int q)
     for (int b = 0; b < 4 * NT; ++b) {
         if (4 * b >= n) break;
         const int jb = b >> 2, e = b & 3, j0 = 4 * e, have = n - 4 * b;
-        double bv;
-        ok &= pivot_inverse(T[tile_lower(jb, jb)][e], j0, have, p, q, bv);
-        double P[NT], W[NT];
+        double li, lt, di;
+        ok &= pivot_factors(T[tile_lower(jb, jb)][e], j0, have, p, q, li, lt, di);
+        double V[NT], W[NT];
 #pragma unroll
         for (int r = jb; r < NT; ++r) {
-            P[r] = T[tile_lower(jb, r)][e];
-            if (r == jb && !(p >= j0 + (have < 4 ? have : 4))) P[r] = 0.0;  // finished rows
-            if (have < 4 && q >= have) P[r] = 0.0;       // columns that are no pivots
-            W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(bv, P[r], 0.0, 0, 0, 0);
-            T[tile_lower(jb, r)][e] = W[r];
+            double P = T[tile_lower(jb, r)][e];
+            if (r == jb && !(p >= j0 + (have < 4 ? have : 4))) P = 0.0;  // finished rows
+            if (have < 4 && q >= have) P = 0.0;                          // columns that are no pivots
+            V[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(li, P, 0.0, 0, 0, 0);
+            W[r] = V[r] * di;
+            T[tile_lower(jb, r)][e] = r == jb && (p >> 2) == e && (p & 3) < have ? lt : W[r];
         }
         if (!__builtin_constant_p(n) || 4 * b + 4 < n) {
 #pragma unroll
@@ -245,22 +243,21 @@ __device__ __forceinline__ bool tile_ldl(f64x4 (&T)[TILES], int n, int p, int q)
                 for (int c = jb; c <= r; ++c)
                     if (!__builtin_constant_p(n) || 16 * c < n)
                         T[tile_lower(c, r)] =
-                            __builtin_amdgcn_mfma_f64_16x16x4f64(P[c], -W[r], T[tile_lower(c, r)], 0, 0, 0);
+                            __builtin_amdgcn_mfma_f64_16x16x4f64(V[c], -W[r], T[tile_lower(c, r)], 0, 0, 0);
         }
     }
     if (!__builtin_constant_p(n)) settle<18>();
     return ok;
 }
 
-// The solution from the factor that tile_ldl left: x_{4b+k} = W(n, k) -
-// sum_{r > 4b+3} W(r, k) x_r, four unknowns per step, the sum over the rows
-// of a lane group by DPP.  X[r] of lane 16 q + p is x_{16 r + p} (-1 at n,
-// zero past it).
+// The solution from the factor that tile_ldl left, four unknowns per step:
+// y_k = (V D^-1)(n, k) - sum_{r > 4b+3} (V D^-1)(r, k) x_r, the sum over the
+// rows of a lane group by DPP, and x = L^-T y of the block over the lane
+// groups.  X[r] of lane 16 q + p is x_{16 r + p} (-1 at n, zero past it).
 template <int NT, int TILES>
 __device__ __forceinline__ void tile_back_rows(const f64x4 (&T)[TILES], int n, int p, int q, double (&X)[NT]) {
 #pragma unroll
     for (int r = 0; r < NT; ++r) X[r] = 16 * r + p == n ? -1.0 : 0.0;
-    const bool p1 = p & 1, p2 = p & 2;
 #pragma unroll
     for (int b = 4 * NT - 1; b >= 0; --b) {
         if (4 * b >= n) continue;
@@ -269,10 +266,8 @@ __device__ __forceinline__ void tile_back_rows(const f64x4 (&T)[TILES], int n, i
 #pragma unroll
         for (int r = jb; r < NT; ++r)
             s = fma(-T[tile_lower(jb, r)][e], X[r], s);
-        s = row_sum(s);
-        const double x0 = lane_get(s, 0), x1 = lane_get(s, 16), x2 = lane_get(s, 32), x3 = lane_get(s, 48);
-        const double v = p2 ? (p1 ? x3 : x2) : (p1 ? x1 : x0);
-        if ((p >> 2) == e && (p & 3) < have) X[jb] = v;
+        const double x = group_sum(T[tile_lower(jb, jb)][e] * row_sum(s));
+        if ((p >> 2) == e && (p & 3) < have) X[jb] = x;
     }
 }
 
@@ -297,18 +292,19 @@ __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, in
     for (int b = 0; b < 4 * NT; ++b) {
         if (4 * b >= n) break;
         const int jb = b >> 2, e = b & 3, have = n - 4 * b;
-        double bv;
-        ok &= pivot_inverse(T[jb * NT + jb][e], 4 * e, have, p, q, bv);
+        double li, lt, di;
+        ok &= pivot_factors(T[jb * NT + jb][e], 4 * e, have, p, q, li, lt, di);
         const bool in = (p >> 2) == e && (p & 3) < have;  // this lane's row of tile row jb is a pivot
-        double P[NT], W[NT], R[NT];
+        double V[NT], U[NT], W[NT];
 #pragma unroll
         for (int r = 0; r < NT; ++r) {
-            P[r] = T[r * NT + jb][e];
-            if (r == jb && in) P[r] = 0.0;
-            if (have < 4 && q >= have) P[r] = 0.0;
-            W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(bv, P[r], 0.0, 0, 0, 0);
-            // pivot rows: H(c, pivot) <- W(c, .) = sum_k P(c, k) B^-1(k, .)
-            R[r] = r == jb && in ? bv : -W[r];
+            double P = T[r * NT + jb][e];
+            if (r == jb && in) P = 0.0;
+            if (have < 4 && q >= have) P = 0.0;
+            V[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(li, P, 0.0, 0, 0, 0);
+            // pivot rows: H(c, pivot) <- V D^-1 L^-1 = P B^-1, and -B^-1 in the block itself
+            U[r] = (r == jb && in ? -lt : V[r]) * di;
+            W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(lt, U[r], 0.0, 0, 0, 0);
         }
         if (in) {
 #pragma unroll
@@ -319,12 +315,8 @@ __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, in
 #pragma unroll
             for (int c = 0; c < NT; ++c) {
                 const double old = T[r * NT + c][e];
-                T[r * NT + c] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[c], R[r], T[r * NT + c], 0, 0, 0);
-                if (c == jb) {
-                    // the pivot columns: W, and -B^-1 in the block itself
-                    const double w = r == jb && in ? -bv : W[r];
-                    T[r * NT + c][e] = have < 4 && q >= have ? old : w;
-                }
+                T[r * NT + c] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[c], -U[r], T[r * NT + c], 0, 0, 0);
+                if (c == jb) T[r * NT + c][e] = have < 4 && q >= have ? old : W[r];  // the pivot columns
             }
     }
     return ok;
@@ -341,7 +333,7 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p
     for (int b = 0; b < 4 * NT; ++b) {
         if (4 * b >= n) break;
         const int jb = b >> 2, e = b & 3, have = n - 4 * b;
-        double bv;
+        double li, lt, di;
         const bool at = (p >> 2) == e;
         if (jb > 0) {
             wave_sync();
@@ -353,14 +345,15 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p
             }
             wave_sync();
         }
-        ok &= pivot_inverse(T[tile_lower(jb, jb)][e], 4 * e, have, p, q, bv);
+        ok &= pivot_factors(T[tile_lower(jb, jb)][e], 4 * e, have, p, q, li, lt, di);
         const bool in = at && (p & 3) < have;  // this lane's row of tile row jb is a pivot
-        double P[NT], W[NT];
+        double V[NT];
 #pragma unroll
         for (int r = 0; r < NT; ++r) {
-            P[r] = r < jb ? scr[64 * r + 16 * q + p] : T[tile_lower(jb, r < jb ? jb : r)][e];
-            if (r == jb && in) P[r] = 0.0;
-            if (have < 4 && q >= have) P[r] = 0.0;
+            double P = r < jb ? scr[64 * r + 16 * q + p] : T[tile_lower(jb, r < jb ? jb : r)][e];
+            if (r == jb && in) P = 0.0;
+            if (have < 4 && q >= have) P = 0.0;
+            V[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(li, P, 0.0, 0, 0, 0);
         }
         if (in) {
 #pragma unroll
@@ -368,16 +361,13 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p
         }
 #pragma unroll
         for (int r = 0; r < NT; ++r) {
-            W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(bv, P[r], 0.0, 0, 0, 0);
-            const double R = r == jb && in ? bv : -W[r];
+            const double U = (r == jb && in ? -lt : V[r]) * di;
+            const double W = __builtin_amdgcn_mfma_f64_4x4x4f64(lt, U, 0.0, 0, 0, 0);
 #pragma unroll
             for (int c = 0; c <= r; ++c) {
                 const double old = T[tile_lower(c, r)][e];
-                T[tile_lower(c, r)] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[c], R, T[tile_lower(c, r)], 0, 0, 0);
-                if (c == jb) {
-                    const double w = r == jb && in ? -bv : W[r];
-                    T[tile_lower(c, r)][e] = have < 4 && q >= have ? old : w;
-                }
+                T[tile_lower(c, r)] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[c], -U, T[tile_lower(c, r)], 0, 0, 0);
+                if (c == jb) T[tile_lower(c, r)][e] = have < 4 && q >= have ? old : W;
             }
         }
     }
