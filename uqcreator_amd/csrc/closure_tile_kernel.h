@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
                 if (k < QP) {
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
-                        Ub[s * QP + k] = U[s];
+                        Ub[s * QP + k] = k < Q ? U[s] : 0.0;  // (an infinity times the table's zero is NaN)
                         DUb[s * QP + k] = t4[s];
                     }
                 }

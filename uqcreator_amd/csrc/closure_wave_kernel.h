@@ -294,6 +294,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     double* Ub = wb + W::UB;
     double* yb = wb + W::YB;
     double* bh = wb + W::BH;
+    // the places past Q stay zero: an infinite U would give NaN there, against
+    // the table's zero, and the line search has to see the infinity
+    for (int t = lane; t < S * (QP - Q); t += 64) Ub[t % S * QP + Q + t / S] = 0.0;
 
     // this lane's dual (s, i) = (q4, p16): its place in a cell's arrays and
     // its unknown in the system
@@ -433,7 +436,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             double L[S], Uv[S];
             point_lambda(X, L);
             closure_U<KIND>(c, L, Uv);
-            if (lane < QP) {
+            if (lane < Q) {
 #pragma unroll
                 for (int s = 0; s < S; ++s) Ub[s * QP + lane] = Uv[s];
             }
@@ -533,7 +536,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
             double y[P];
             closure_DU<KIND>(c, Lk, rk, y);
             wave_sync();
-            if (lane < QP) {
+            if (lane < Q) {
 #pragma unroll
                 for (int l = 0; l < S; ++l) {
                     double w = 0.0;

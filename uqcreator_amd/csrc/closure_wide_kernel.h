@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                 if (k < QP) {
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
-                        Ub[s * QP + k] = U[s];
+                        Ub[s * QP + k] = k < Q ? U[s] : 0.0;  // (an infinity times the table's zero is NaN)
                         DUb[s * QP + k] = L[s];
                     }
                 }
@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
                                 for (int m = 0; m < S; ++m)
                                     w += y[l >= m ? l * (l + 1) / 2 + m : m * (m + 1) / 2 + l] * L[m];
-                                Ub[l * QP + k] = w;
+                                Ub[l * QP + k] = k < Q ? w : 0.0;
                             }
                         }
                     });
