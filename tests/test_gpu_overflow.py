@@ -73,3 +73,23 @@ def test_overflow_at_the_last_point_halves_the_step(oracle, kind, d, degrees, q1
         g = oracle.gradient(c, b.phi, b.phiw, lam[j], u[j])
         # the kernel's ||grad L|| < 1e-10 to the rounding of its Q-term sums
         assert np.linalg.norm(g) < 1e-10 + 1e-13 * np.abs(u[j]).max(), j
+
+
+@pytest.mark.parametrize("kind", [native.EULER1D, native.EULER2D])
+def test_density_of_an_infinite_exponent(oracle, kind):
+    """|v|^2 past the largest double: the density is infinite, as the
+    reference's exponential gives it, not NaN."""
+    b = native.Basis(1, [0], 1)
+    S = native.STATES[kind]
+    c = oracle.closure(oracle.EULER1D if kind == native.EULER1D else oracle.EULER2D)
+    lam = np.full((8, 1, S), 0.5)
+    lam[:, 0, -1] = -1.0
+    lam[:, 0, 1] = [1e150, 1e153, 1.4e154, 1e155, 1e160, -1e170, 1e200, -1e300]
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = oracle.mean_var(c, b.phi, b.phiw, lam)[:, :S]
+    print("case: infinite exponent kind", kind, want.tolist(), flush=True)
+    assert np.isinf(want).all()
+    cl = native.GpuClosure(kind, b)
+    mv = native.DeviceArray((8, 2 * S))
+    cl.mean_var(native.DeviceArray.from_host(lam), mv)
+    np.testing.assert_array_equal(mv.download()[:, :S], want)

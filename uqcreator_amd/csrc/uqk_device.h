@@ -79,7 +79,8 @@ __device__ __forceinline__ double euler_rho(double v0, double q, double w, doubl
 #pragma clang fp contract(off)
     const double x = fma(-0.5 * q, r, (v0 - log(-w)) - gm), g1 = gm - 1.0, k = recip_f64(g1);
     const double e = x * k;
-    return exp(fma(fma(-e, g1, x), k, e));  // (the quotient corrected once: exp magnifies its error)
+    // (the quotient corrected once: exp magnifies its error; an infinite one stays)
+    return exp(__builtin_isfinite(e) ? fma(fma(-e, g1, x), k, e) : e);
 }
 
 // Vector form of U (the one Closure::Gradient uses).
