@@ -14,8 +14,16 @@ hipError_t newton_wide_shallow(const NewtonArgs& a, int max_lds, int num_cu, hip
 hipError_t newton_wide_shallow_barrier(const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
                                        const LaunchShape& shape);
 
-bool newton_wide_fits(int S, int M, int Q, int max_lds) {
-    return S * M <= wide_limit(S) && wide_waves(S, M, Q, max_lds) > 0;
+// The kernel is taken where it is the faster one (8,192 cells, one closure in
+// FP64, against the workgroup kernel as it is resident): with four wavefronts
+// in LDS beside the tables 0.23..0.34 of its time, with three 0.25..0.46, with
+// two 0.38..0.71; with one, which leaves three SIMDs idle, 1.00..1.42 where two
+// workgroups are resident (n = 105: 9.8 ms against 7.9 at 216 points), and
+// 0.77..0.84 where one is (n = 112, 124).
+bool newton_wide_takes(int S, int M, int Q, int max_lds) {
+    const int waves = S * M <= wide_limit(S) ? wide_waves(S, M, Q, max_lds) : 0;
+    if (waves != 1) return waves > 1;
+    return !newton_block_fits(S, M, Q, max_lds) || 2 * newton_block_lds(S, M, Q) > (size_t)max_lds;
 }
 
 long newton_wide_kept_floats(int S, int M) {

@@ -102,12 +102,12 @@ int check_mesh(uqk_ctx* ctx, const uqk_mesh* m) {
 }
 
 // Whether a kernel for large systems takes the shape (UQK_KERNEL_BLOCK): one
-// wavefront per cell below 128 duals, else a workgroup per cell.
-bool wide_fits(const uqk_ctx* ctx) {
-    return uqk::newton_wide_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+// wavefront per cell where newton_wide_takes says so, else a workgroup per cell.
+bool wide_takes(const uqk_ctx* ctx) {
+    return uqk::newton_wide_takes(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
 }
 bool large_fits(const uqk_ctx* ctx) {
-    return wide_fits(ctx) || uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+    return wide_takes(ctx) || uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
 }
 
 // Kept inverse factors of the mixed wave kernel across time steps: grows
@@ -136,7 +136,7 @@ int ensure_factor_buffers(uqk_ctx* ctx, long n_cells, int mode) {
     const long n = (long)ctx->S * ctx->M;
     // mode 1: the FP32 inverse; mode 2: the same in tiles, or the FP32 factor (packed U)
     const long nn = mode == 1 ? uqk::newton_wave_kept_floats(ctx->S, ctx->M)
-                    : wide_fits(ctx) ? uqk::newton_wide_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
+                    : wide_takes(ctx) ? uqk::newton_wide_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
     if (ctx->pinv_cell_cap >= n_cells && ctx->factor_mode == mode) return 0;
     if (ctx->capturing) return fail(ctx, -1, "kept factors: buffers must exist before graph capture");
     hipFree(ctx->pinv_cell);
@@ -352,7 +352,7 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
             a.grad_at_lam = ctx->check_grad;
             a.dt_cell = ca.dt_cell;
         }
-        UQK_HIP(ctx, (wide_fits(ctx) ? uqk::newton_wide_launch : uqk::newton_block_launch)(
+        UQK_HIP(ctx, (wide_takes(ctx) ? uqk::newton_wide_launch : uqk::newton_block_launch)(
                          ctx->kind, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream, ctx->shape));
         if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev1, ctx->stream));
         ctx->step_recon = a.dt_cell != nullptr;
@@ -1148,7 +1148,7 @@ int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda,
         if (wave)
             uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, waves, &wm, &oc);
         else
-            oc = wide_fits(ctx) ? 1 : uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
+            oc = wide_takes(ctx) ? 1 : uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
         for (int per_cu = 1; per_cu <= oc && rc == 0; ++per_cu) {
             ctx->shape.waves = waves;
             ctx->shape.blocks_per_cu = per_cu;

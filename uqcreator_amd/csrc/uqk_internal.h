@@ -149,9 +149,10 @@ bool newton_wave_limits(int kind, int M, int Q, int prec, int max_lds, int waves
 // orders (closure_tile_kernel.h)
 bool newton_tile_fits(int S, int M, int Q, int max_lds);
 hipError_t newton_tile_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st);
-// one-wavefront kernel for n = S*M < 128 with one wavefront per SIMD, per-cell
-// orders, FP64 or mixed with kept inverses (closure_wide_kernel.h)
-bool newton_wide_fits(int S, int M, int Q, int max_lds);
+// one-wavefront kernel for n = S*M < 128 (fewer than four states: < 112) with
+// one wavefront per SIMD, per-cell orders, FP64 or mixed with kept inverses
+// (closure_wide_kernel.h); whether it takes the shape
+bool newton_wide_takes(int S, int M, int Q, int max_lds);
 // floats of a cell's kept inverse
 long newton_wide_kept_floats(int S, int M);
 hipError_t newton_wide_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
@@ -159,6 +160,7 @@ hipError_t newton_wide_launch(int kind, const NewtonArgs& a, int max_lds, int nu
 int newton_fp64_wave_doubles(int S, int M, int Q);
 // workgroup-per-cell kernel for n = S*M up to 128 (closure_block.hip)
 bool newton_block_fits(int S, int M, int Q, int max_lds);
+size_t newton_block_lds(int S, int M, int Q);  // bytes of a workgroup
 // shape.blocks_per_cu > 0 caps the persistent workgroups per CU
 hipError_t newton_block_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
                                const LaunchShape& shape = LaunchShape());
