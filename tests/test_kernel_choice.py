@@ -2,17 +2,20 @@
 that a workgroup needs, asked of the library itself."""
 import ctypes
 
+import numpy as np
 import pytest
 
-from uqcreator_amd import native
+from uqcreator_amd import mesh as meshes
+from uqcreator_amd import native, solver, workloads
 
-LDS = 160 * 1024
+LDS, CUS = 160 * 1024, 256
 
 
-def _wide_takes(S, M, Q):
-    f = getattr(native.lib(), "_ZN3uqk17newton_wide_takesEiiii")  # uqk::newton_wide_takes(int, int, int, int)
+def _wide_takes(S, M, Q, cells=100000):
+    # uqk::newton_wide_takes(int, int, int, int, int, long)
+    f = getattr(native.lib(), "_ZN3uqk17newton_wide_takesEiiiiil")
     f.restype = ctypes.c_bool
-    return f(S, M, Q, LDS)
+    return f(S, M, Q, LDS, CUS, ctypes.c_long(cells))
 
 
 @pytest.mark.parametrize("S,M,Q,takes", [
@@ -26,3 +29,38 @@ def _wide_takes(S, M, Q):
 ])
 def test_wide_kernel(S, M, Q, takes):
     assert _wide_takes(S, M, Q) == takes
+
+
+@pytest.mark.parametrize("S,M,Q,cells,takes", [
+    (1, 64, 66, 1, False), (1, 64, 66, 512, False), (1, 64, 66, 513, True),  # two workgroups resident
+    (1, 76, 78, 512, False), (1, 76, 78, 513, True), (4, 16, 40, 1, True), (3, 35, 125, 1, True),
+])
+def test_wide_kernel_for_few_cells(S, M, Q, cells, takes):
+    assert _wide_takes(S, M, Q, cells) == takes
+
+
+@pytest.mark.gpu
+def test_slots_follow_the_number_of_cells():
+    """One context that runs many cells, few and many again: what the kernel of
+    one size keeps of a cell's factorisation is not read by that of the other."""
+    b = native.Basis(1, [63], 66)
+    prob = native.problem(native.BURGERS, flux=native.FLUX_LAX_FRIEDRICHS, cfl=0.5)
+    kw = dict(u_minus=2.9, u_plus=12.1, epsilon=1e-6, precision=native.MIXED)
+
+    def run(cl, cells):
+        print("case: 64 duals, one state,", cells, "cells", flush=True)
+        m = meshes.mesh1d(cells, 0.0, 3.0)
+        u = workloads.project_ic(workloads.burgers_step_ic(), m.center, b)
+        u[:, 1:] *= 0.1
+        s = solver.GpuMomentSolver(cl, prob, m)
+        s.set_state(u, np.zeros_like(u))
+        s.run_device(1e3, max_steps=6)
+        assert (s.status.download() == 0).all()
+        return s.u.download(), s.lam.download(), s.newton_steps, cl.last_closure_factorizations()
+
+    one = native.GpuClosure(native.BOUNDED_BARRIER, b, **kw)
+    for cells in (700, 300, 700):
+        got, want = run(one, cells), run(native.GpuClosure(native.BOUNDED_BARRIER, b, **kw), cells)
+        assert got[2:] == want[2:] and got[3][1] > 0
+        np.testing.assert_array_equal(got[0], want[0])
+        np.testing.assert_array_equal(got[1], want[1])

@@ -19,11 +19,17 @@ hipError_t newton_wide_shallow_barrier(const NewtonArgs& a, int max_lds, int num
 // in LDS beside the tables 0.23..0.34 of its time, with three 0.25..0.46, with
 // two 0.38..0.71; with one, which leaves three SIMDs idle, 1.00..1.42 where two
 // workgroups are resident (n = 105: 9.8 ms against 7.9 at 216 points), and
-// 0.77..0.84 where one is (n = 112, 124).
-bool newton_wide_takes(int S, int M, int Q, int max_lds) {
+// 0.77..0.84 where one is (n = 112, 124).  With one state a cell is one long
+// chain for its wavefront (every basis pair, and one product in four used), so
+// as many cells as workgroups are resident go to the workgroup kernel (n = 64,
+// 66 points: 64 cells 0.45 ms against 0.32, 512 cells 0.47 against 0.38), more
+// of them here (1,024 cells 0.48 against 0.68).
+bool newton_wide_takes(int S, int M, int Q, int max_lds, int num_cu, long ncell) {
     const int waves = S * M <= wide_limit(S) ? wide_waves(S, M, Q, max_lds) : 0;
-    if (waves != 1) return waves > 1;
-    return !newton_block_fits(S, M, Q, max_lds) || 2 * newton_block_lds(S, M, Q) > (size_t)max_lds;
+    if (waves == 0 || !newton_block_fits(S, M, Q, max_lds)) return waves > 0;
+    const int resident = 2 * newton_block_lds(S, M, Q) <= (size_t)max_lds ? 2 : 1;
+    if (waves == 1 && resident == 2) return false;
+    return S > 1 || ncell > (long)resident * num_cu;
 }
 
 long newton_wide_kept_floats(int S, int M) {

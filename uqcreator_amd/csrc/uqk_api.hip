@@ -101,32 +101,29 @@ int check_mesh(uqk_ctx* ctx, const uqk_mesh* m) {
     return 0;
 }
 
-// Whether a kernel for large systems takes the shape (UQK_KERNEL_BLOCK): one
+// Whether a kernel for large systems takes n cells (UQK_KERNEL_BLOCK): one
 // wavefront per cell where newton_wide_takes says so, else a workgroup per cell.
-bool wide_takes(const uqk_ctx* ctx) {
-    return uqk::newton_wide_takes(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+bool wide_takes(const uqk_ctx* ctx, long n) {
+    return uqk::newton_wide_takes(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds, ctx->num_cu, n);
 }
-bool large_fits(const uqk_ctx* ctx) {
-    return wide_takes(ctx) || uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
+bool large_fits(const uqk_ctx* ctx, long n) {
+    return wide_takes(ctx, n) || uqk::newton_block_fits(ctx->S, ctx->M, ctx->Q, (int)ctx->max_lds);
 }
 
-// Kept inverse factors of the mixed wave kernel across time steps: grows
-// the per-cell slots (flags cleared) to n cells.  Allocates only outside
-// graph capture.
-// Kept factorisations of the time loop's mixed closure, by the kernel the
-// launch takes: 1 the wave kernel's kept inverses, 2 those of the kernels for
-// large systems (below 128 duals inverses in tiles, else the workgroup kernel's
-// kept FP32 factors), 0 none.
-int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
+// Kept factorisations of the time loop's mixed closure of n cells, by the
+// kernel the launch takes: 1 the wave kernel's kept inverses, 2 the workgroup
+// kernel's kept FP32 factors, 3 the inverses in tiles of the one-wavefront
+// kernel for large systems, 0 none.
+int factor_mode(const uqk_ctx* ctx, bool per_cell_orders, long n) {
     if (ctx->precision != UQK_MIXED || !ctx->factor_reuse || ctx->c.max_iter == 1) return 0;
     int wm = 0, wo = 0;
     if ((ctx->kernel == UQK_KERNEL_AUTO || ctx->kernel == UQK_KERNEL_WAVE) && !per_cell_orders &&
         uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, 1, &wm, &wo))
         return uqk::newton_wave_reuse_fits(ctx->kind, ctx->M, ctx->Q, (int)ctx->max_lds) ? 1 : 0;
     if (ctx->kernel == UQK_KERNEL_WAVE) return 0;
-    const bool block_ok = large_fits(ctx);
-    if (block_ok && (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64)))
-        return 2;
+    if (large_fits(ctx, n) &&
+        (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64)))
+        return wide_takes(ctx, n) ? 3 : 2;
     return 0;
 }
 
@@ -134,9 +131,10 @@ int factor_mode(const uqk_ctx* ctx, bool per_cell_orders) {
 // capture only; a change of mode starts with no kept factor.
 int ensure_factor_buffers(uqk_ctx* ctx, long n_cells, int mode) {
     const long n = (long)ctx->S * ctx->M;
-    // mode 1: the FP32 inverse; mode 2: the same in tiles, or the FP32 factor (packed U)
-    const long nn = mode == 1 ? uqk::newton_wave_kept_floats(ctx->S, ctx->M)
-                    : wide_takes(ctx) ? uqk::newton_wide_kept_floats(ctx->S, ctx->M) : n * (n + 1) / 2;
+    // mode 1: the FP32 inverse; mode 2: the FP32 factor (packed U); mode 3: the FP32 inverse in tiles
+    const long nn = mode == 1   ? uqk::newton_wave_kept_floats(ctx->S, ctx->M)
+                    : mode == 3 ? uqk::newton_wide_kept_floats(ctx->S, ctx->M)
+                                : n * (n + 1) / 2;
     if (ctx->pinv_cell_cap >= n_cells && ctx->factor_mode == mode) return 0;
     if (ctx->capturing) return fail(ctx, -1, "kept factors: buffers must exist before graph capture");
     hipFree(ctx->pinv_cell);
@@ -242,7 +240,7 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
     // wave kernel's inverses or those of the kernel for large systems; in
     // registers for a single closure call);
     // the buffers exist before a graph is captured
-    const int fmode = factors_per_cell ? factor_mode(ctx, nt != nullptr) : 0;
+    const int fmode = factors_per_cell ? factor_mode(ctx, nt != nullptr, n) : 0;
     if (fmode) {
         if (int rc = ensure_factor_buffers(ctx, n, fmode)) return rc;
         a.pinv_mode = 1;
@@ -318,10 +316,11 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
         a.grad_at_lam = nullptr;
         a.dt_cell = nullptr;
     }
-    const bool block_ok = large_fits(ctx);
+    const bool block_ok = large_fits(ctx, n);
     if (ctx->kernel == UQK_KERNEL_BLOCK || (ctx->kernel == UQK_KERNEL_AUTO && ctx->S * ctx->M >= 64 && block_ok)) {
         if (!block_ok) return fail(ctx, -3, "closure too large for the workgroup kernel");
-        if (a.pinv_mode == 1 && ctx->factor_mode != 2) a.pinv_mode = 0;  // (the slots hold inverses)
+        const bool wide = wide_takes(ctx, n);
+        if (a.pinv_mode == 1 && ctx->factor_mode != (wide ? 3 : 2)) a.pinv_mode = 0;  // (the slots hold another form)
         const bool fuse = uq_out && u_out && ctx->c.max_iter != 1 && !refining;
         a.uq_out = fuse ? uq_out : nullptr;
         a.u_out = fuse ? u_out : nullptr;
@@ -352,7 +351,7 @@ int launch_closure(uqk_ctx* ctx, int64_t n, const int32_t* nt, const double* u, 
             a.grad_at_lam = ctx->check_grad;
             a.dt_cell = ca.dt_cell;
         }
-        UQK_HIP(ctx, (wide_takes(ctx) ? uqk::newton_wide_launch : uqk::newton_block_launch)(
+        UQK_HIP(ctx, (wide ? uqk::newton_wide_launch : uqk::newton_block_launch)(
                          ctx->kind, a, (int)ctx->max_lds, ctx->num_cu, ctx->stream, ctx->shape));
         if (ev) UQK_HIP(ctx, hipEventRecord(ctx->tev1, ctx->stream));
         ctx->step_recon = a.dt_cell != nullptr;
@@ -927,7 +926,7 @@ int64_t uqk_run_steps(uqk_ctx* ctx, const uqk_problem* prob, const uqk_mesh* mes
     // the warm start's and the kept inverses' buffers must exist before the
     // step is captured
     if (int rc = uqk::prepare_warm_start(ctx, mesh->n_cells)) return rc;
-    if (const int fmode = factor_mode(ctx, nt != nullptr))
+    if (const int fmode = factor_mode(ctx, nt != nullptr, mesh->n_cells))
         if (mesh->n_cells > 0)
             if (int rc = ensure_factor_buffers(ctx, mesh->n_cells, fmode)) return rc;
     if (ctx->residual_check && mesh->n_cells > 0)
@@ -1131,7 +1130,7 @@ int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda,
                       uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, 4, &wmax,
                                               &occ);
     const bool block = !wave && (ctx->kernel == UQK_KERNEL_AUTO || ctx->kernel == UQK_KERNEL_BLOCK) &&
-                       large_fits(ctx);
+                       large_fits(ctx, n);
     if (!wave && !block) return fail(ctx, -3, "uqk_autotune: no specialised closure kernel for this shape");
     if (block) wmax = 4;
     const size_t bytes = sizeof(double) * (size_t)n * ctx->S * ctx->M;
@@ -1148,7 +1147,7 @@ int uqk_autotune(uqk_ctx* ctx, int64_t n, const double* u, const double* lambda,
         if (wave)
             uqk::newton_wave_limits(ctx->kind, ctx->M, ctx->Q, ctx->precision, (int)ctx->max_lds, waves, &wm, &oc);
         else
-            oc = wide_takes(ctx) ? 1 : uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
+            oc = wide_takes(ctx, n) ? 1 : uqk::newton_block_occupancy(ctx->kind, ctx->M, ctx->Q, ctx->precision);
         for (int per_cu = 1; per_cu <= oc && rc == 0; ++per_cu) {
             ctx->shape.waves = waves;
             ctx->shape.blocks_per_cu = per_cu;

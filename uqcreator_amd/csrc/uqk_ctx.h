@@ -63,7 +63,8 @@ struct uqk_ctx {
     float* pinv_cell = nullptr;
     int* pinv_ok = nullptr;
     // what the buffers hold: 1 the wave kernel's kept inverses, 2 the
-    // workgroup kernel's kept FP32 factors; 0 none
+    // workgroup kernel's kept FP32 factors, 3 the inverses in tiles of the
+    // one-wavefront kernel for large systems; 0 none
     int factor_mode = 0;
     // residual check before the wave kernel in the time loop (on by
     // default): the cells it leaves to the Newton kernel

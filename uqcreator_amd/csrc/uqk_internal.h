@@ -151,8 +151,8 @@ bool newton_tile_fits(int S, int M, int Q, int max_lds);
 hipError_t newton_tile_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st);
 // one-wavefront kernel for n = S*M < 128 (fewer than four states: < 112) with
 // one wavefront per SIMD, per-cell orders, FP64 or mixed with kept inverses
-// (closure_wide_kernel.h); whether it takes the shape
-bool newton_wide_takes(int S, int M, int Q, int max_lds);
+// (closure_wide_kernel.h); whether it takes ncell cells of the shape
+bool newton_wide_takes(int S, int M, int Q, int max_lds, int num_cu, long ncell);
 // floats of a cell's kept inverse
 long newton_wide_kept_floats(int S, int M);
 hipError_t newton_wide_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
