@@ -44,6 +44,8 @@ constexpr int kTile = 64;   // GEMM workgroup tile (rows and columns)
 constexpr int kKs = 32;     // GEMM K step (one MFMA 16x16x32)
 constexpr int kLdsStride = 40;  // bf16 per LDS tile row (32 + 8 pad)
 constexpr long kNetSmallRows = 4096;  // rows up to which the fused network takes 16 per workgroup
+constexpr int kNetWidest = 416;       // widest layer of the fused network,
+constexpr int kNetWidestAlone = 288;  // and where 16 rows leave it one workgroup
 constexpr long kPredictChunk = 1L << 16;  // rows per inference pass of the warm start
 
 enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2, EPI_ATOMIC = 3 };
@@ -898,12 +900,17 @@ int ensure_rows(uqk_mlp* n, long rows) {
 int forward(uqk_mlp* n, long rows, bool store_z) {
     // the fused network where its activations leave two workgroups per CU:
     // 64 rows per workgroup for many rows, 16 for a training batch (which
-    // would fill a few CUs only, and with more rows read the weights too often)
+    // would fill a few CUs only, and with more rows read the weights too often).
+    // Not for wide layers, whose weights every workgroup reads as one chain
+    // where the GEMMs deal them out: of 1,024 rows a forward pass takes 37 us
+    // fused and 54 layer by layer at 256 hidden units, 56 and 63 at 416, 66
+    // and 62 at 448, 218 and 115 at 1,024; of one row 34 and 36 at 256, 35 and
+    // 41 at 288, 43 and 41 at 320, 217 and 75 at 1,024.
     int widest = 0;
     for (int l = 0; l <= kLayers; ++l) widest = std::max(widest, n->dims[l]);
     const int rt = rows > kNetSmallRows ? 4 : 1;
     const size_t lds = sizeof(__bf16) * 2 * 16 * rt * (size_t)(widest + 8);
-    bool whole = rows > 0 && lds <= 80 * 1024;
+    bool whole = rows > 0 && lds <= 80 * 1024 && widest <= (rows <= 16 ? kNetWidestAlone : kNetWidest);
     for (int l = 0; l <= kLayers; ++l) whole = whole && n->dims[l] % kKs == 0;
     if (whole) {
         NetArgs a{};
