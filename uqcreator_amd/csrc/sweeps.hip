@@ -93,6 +93,28 @@ __global__ void __launch_bounds__(kSweepThreads) reconstruct_kernel(SweepArgs a)
     }
 }
 
+// The same with one thread per moment, for few of them over few points: a
+// wavefront of reconstruct_kernel then has four cells and hardly any product
+// (262,144 cells of four states: 4 moments at 5 points 38 us here, 45 there; 3
+// at 3 28 and 44; 1 at 1 16 and 39; but 4 at 8 48 and 45, 3 at 12 51 and 47).
+constexpr int kReconstructSmall = 32;  // moments times points below which it is taken
+template <int S>
+__global__ void __launch_bounds__(kSweepThreads) reconstruct_small_kernel(SweepArgs a) {
+    UQK_SKIP_IF_INACTIVE(a)
+    const int M = a.M, Q = a.Q;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.ncell * S * M) return;
+    const long cell = t / (S * M);
+    const int e = (int)(t - cell * S * M), i = e / S, s = e - i * S;
+    const int nt = a.nt_cell ? a.nt_cell[cell] : M;
+    double acc = 0.0;
+    if (i < nt) {
+        const double* q = a.uq + cell * S * Q;
+        for (int k = 0; k < Q; ++k) acc += q[k * S + s] * a.phiw[k * M + i];
+    }
+    a.u_out[t] = acc;
+}
+
 // MomentSolver refinement (momentsolver.cpp:104-117) with ComputeRefIndicator
 // (:271-289), one thread per cell.  The indicator of a cell at level l is
 // |u(0, nt-1)| + |u(0, nt-2)| for one uncertain dimension, else the sum of
@@ -605,14 +627,22 @@ hipError_t launch_refine(const RefineArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
+template <int S> static void go_reconstruct(const SweepArgs& a, hipStream_t st) {
+    const bool few = a.M * a.Q < kReconstructSmall;
+    // work items (moments or cells) per workgroup
+    const long items = few ? a.ncell * S * a.M : a.ncell, per = few ? kSweepThreads : (kSweepThreads / 64) * (16 / S);
+    const dim3 blocks((unsigned)((items + per - 1) / per));
+    if (few)
+        hipLaunchKernelGGL(reconstruct_small_kernel<S>, blocks, dim3(kSweepThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL(reconstruct_kernel<S>, blocks, dim3(kSweepThreads), 0, st, a);
+}
 hipError_t launch_reconstruct(const SweepArgs& a, hipStream_t st) {
     if (a.ncell <= 0) return hipSuccess;
-    const long per = (kSweepThreads / 64) * (16 / a.S);
-    const dim3 blocks((unsigned)((a.ncell + per - 1) / per));
     switch (a.S) {
-        case 1: hipLaunchKernelGGL(reconstruct_kernel<1>, blocks, dim3(kSweepThreads), 0, st, a); break;
-        case 3: hipLaunchKernelGGL(reconstruct_kernel<3>, blocks, dim3(kSweepThreads), 0, st, a); break;
-        case 4: hipLaunchKernelGGL(reconstruct_kernel<4>, blocks, dim3(kSweepThreads), 0, st, a); break;
+        case 1: go_reconstruct<1>(a, st); break;
+        case 3: go_reconstruct<3>(a, st); break;
+        case 4: go_reconstruct<4>(a, st); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
