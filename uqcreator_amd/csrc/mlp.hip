@@ -720,11 +720,13 @@ __global__ __launch_bounds__(256) void apply_kernel(long n, const double* u, con
 // Persistent workgroups: phi and phiW are staged in LDS once per workgroup,
 // each wave walks cells with a grid stride and stages the candidate duals of
 // its cell in LDS (the sums run in the same order as a plain loop over k, i).
+// Five wavefronts per SIMD, for the wait on the exponentials' chain: 65,536
+// cells of 45 duals at 49 points, the whole call 228 us, and 247 with the four
+// that the compiler's own choice of 100 registers leaves.
 template <int KIND>
-__global__ __launch_bounds__(256) void select_kernel(uqk::ClosureParams cp, long ncell, int M, int Q,
-                                                     const double* phi, const double* phiw, const double* u,
-                                                     double* lam, const double* lam_alt, const int* nt,
-                                                     unsigned long long* counter, const int* active) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void select_kernel(
+    uqk::ClosureParams cp, long ncell, int M, int Q, const double* phi, const double* phiw, const double* u,
+    double* lam, const double* lam_alt, const int* nt, unsigned long long* counter, const int* active) {
     constexpr int S = uqk::KindInfo<KIND>::S;
     if (active && *active == 0) return;
     extern __shared__ double sel_lds[];
