@@ -64,3 +64,32 @@ def test_slots_follow_the_number_of_cells():
         assert got[2:] == want[2:] and got[3][1] > 0
         np.testing.assert_array_equal(got[0], want[0])
         np.testing.assert_array_equal(got[1], want[1])
+
+
+@pytest.mark.gpu
+def test_wave_count_is_the_wave_kernels():
+    """The launch shape's number of wavefronts is the wave kernel's: set before
+    (a tuned context, say), it does not idle the large systems' SIMDs."""
+    b = native.Basis(3, [4], 5)
+    rng = np.random.default_rng(47)
+    n = 4096
+    h, vx, vy = rng.uniform(1, 3, n), rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    lam = np.zeros((n, b.M, 3))
+    lam[:, 0] = np.stack([9.81 * h - 0.5 * (vx * vx + vy * vy), vx, vy], -1)
+    lam[:, 1:] = rng.normal(0, 0.01, (n, b.M - 1, 3)) * np.abs(lam[:, :1])
+    cl = native.GpuClosure(native.SHALLOW_WATER2D_BARRIER, b, epsilon=1e-8, barrier=0.01, safe_line_search=1)
+    dl, uq, u = native.DeviceArray.from_host(lam), native.DeviceArray((n, b.Q, 3)), native.DeviceArray((n, b.M, 3))
+    cl.eval_uq(dl, uq)
+    cl.reconstruct(uq, u)
+    lam[:, 1:] = 0.0
+    times = {}
+    for waves in (0, 1):
+        cl.set_launch_shape(waves, 0)
+        for _ in range(4):
+            x = native.DeviceArray.from_host(lam)
+            assert cl.solve(u, x) == 0 and cl.last_kernel() == native.KERNEL_BLOCK
+            times[waves] = min(times.get(waves, np.inf), cl.last_closure_ms())
+    print("case: 105 duals, launch shape of one wavefront", times, flush=True)
+    # equal work; the tables leave LDS for one workgroup, whose one wavefront
+    # would take three to four times as long
+    assert times[1] < 1.5 * times[0]

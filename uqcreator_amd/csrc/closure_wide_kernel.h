@@ -793,9 +793,8 @@ static hipError_t wide_go(const NewtonArgs& args, int max_lds, int num_cu, hipSt
     NewtonArgs a = args;
     a.wave_doubles = wide_ring(S, a.M);
     const WideLds at(S, a.M, a.Q, a.wave_doubles);
-    int waves = wide_waves(S, a.M, a.Q, max_lds);
+    const int waves = wide_waves(S, a.M, a.Q, max_lds);  // (shape.waves is the wave kernel's)
     if (waves < 1) return hipErrorInvalidValue;
-    if (shape.waves > 0 && shape.waves < waves) waves = shape.waves;
     const size_t shmem = sizeof(double) * ((size_t)at.tables + (size_t)waves * at.wave);
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, newton_wide_kernel<KIND, NT, KEEP>, 64 * waves, shmem) !=
