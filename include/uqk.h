@@ -264,9 +264,11 @@ int uqk_last_closure_stats(const uqk_ctx* ctx, int64_t* newton_steps, int64_t* g
  * a contraction clearly worse than a damped Newton step's (above
  * 1.2 (1 - alpha) + 1e-3; + 0.05 from n = 64 on, where a factorisation costs
  * over ten steps on the kept one), the cell's current Hessian is factored
- * and the reference Newton step runs.  Memory per cell: n times n rounded up
- * to a multiple of four floats (wave kernel), n (n + 1) / 2 floats (workgroup
- * kernel), n = S M.  In a single closure call (wave kernel, uniform
+ * and the reference Newton step runs.  Memory per cell, n = S M: n times n rounded
+ * up to a multiple of four floats (wave kernel), 128 r (r + 1) floats with r =
+ * n / 16 rounded up (one-wavefront kernel for large systems: 10 KB at n = 64,
+ * 28 KB from 97 to 112, 36 KB above), n (n + 1) / 2 floats (workgroup
+ * kernel).  In a single closure call (wave kernel, uniform
  * orders, damped Newton: alpha < 1, whose steps contract linearly anyway)
  * a cell's Newton steps after a factorisation
  * apply that step's FP64 inverse (d = H^{-1} g) under the same accept and

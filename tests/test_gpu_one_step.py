@@ -21,10 +21,10 @@ WAVE_CASES = [(native.BOUNDED_BARRIER, 1, [5], 12), (native.EULER1D, 2, [4], 7),
 TILE_CASES = [c for c in TILE_CASES if c[2][-1] > 1]
 
 
-def _problem(oracle, kind, d, degrees, q1, n, alpha, seed, uniform=False):
+def _problem(oracle, kind, d, degrees, q1, n, alpha, seed):
     """Cells, a start at which the gradient's norm is about 1e-2, the oracle's
     next iterate, and the norms of both."""
-    b = native.Basis(d, degrees[-1:] if uniform else degrees, q1)
+    b = native.Basis(d, degrees, q1)
     rng = np.random.default_rng(seed)
     levels = np.asarray(b.ntotal_per_level, np.int32)
     nt = levels[rng.integers(0, len(levels), n)].astype(np.int32)

@@ -39,6 +39,13 @@ def test_wide_kernel_for_few_cells(S, M, Q, cells, takes):
     assert _wide_takes(S, M, Q, cells) == takes
 
 
+@pytest.mark.parametrize("S,M,tile_rows", [(4, 16, 4), (3, 22, 5), (4, 24, 6), (3, 35, 7), (4, 28, 7), (4, 31, 8)])
+def test_kept_inverse_takes_the_tiles_of_its_rows(S, M, tile_rows):
+    f = getattr(native.lib(), "_ZN3uqk23newton_wide_kept_floatsEii")  # uqk::newton_wide_kept_floats(int, int)
+    f.restype = ctypes.c_long
+    assert f(S, M) == 256 * (tile_rows * (tile_rows + 1) // 2)
+
+
 @pytest.mark.gpu
 def test_slots_follow_the_number_of_cells():
     """One context that runs many cells, few and many again: what the kernel of

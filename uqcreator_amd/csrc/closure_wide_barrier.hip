@@ -32,10 +32,7 @@ bool newton_wide_takes(int S, int M, int Q, int max_lds, int num_cu, long ncell)
     return S > 1 || ncell > (long)resident * num_cu;
 }
 
-long newton_wide_kept_floats(int S, int M) {
-    const int nt = wide_tiles(S * M) < 6 ? 6 : wide_tiles(S * M);
-    return 256l * (nt * (nt + 1) / 2);
-}
+long newton_wide_kept_floats(int S, int M) { return wide_kept(S * M); }
 
 hipError_t newton_wide_launch(int kind, const NewtonArgs& a, int max_lds, int num_cu, hipStream_t st,
                               const LaunchShape& shape) {

@@ -48,6 +48,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // tiles of 16 rows that n duals and the right-hand side take
 __host__ __device__ constexpr int wide_tiles(int n) { return n / 16 + 1; }
 
+// floats of a cell's kept inverse: the lower tiles of the rows that n duals
+// take (without the right-hand side's)
+__host__ __device__ constexpr long wide_kept(int n) {
+    const long r = (n + 15) / 16;
+    return 256 * (r * (r + 1) / 2);
+}
+
 // Largest system: 127 duals and the right-hand side are eight tile rows; with
 // fewer than four states a lane holds more duals of every vector, for which
 // the registers beside that many tiles do not last.
@@ -170,7 +177,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
         for (int t = 0; t < TILES; ++t) K[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (cl < 0 || tag_n != nt_n || tag_n == 0) return;
-        const f32x4* src = reinterpret_cast<const f32x4*>(a.pinv + cl * (long)(256 * TILES)) + lane;
+        const f32x4* src = reinterpret_cast<const f32x4*>(a.pinv + cl * wide_kept(SM)) + lane;
 #pragma unroll
         for (int tr = 0; tr < NT; ++tr) {
             if (16 * tr >= S * nt_n) break;
@@ -512,7 +519,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                                 if (16 * tc + 4 * e + q4 < n) yb[16 * tc + 4 * e + q4] = T[tile_lower(tc, tr)][e];
                     }
                 if (spd && reuse) {
-                    f32x4* dst = reinterpret_cast<f32x4*>(a.pinv + cell * (long)(256 * TILES)) + lane;
+                    f32x4* dst = reinterpret_cast<f32x4*>(a.pinv + cell * wide_kept(SM)) + lane;
 #pragma unroll
                     for (int tr = 0; tr < NT; ++tr) {
                         if (16 * tr >= n) break;
