@@ -14,8 +14,9 @@ captured step graph, with u and lambda resident in HBM.
     python bench.py [--steps K] [--warmup W] [--legs fp64,mixed,mixed_warm_start]
                     [--no-cpu] [--no-c2]
 
-Legs: plain FP64 closure; mixed closure (Hessian on FP32 MFMA, FP64
-Cholesky, gradient and accept test); mixed closure with the learned warm start
+Legs: plain FP64 closure; mixed closure (steps on kept FP32 inverses; Hessian,
+factorisation, gradient and accept test in FP64); mixed closure with the learned
+warm start
 (a network trained here, outside the timed regions, on (u, lambda) pairs the
 FP64 leg's Newton solver produced; the prediction and the per-cell selection
 run inside every step).  `value` is the mixed leg.  Each leg reports the
@@ -132,7 +133,7 @@ class C3:
         kname = ("closure_recheck_kernel<2,10,25> (closure_check_kernel<2,10,25> in the first step) + " +
                  "newton_wave_kernel<2,10,25,%d>" % (2 if lagged > 0 else 0))
         roof_c = closure_roofline(kname, closure_ms / timed_steps, newton / args.steps, grads / args.steps, fm,
-                                  precision == native.MIXED, factors / args.steps, lagged / args.steps)
+                                  factors / args.steps, lagged / args.steps)
         adv_ms = advance_ms / timed_steps
         roof_a = advance_roofline("advance_kernel<2>", adv_ms, S, M, Q, self.m.nbr.shape[1], 2, self.n)
         out = {
@@ -283,7 +284,7 @@ def c2_leg(native, np, b, u, lam0, lam_star, args, precision, warm=None):
         "status_counts": np.bincount(status, minlength=5).tolist(),
         "lambda_rel_err_vs_known": float((np.abs(lam_h - lam_star) / scale).max()),
         "roofline": closure_roofline(kname, float(np.mean(kernel_ms)), newton / args.c2_steps,
-                                     grads / args.c2_steps, fm, precision == native.MIXED, factors / args.c2_steps,
+                                     grads / args.c2_steps, fm, factors / args.c2_steps,
                                      lagged / args.c2_steps, reuse="factor"),
     }
     if net is not None:

@@ -119,11 +119,12 @@ int uqk_synchronize(uqk_ctx* ctx);
 
 /* Closure kernel selection: AUTO picks the compile-time specialised wave
  * kernel when one exists for (closure, M, Q) and the batch has one order,
- * else the kernel for large systems (UQK_KERNEL_BLOCK; 64..128 duals: one
- * wavefront per cell below 128, where LDS holds the tables, else a workgroup
- * per cell), else the generic wave-per-cell kernel (any size, per-cell orders, FP64; below 64
- * duals in register tiles, where it outruns the mixed precision of the
- * kernel for large systems, which UQK_KERNEL_BLOCK still selects). */
+ * else from 64 duals on a kernel for large systems (UQK_KERNEL_BLOCK, two of
+ * them: up to 127 duals of four states and 111 of fewer one wavefront per
+ * cell where that is the faster one, else a workgroup per cell, up to 128
+ * duals), else the generic wave-per-cell kernel (any size, per-cell orders,
+ * FP64; below 64 duals in register tiles, where it outruns the kernels for
+ * large systems, which UQK_KERNEL_BLOCK still selects). */
 enum { UQK_KERNEL_AUTO = 0, UQK_KERNEL_GENERIC = 1, UQK_KERNEL_WAVE = 2, UQK_KERNEL_BLOCK = 3 };
 int uqk_set_closure_kernel(uqk_ctx* ctx, int32_t kernel);
 /* Kernel used by the last closure call (UQK_KERNEL_GENERIC / _WAVE / _BLOCK). */
@@ -254,11 +255,10 @@ int uqk_last_closure_stats(const uqk_ctx* ctx, int64_t* newton_steps, int64_t* g
  * a cell's FP64 factorisation of its Hessian in one step, the library keeps
  * P = H^{-1} of the factored matrix as an explicit inverse (computed in
  * FP64 with the step, kept in FP32): the wave kernel (uniform orders, n < 64)
- * and the kernel for 64 to 127 duals (per-cell orders too, tagged with the
- * cell's order); the workgroup kernel keeps the factor U rounded to FP32,
+ * and the one-wavefront kernel for large systems (per-cell orders too, tagged
+ * with the cell's order); the workgroup kernel keeps the factor U rounded to FP32,
  * replaced by U^{-1} (P = U^{-1} U^{-T}) the first time a later step uses it.
- * The
- * cell's Newton steps in later time steps take d = P g refined once with
+ * The cell's Newton steps in later time steps take d = P g refined once with
  * the FP64 Hessian-vector product (d += P (g - H d)) and keep it when the
  * full step lowers ||grad L|| (the FP64 accept test); otherwise, and after
  * a contraction clearly worse than a damped Newton step's (above
@@ -282,8 +282,8 @@ int uqk_set_factor_reuse(uqk_ctx* ctx, int32_t on);
  * Closure::SolveClosure stops at once when ||grad L||_2 < epsilon at the
  * cell's lambda (closure.cpp:133-193); a check kernel evaluates that
  * gradient for every cell -- one lane per cell for the one-wavefront
- * kernel's shapes, one wave per cell for the workgroup kernel's (n up to
- * 128, per-cell orders too) -- finishes the cells that pass (uQ, the
+ * kernel's shapes, one wave per cell for the large systems' (n up to 128,
+ * per-cell orders too) -- finishes the cells that pass (uQ, the
  * moments, ComputeDt, status, zero iterations) and lists the others, which
  * the Newton kernel then takes, starting from the gradient the check
  * found.  Within one uqk_run_steps call, the steps after the first take

@@ -171,7 +171,7 @@ def _legs(make_closure, prob, m, u, lam0, nt, steps, params, closure_from_lam0, 
             # (the mixed time loop of large systems is the instantiation that keeps inverses, <.., 1>)
             r["roofline_closure"] = roofline.closure_roofline(
                 kernels["closure"] % int(block and prec == native.MIXED), cms, newton / steps,
-                grads / steps, fm, prec == native.MIXED, factors / steps, lagged / steps)
+                grads / steps, fm, factors / steps, lagged / steps)
         print("case:", leg, "loop", {k: r[k] for k in ("value", "ms_per_step", "newton_steps_per_cell_step",
                                                        "mean_var_rel_l2_vs_fp64")}, file=sys.stderr, flush=True)
         if net is not None:

@@ -1,6 +1,8 @@
 // closure_block.hip -- batched FP64 Newton dual closure for large systems
 // (n = S * nTotal up to 128) that closure_wide_kernel.h does not take: 128
-// duals, and tables that LDS does not hold.  One 256-thread workgroup per cell.
+// duals, 112 and more with fewer than four states, tables that leave LDS for
+// one wavefront or none, and few cells of one state (newton_wide_takes).  One
+// 256-thread workgroup per cell.
 //
 // Restates Closure::SolveClosure / SolveClosureSafe (closure.cpp:133-193,
 // :297-339), like closure_fp64.hip, with the work of a cell spread over four

@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(kCheckThreads) closure_recheck_kernel(NewtonAr
     add_counts(none, wave_min((conv && a.dt_min) ? a.dt_cell[cs] : 1e10), red, a.counter, a.dt_min);
 }
 
-// The same check for the workgroup kernel's sizes (n = S*M up to 128, any
+// The same check for the large systems' kernels (n = S*M up to 128, any
 // Q, per-cell orders): one wave per cell, the workgroup's waves strided over
 // the cells.  Lanes over points evaluate Lambda (over the cell's nTotal), U
 // and uQ; lanes over duals (i, s), i < nTotal, sum the projection over the
@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(kCheckThreads) closure_recheck_kernel(NewtonAr
 // network's candidate, which replaces lambda when its ||grad L|| is smaller
 // (a NaN norm never wins), as the wave kernel chooses; a candidate that
 // passes finishes the cell.  The gradients of the listed cells at the duals
-// they keep are stored for the workgroup kernel, which starts from them.  In
+// they keep are stored for the Newton kernel, which starts from them.  In
 // a run's later steps (*recon_ok) the gradient at lambda comes from the last
 // step's moments, as in closure_recheck_kernel.
 template <int KIND>

@@ -13,7 +13,7 @@
 // What bounds it: the latency of a cell's chain, as in the wave kernel.  It
 // replaced a column-by-column Cholesky in LDS (closure_fp64.hip, which is
 // left with the systems of 64 duals and more): Euler 2D, 65,536 cells on
-// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 22.1 ms
+// refinement levels of 12, 24 and 40 duals, 25 points, 40 time steps: 21.0 ms
 // against 52.6 (26.2 with DU through the exponential and with the lane's
 // numbers kept over the cell: 4 to 48 registers spilled; 22.8 with reads of 8
 // bytes from LDS and tile rows skipped by branches).

@@ -30,9 +30,9 @@
 // 3.4 K (register tiles spread over the wave with one LDS round trip per two
 // pivots: 23.4 K and 19.2 K), Hessian 3.7 K (pairs over lanes, DU by
 // v_readlane, with an exponential and a logarithm: 14.6 K), gradient 3.6 K
-// (4.3 K); 65,536 cells, 40 time steps: 21.4 ms against 39.0 (FP64), 16.5
+// (4.3 K); 65,536 cells, 40 time steps: 20.2 ms against 39.0 (FP64), 15.4
 // against 30.7 (mixed).  At n = 45, 49 points, one closure of 100,003 cells:
-// 29.9 ms against 47.4 (FP64), 10.0 against 19.5 (mixed: a step on the kept
+// 29.2 ms against 47.4 (FP64), 10.0 against 19.5 (mixed: a step on the kept
 // inverse is a matrix-vector product from registers, 1.3 K cycles, in place
 // of two triangular solves from LDS, 13.9 K).
 // The next cell's moments, duals, density and kept inverse are asked for

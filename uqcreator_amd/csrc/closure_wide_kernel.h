@@ -1,7 +1,8 @@
-// closure_wide_kernel.h -- the Newton closure for systems of 64 <= n = S
-// nTotal < 128 duals of any basis, quadrature and per-cell order, one
-// wavefront per cell and one wavefront per SIMD: the whole system, up to 36
-// tiles of 16 x 16 doubles, lies in that wavefront's 512 registers.
+// closure_wide_kernel.h -- the Newton closure for systems of n = S nTotal >= 64
+// duals, up to 127 with four states and 111 with fewer (wide_limit), of any
+// basis, quadrature and per-cell order, one wavefront per cell and one
+// wavefront per SIMD: the whole system, up to 36 tiles of 16 x 16 doubles,
+// lies in that wavefront's 512 registers.
 // Instantiated per closure kind (closure_wide_*.hip) and per number of
 // 16-row tiles that the largest order needs.
 //
@@ -28,9 +29,9 @@
 // workgroup of four wavefronts per cell (closure_block.hip), two resident per
 // CU, takes 75 K, 149 K and 18 K for the first three, which is four to nine
 // times as much per wavefront and cell: 65,536 cells of the dam break, 12 time
-// steps: 35 ms against 89.  Orders of 12 to 112 duals, 49 points, 16,384 cells,
-// 12 steps: 9.3 ms against 28.  The workgroup kernel is left with 128 duals,
-// and with tables of which LDS holds none beside a wavefront's part.
+// steps: 31 ms against 89.  Orders of 12 to 112 duals, 49 points, 16,384 cells,
+// 12 steps: 9.2 ms against 28.  The workgroup kernel is left with more duals,
+// and with the sizes at which newton_wide_takes finds it faster.
 #pragma once
 #include <hip/hip_runtime.h>
 

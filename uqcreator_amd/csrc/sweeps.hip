@@ -215,6 +215,11 @@ __host__ __device__ inline int advance_wave_doubles(int S, int Q) {
     return advance_cells_per_wave(S, Q) * Q * S;
 }
 
+// a read-only value at a uniform address, through the scalar cache
+template <class T> __device__ __forceinline__ T uniform_load(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)p;
+}
+
 // ExplicitEuler::Advance (expliciteuler.cpp:8-75) with numFlux
 // (momentsolver.cpp:413-416) for a wavefront's cells: each lane owns a
 // quadrature point of one cell and sums the point fluxes of all the cell's
@@ -233,11 +238,6 @@ __host__ __device__ inline int advance_wave_doubles(int S, int Q) {
 // registers, 2,048 workgroups instead of 8,192 that each load the projection's
 // table: 94 -> 79 us there, 777 -> 466 us for 65,536 cells at 125 points and
 // three states, whose projection took 16-row products for 3 rows.
-// a read-only value at a uniform address, through the scalar cache
-template <class T> __device__ __forceinline__ T uniform_load(const T* p) {
-    return *(const __attribute__((address_space(4))) T*)p;
-}
-
 // ONE: a wavefront has one cell (Q > 32).  The cell, its edges and their
 // normals are then uniform, in scalar registers.
 // (four waves per SIMD: the kernel waits on memory, and the register budget

@@ -190,7 +190,7 @@ bool wave_check(const uqk_ctx* ctx, bool per_cell_orders) {
 // Launch the Newton closure kernel; leaves the failed-cell counts in counters
 // (counters: the context's d_counters unless the caller brings its own
 // kClosureCounters).
-// When uq_out/u_out are given and the specialised or the workgroup kernel runs
+// When uq_out/u_out are given and a kernel that fuses them runs
 // (not one-shot), it also writes uQ and the reconstructed moments and *fused
 // is set.
 // With dt_out as well (the step), the fused kernels also reduce

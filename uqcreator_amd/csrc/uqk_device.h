@@ -203,10 +203,10 @@ __device__ __forceinline__ void closure_DU(const ClosureParams& c, const double*
 }
 
 // ---------------------------------------------------------------------------
-// 1/x and sqrt(x) to an ulp: v_rcp_f64 and v_rsq_f64 with two refinements,
-// in place of the correctly rounded divide and root, which take four times
-// the instructions (and most of the time of the point fluxes).  Zero,
-// infinities and NaN as 1/x and sqrt(x) have them.
+// 1/x and sqrt(x) to an ulp: v_rcp_f64 with two Newton steps and v_rsq_f64
+// with two of Goldschmidt's, in place of the correctly rounded divide and root,
+// which take four times the instructions (and most of the time of the point
+// fluxes).  Zero, infinities and NaN as 1/x and sqrt(x) have them.
 __device__ __forceinline__ double recip_any(double x) {
     const double r = __builtin_amdgcn_rcp(x);
     double e = fma(-x, r, 1.0);

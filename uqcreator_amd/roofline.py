@@ -1,7 +1,7 @@
 """Roofline models of the closure and advance kernels on one MI355X.
 
-Algorithmic flops of the Newton closure per step kind, the time-weighted peak
-of the units they run on, and the algorithmic HBM bytes of the fused advance.
+Algorithmic flops of the Newton closure per step kind against the FP64 peak, on
+which all of them run, and the algorithmic HBM bytes of the fused advance.
 Shared by bench.py and the configuration runner (uqcreator_amd.configs).
 """
 import numpy as np
@@ -36,13 +36,12 @@ def advance_bytes_per_cell(S, M, Q, edges, dim):
     return 8 * S * Q + 8 * S * M + 8 * S * M + geometry
 
 
-def closure_roofline(kernel, kernel_ms, newton, grads, fm, precision_mixed, factors=None, lagged=0.0,
+def closure_roofline(kernel, kernel_ms, newton, grads, fm, factors=None, lagged=0.0,
                      reuse="inverse"):
     """Roofline of a closure launch: algorithmic flops over its HIP-event
-    time against the FP64 peak, on which all of them run (the mixed closure's
-    Hessian too; precision_mixed changes nothing any more).  factors / lagged: factored Newton
-    steps and steps on a kept factorisation (mixed closure; by default every
-    Newton step is factored).  reuse: "inverse" (the time loop keeps an
+    time against the FP64 peak.  factors / lagged: factored Newton steps and
+    steps on a kept factorisation (mixed closure; by default every Newton step
+    is factored).  reuse: "inverse" (the time loop keeps an
     inverse per factorisation, F_inv + F_lag) or "factor" (a single call solves
     with its last factor, F_tri)."""
     if factors is None:
