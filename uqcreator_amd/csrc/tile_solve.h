@@ -285,6 +285,8 @@ __device__ __forceinline__ double tile_back(const f64x4 (&T)[TILES], int n, int 
 // In place on all NT x NT tiles (tile (tc, tr) at tr * NT + tc): the sweep
 // of every pivot block, which leaves -H^-1 in the rows and columns below n
 // and H^-1 g in column n (where row and column n held the right-hand side).
+// The pivot columns, set to zero beforehand, get P B^-1, and -B^-1 in the block
+// itself, from the same products: -L^-T stands in the place of V's pivot rows.
 template <int NT>
 __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, int q) {
     bool ok = true;
@@ -295,16 +297,16 @@ __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, in
         double li, lt, di;
         ok &= pivot_factors(T[jb * NT + jb][e], 4 * e, have, p, q, li, lt, di);
         const bool in = (p >> 2) == e && (p & 3) < have;  // this lane's row of tile row jb is a pivot
-        double V[NT], U[NT], W[NT];
+        double V[NT], U[NT];
 #pragma unroll
         for (int r = 0; r < NT; ++r) {
             double P = T[r * NT + jb][e];
             if (r == jb && in) P = 0.0;
             if (have < 4 && q >= have) P = 0.0;
             V[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(li, P, 0.0, 0, 0, 0);
-            // pivot rows: H(c, pivot) <- V D^-1 L^-1 = P B^-1, and -B^-1 in the block itself
-            U[r] = (r == jb && in ? -lt : V[r]) * di;
-            W[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(lt, U[r], 0.0, 0, 0, 0);
+            if (r == jb && in) V[r] = -lt;
+            U[r] = V[r] * di;
+            if (!(have < 4 && q >= have)) T[r * NT + jb][e] = 0.0;
         }
         if (in) {
 #pragma unroll
@@ -313,11 +315,8 @@ __device__ __forceinline__ bool tile_sweep(f64x4 (&T)[NT * NT], int n, int p, in
 #pragma unroll
         for (int r = 0; r < NT; ++r)
 #pragma unroll
-            for (int c = 0; c < NT; ++c) {
-                const double old = T[r * NT + c][e];
+            for (int c = 0; c < NT; ++c)
                 T[r * NT + c] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[c], -U[r], T[r * NT + c], 0, 0, 0);
-                if (c == jb) T[r * NT + c][e] = have < 4 && q >= have ? old : W[r];  // the pivot columns
-            }
     }
     return ok;
 }
@@ -354,6 +353,7 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p
             if (r == jb && in) P = 0.0;
             if (have < 4 && q >= have) P = 0.0;
             V[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(li, P, 0.0, 0, 0, 0);
+            if (r == jb && in) V[r] = -lt;
         }
         if (in) {
 #pragma unroll
@@ -361,14 +361,11 @@ __device__ __forceinline__ bool tile_sweep_lower(f64x4 (&T)[TILES], int n, int p
         }
 #pragma unroll
         for (int r = 0; r < NT; ++r) {
-            const double U = (r == jb && in ? -lt : V[r]) * di;
-            const double W = __builtin_amdgcn_mfma_f64_4x4x4f64(lt, U, 0.0, 0, 0, 0);
+            const double U = V[r] * di;
+            if (jb <= r && !(have < 4 && q >= have)) T[tile_lower(jb <= r ? jb : r, r)][e] = 0.0;
 #pragma unroll
-            for (int c = 0; c <= r; ++c) {
-                const double old = T[tile_lower(c, r)][e];
+            for (int c = 0; c <= r; ++c)
                 T[tile_lower(c, r)] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[c], -U, T[tile_lower(c, r)], 0, 0, 0);
-                if (c == jb) T[tile_lower(c, r)][e] = have < 4 && q >= have ? old : W;
-            }
         }
     }
     if (!__builtin_constant_p(n)) settle<18>();
