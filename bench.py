@@ -135,7 +135,7 @@ class C3:
         roof_c = closure_roofline(kname, closure_ms / timed_steps, newton / args.steps, grads / args.steps, fm,
                                   factors / args.steps, lagged / args.steps)
         adv_ms = advance_ms / timed_steps
-        roof_a = advance_roofline("advance_kernel<2>", adv_ms, S, M, Q, self.m.nbr.shape[1], 2, self.n)
+        roof_a = advance_roofline("advance_kernel<2,false>", adv_ms, S, M, Q, self.m.nbr.shape[1], 2, self.n)
         out = {
             "value": self.n * args.steps / elapsed,
             "ms_per_step": 1e3 * elapsed / args.steps,
@@ -462,7 +462,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f64" if prec_head == native.FP64 else "f64+f32-mfma",
+        "dtype": "f64" if prec_head == native.FP64 else "f64+f32",
         "data": "synthetic",
         "config": {
             "workload": "2D Euler IPM time loop, NACA0012 O-grid 512x128 (65,536 cells), AoA 1.25+0.5 xi1 deg, "

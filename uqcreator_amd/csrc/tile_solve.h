@@ -9,7 +9,8 @@
 // p, k = q) and the B operand (k = q, columns p) of a rank-4 update.  So four
 // pivots are eliminated per step without moving the panel:
 //   B   = L D L^T, the 4 x 4 pivot block, factored by every lane from
-//         v_readlane'd scalars (three reciprocals in sequence);
+//         v_readlane'd scalars (four reciprocals in sequence, of which V
+//         waits for three);
 //   V   = P L^-T, one v_mfma_f64_4x4x4_4b per 16 rows of the panel P;
 //   H  -= V D^-1 V^T on the tiles that are left, one v_mfma_f64_16x16x4 each.
 // There is no LDS round trip and no lane mask per entry.
